@@ -11,9 +11,9 @@
 // dispatch: one query row in bf16 / f16 at head dim 128 without ALiBi goes to the
 // split-K decode kernels (decode.hip), any other row alone over more than 768
 // keys (few rows and heads) to this kernel split over 256-key chunks (partials
-// merged by mha_split_combine_kernel); bf16 / f16 causal or non-causal prefill at head
-// dim 128 or 64, with or without a sliding window or ALiBi, to the MFMA flash
-// kernel (prefill.hip).
+// merged by mha_split_combine_kernel); prefill, causal or not, with or without a
+// sliding window or ALiBi, to the MFMA flash kernels (prefill.hip): bf16 / f16 at head
+// dims of 8 n up to 256, f32 at 4 n.
 #include "attention.hpp"
 
 namespace puter {

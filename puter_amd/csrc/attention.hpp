@@ -19,12 +19,14 @@ struct MhaArgs {
     // (max, sum) and unnormalised output row; null otherwise
     float2 *part_ml = nullptr;
     float *part_o = nullptr;
+    int nan_rows = 0;  // FlashAttention's rows with a NaN score are NaN, MultiHeadAttention's zeros (padded head dims)
 };
 
 // MFMA flash prefill (prefill.hip).  Returns true and sets *status when the
-// shape is one it serves (bf16 / f16, head_dim 128 or 64, causal or not, sliding window, ALiBi;
-// head dim 64 only for more than one query row; f32, head_dim 128 or 64, at least 16
-// query rows, causal or not, sliding window, ALiBi).
+// shape is one it serves (bf16 / f16, head_dim a multiple of 8 up to 256, causal or not,
+// sliding window, ALiBi; head dims other than 128 only for more than one query row; f32,
+// head_dim a multiple of 4 up to 256, at least 16 query rows, causal or not, sliding
+// window, ALiBi).
 bool launch_prefill_mfma(const MhaArgs &a, int dtype, hipStream_t s, int *status);
 // one query row per sequence (bf16 / f16, head_dim 128): the paged decode kernels
 bool launch_decode_contiguous(const MhaArgs &m, int dtype, hipStream_t s, int *status);

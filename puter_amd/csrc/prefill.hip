@@ -1,6 +1,7 @@
 // MFMA flash-attention prefill: bf16 or f16 Q/K/V (prefill_kernel<dtype, head
 // dim, window>; f32 Q/K/V on prefill_f32_kernel, described where it is defined),
-// f32 accumulation, output in the input format, head_dim 128 or 64, GQA,
+// f32 accumulation, output in the input format, head_dim 128 or 64 (tuned) or any multiple
+// of 8 up to 256 (4 in f32; rows padded with zero chunks in LDS, see PfDim), GQA,
 // optional causal mask: key k is visible to query q when
 // k <= q + shift.  MultiHeadAttention passes shift = seqK - seqQ (bottom-right
 // aligned, device/cpu/attention/typed_compute.go:166-168);
@@ -70,6 +71,8 @@
 #include "attention.hpp"
 
 #include <climits>
+#include <cmath>
+#include <type_traits>
 
 namespace puter {
 
@@ -101,28 +104,32 @@ constexpr float RESCALE_SLACK = 8.0f;   // log2 headroom before O and l are resc
 constexpr float RESCALE_LIMIT = 256.0f; // 2^RESCALE_SLACK: the largest p allowed
 // buffer descriptor word 3 for raw (untyped, stride 0) dword access on gfx9
 constexpr int BUF_WORD3 = 0x00020000;
+constexpr int OOB = 0x7FFFFFF0;  // an offset past every descriptor's range
 }  // namespace fa
 
-// Per-head-dim layout of the K / V tiles (D = 128 or 64; 16-bit elements).
-// Rows are D * 2 bytes (16 or 8 chunks of 16 bytes).  K row r keeps chunk c at
-// c ^ kswz(r): with 256-byte rows kswz = r % 16, with 128-byte rows (two rows per
-// 64-bank line) kswz = (r / 2) % 8, so the 16 rows a fragment read touches fall
-// on distinct banks either way.  V row r keeps chunk c at c ^ vswz(r): 4 (r % 4)
-// for 256-byte rows, 4 ((r / 2) % 2) for 128-byte rows, so the four rows x 32
+// Layout of the K / V tiles for head dims up to D (D = 64, 96, 128 or 256; 16-bit
+// elements).  Rows are 128, 256 or 512 bytes (8, 16 or 32 chunks of 16 bytes), the
+// power of two that holds D, so a lane's row and chunk are a shift and a mask; a head
+// dim below D (any multiple of 8) leaves the chunks past it zero, and 96 computes 6 of
+// a 128-row's 8 k-steps and 3 of its 4 output blocks.  K row r keeps chunk c at
+// c ^ kswz(r): with rows of 256 bytes or more kswz = r % 16, with 128-byte rows (two
+// rows per 64-bank line) kswz = (r / 2) % 8, so the 16 rows a fragment read touches
+// fall on distinct banks either way.  V row r keeps chunk c at c ^ vswz(r): 4 (r % 4)
+// for rows of 256 bytes or more, 4 ((r / 2) % 2) for 128-byte rows, so the four rows x 32
 // bytes of each transposing read (and the rows two apart that share a bank
 // line) do not collide.  Both swizzles are unchanged by row offsets of 8, 16
 // and 32, which the fragment reads add to a base row.
 template <int D> struct PfDim {
-    static_assert(D == 128 || D == 64, "head dim 128 or 64");
-    static constexpr int RB = D * 2;           // row bytes
+    static_assert(D == 256 || D == 128 || D == 96 || D == 64, "head dim 256, 128, 96 or 64");
+    static constexpr int RB = D > 128 ? 512 : D > 64 ? 256 : 128;   // row bytes
     static constexpr int NC = RB / 16;         // 16-byte chunks per row
-    static constexpr int TILE = fa::BN * RB;   // one K or V tile: 16 or 8 KB
+    static constexpr int TILE = fa::BN * RB;   // one K or V tile: 32, 16 or 8 KB
     static constexpr int KS = D / 16;          // S MFMA k-steps (16 dims each)
     static constexpr int DB = D / 32;          // O^T blocks of 32 dims
     static constexpr int RPI = 64 / NC;        // rows per copy instruction (64 lanes x 16 B)
     static constexpr int NI = 16 / RPI;        // copy instructions per wave and tensor
-    static constexpr int kswz(int r) { return D == 128 ? (r & 15) : ((r >> 1) & 7); }
-    static constexpr int vswz(int r) { return D == 128 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); }
+    static constexpr int kswz(int r) { return RB >= 256 ? (r & 15) : ((r >> 1) & 7); }
+    static constexpr int vswz(int r) { return RB >= 256 ? ((r & 3) << 2) : (((r >> 1) & 1) << 2); }
 };
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -133,11 +140,14 @@ struct PrefillArgs {
     const uint16_t *q, *k, *v;
     uint16_t *o;
     int batch, seq_q, seq_k, heads, kv_heads, qtiles;
+    int nan_rows;      // padded kernels: a row with a NaN score is NaN (else zeros)
+    int dim;           // head dim: a multiple of 8 (16-bit) or 4 (f32), at most the kernel's D
     int causal, xcd_map;
     int shift;         // causal: key k visible to query q iff k <= q + shift
     int window;        // > 0: key k visible to query q only if k > q - window
     float alibi_s;     // ALiBi slope / scale: the dot gains alibi_s * (k - q) before scaling
     float scale_log2;  // softmax scale * log2(e)
+    float scale_log2_lo = 0.0f;  // what scale_log2's rounding left (padded f32 head dims)
     // f32 kernel, key range split over blockIdx.y (split_tiles key tiles each): per
     // split, query row and head the (max, sum) and the unnormalised output row, in
     // [split][batch][query][head] order; null when unsplit
@@ -169,16 +179,17 @@ __device__ __forceinline__ void wait_tile_copies() {
 // fills RPI consecutive rows (64 lanes x 16 bytes): wave w copies rows
 // 4 RPI i + RPI w + lane / NC (i < NI), lane L filling chunk L % NC of its row
 // with the row's chunk (L % NC) ^ swizzle(row) (kg / vg hold those byte offsets).
-template <int D>
+template <int D, bool PAD>
 __device__ __forceinline__ void prefill_copy_tile(const PrefillArgs &a, const uint16_t *kbase,
                                                   const uint16_t *vbase, int kv0, const int *kg,
                                                   const int *vg, char *kdst, char *vdst, int wave) {
     using namespace fa;
     using T = PfDim<D>;
-    const int rs2 = a.kv_heads * D * 2;  // K/V row stride in bytes
+    const int dim = PAD ? a.dim : D;
+    const int rs2 = a.kv_heads * dim * 2;  // K/V row stride in bytes
     const int rows = min(a.seq_k - kv0, BN);   // <= 0: an empty range, every lane reads zeros
-    const int bytes = rows > 0 ? (rows - 1) * rs2 + D * 2 : 0;
-    const int64_t base = rows > 0 ? (int64_t)kv0 * a.kv_heads * D : 0;
+    const int bytes = rows > 0 ? (rows - 1) * rs2 + dim * 2 : 0;
+    const int64_t base = rows > 0 ? (int64_t)kv0 * a.kv_heads * dim : 0;
     const __amdgpu_buffer_rsrc_t kd =
         __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + base), (short)0, bytes, BUF_WORD3);
     const __amdgpu_buffer_rsrc_t vd =
@@ -203,7 +214,29 @@ __device__ __forceinline__ f32x16 pf_mfma(typename PfFormat<DT>::V8 a, typename 
     else return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-template <int DT, int D, bool GEN>
+// P as MFMA operands: its 16-bit rounding and, with LO, what the rounding left, so that
+// hi + lo carries 16 (bf16) or 22 (f16) bits of p.  The head dims that padded rows serve
+// take both: their products with V keep the f32 probabilities of the general kernel, which
+// is what served these dims before, at half as many MFMAs again (64 and 128 round P once).
+template <int DT, bool LO> struct PfLow {
+    typename PfFormat<DT>::V8 v;
+};
+template <int DT> struct PfLow<DT, false> {};
+template <int DT, bool LO>
+__device__ __forceinline__ void pf_set(typename PfFormat<DT>::V8 &hi, PfLow<DT, LO> &lo, int j, float p) {
+    using E = typename PfFormat<DT>::E;
+    hi[j] = (E)p;
+    if constexpr (LO) lo.v[j] = (E)(p - (float)hi[j]);
+}
+template <int DT, bool LO>
+__device__ __forceinline__ f32x16 pf_pv(typename PfFormat<DT>::V8 v, typename PfFormat<DT>::V8 hi,
+                                        const PfLow<DT, LO> &lo, f32x16 c) {
+    c = pf_mfma<DT>(v, hi, c);
+    if constexpr (LO) c = pf_mfma<DT>(v, lo.v, c);
+    return c;
+}
+
+template <int DT, int D, bool GEN, bool LO>
 __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *ks, const char *vs,
                                              const typename PfFormat<DT>::V8 (&qf)[PfDim<D>::KS], PrefillState<D> &st,
                                              int qi, int kv0, const int (&ka)[PfDim<D>::KS],
@@ -211,7 +244,6 @@ __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *k
     using namespace fa;
     using T = PfDim<D>;
     using V8 = typename PfFormat<DT>::V8;
-    using E = typename PfFormat<DT>::E;
     // S^T chunks: keys kv0 + 32c + (8*(r/4) + 4g + r%4), query qi; two
     // independent accumulation chains interleaved
     f32x16 s[2] = {(f32x16){}, (f32x16){}};
@@ -263,6 +295,7 @@ __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *k
     // far above the reference) the max is taken, O and l rescaled, p redone.
     float psum = 0.0f;
     V8 pf[2][2];
+    PfLow<DT, LO> pl[2][2];
     bool done = false;
     if (!__any(st.m == -INFINITY)) {
 #pragma unroll
@@ -273,7 +306,7 @@ __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *k
                 for (int j = 0; j < 8; ++j) {
                     const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][8 * h + j], a.scale_log2, -st.m));
                     psum += p;
-                    pf[c][h][j] = (E)p;
+                    pf_set<DT, LO>(pf[c][h], pl[c][h], j, p);
                 }
         done = !__any(psum > RESCALE_LIMIT);  // each p of this lane <= its partial sum
     }
@@ -304,7 +337,7 @@ __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *k
                 for (int j = 0; j < 8; ++j) {
                     const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][8 * h + j], a.scale_log2, -mref));
                     psum += p;
-                    pf[c][h][j] = (E)p;
+                    pf_set<DT, LO>(pf[c][h], pl[c][h], j, p);
                 }
     }
     st.l += psum;
@@ -320,7 +353,7 @@ __device__ __forceinline__ void prefill_step(const PrefillArgs &a, const char *k
                 const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p));
                 const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + 8 * T::RB));
                 const V8 vf = __builtin_bit_cast(V8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                st.o[d] = pf_mfma<DT>(vf, pf[c][h], st.o[d]);
+                st.o[d] = pf_pv<DT, LO>(vf, pf[c][h], pl[c][h], st.o[d]);
             }
 }
 
@@ -334,11 +367,10 @@ template <int DT> __device__ __forceinline__ float pf_score(float x) {
 // Online-softmax update for one 32-key chunk that needs the slow path (first
 // tile, or a score more than 2^8 above the reference): take the chunk max,
 // rescale O and l if the reference moves, and redo p against it.
-template <int DT, int D>
+template <int DT, int D, bool LO>
 __device__ __forceinline__ float prefill_chunk_slow(const PrefillArgs &a, const f32x16 &s, PrefillState<D> &st,
-                                                    typename PfFormat<DT>::V8 (&pf)[2]) {
+                                                    typename PfFormat<DT>::V8 (&pf)[2], PfLow<DT, LO> (&pl)[2]) {
     using namespace fa;
-    using E = typename PfFormat<DT>::E;
     float tmax = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, pf_score<DT>(s[r]));
@@ -361,7 +393,7 @@ __device__ __forceinline__ float prefill_chunk_slow(const PrefillArgs &a, const 
         for (int j = 0; j < 8; ++j) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(pf_score<DT>(s[8 * h + j]), a.scale_log2, -mref));
             psum += p;
-            pf[h][j] = (E)p;
+            pf_set<DT, LO>(pf[h], pl[h], j, p);
         }
     return psum;
 }
@@ -382,7 +414,7 @@ __device__ __forceinline__ float prefill_chunk_slow(const PrefillArgs &a, const 
 // one copy instruction beside every other MFMA, instead of as one burst before
 // them (bit-identical; +1-2.5% on B4 S4096 / S2048 causal and non-causal, timed
 // interleaved in one process).
-template <int DT, int D>
+template <int DT, int D, bool PAD>
 __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, const char *ks, const char *vs,
                                                        const typename PfFormat<DT>::V8 (&qf)[PfDim<D>::KS],
                                                        PrefillState<D> &st, const int (&ka)[PfDim<D>::KS],
@@ -390,15 +422,21 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
                                                        const uint16_t *vbase, int kvn, const int (&kg)[PfDim<D>::NI],
                                                        const int (&vg)[PfDim<D>::NI], char *kn, char *vn, int wave) {
     using namespace fa;
-    prefill_copy_tile<D>(a, kbase, vbase, kvn, kg, vg, kn, vn, wave);
+    prefill_copy_tile<D, PAD>(a, kbase, vbase, kvn, kg, vg, kn, vn, wave);
     using T = PfDim<D>;
     using V8 = typename PfFormat<DT>::V8;
-    using E = typename PfFormat<DT>::E;
+    constexpr bool LO = PAD;
     constexpr int KS = T::KS, NM = 2 * T::DB;   // S MFMAs per chunk, P.V MFMAs per chunk
-    constexpr int E2 = 16 / KS, E3 = 16 / NM;   // p values evaluated beside each MFMA (phases 2, 3)
+    // p values evaluated beside MFMA t of phases 2 and 3: [16 t / KS, 16 (t + 1) / KS) and
+    // the same over NM; copy instructions: one where NI (t + 1) / KS steps up
+    auto e2 = [](int t) { return 16 * t / KS; };
+    auto e3 = [](int t) { return 16 * t / NM; };
+    auto cp = [](int t) { return T::NI * (t + 1) / KS - T::NI * t / KS; };
+    constexpr int PV = LO ? 6 : 3;              // VALU instructions per p value
     constexpr int RA = KS < 4 ? KS : 4;         // K reads issued ahead of the first S MFMA
     f32x16 s0 = (f32x16){}, s1 = (f32x16){};
     V8 p0[2], p1[2];
+    PfLow<DT, LO> l0[2], l1[2];
     const float m = st.m, c = a.scale_log2;
     // phase 1 + 2
 #pragma unroll
@@ -412,10 +450,10 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
         const V8 kf = *reinterpret_cast<const V8 *>(ks + 32 * T::RB + ka[t]);
         s1 = pf_mfma<DT>(kf, qf[t], s1);
 #pragma unroll
-        for (int r = E2 * t; r < E2 * t + E2; ++r) {
+        for (int r = e2(t); r < e2(t + 1); ++r) {
             const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(pf_score<DT>(s0[r]), c, -m));
             ps0 += p;
-            p0[r >> 3][r & 7] = (E)p;
+            pf_set<DT, LO>(p0[r >> 3], l0[r >> 3], r & 7, p);
         }
     }
     // K fragment reads run RA ahead of the MFMAs that use them (LDS latency
@@ -424,17 +462,17 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // S chunk 0 MFMA t
-        if ((t & 1) && t / 2 < T::NI) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // a K copy
+        if (cp(t)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // a K copy
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // next K read (c0, then c1)
     }
 #pragma unroll
     for (int t = 0; t < KS; ++t) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // S chunk 1 MFMA t
-        if ((t & 1) && t / 2 < T::NI) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // a V copy
+        if (cp(t)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);   // a V copy
         if (t < KS - RA) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // remaining K reads of c1
-        __builtin_amdgcn_sched_group_barrier(0x002, 3 * E2, 0);  // chunk 0 softmax share
+        __builtin_amdgcn_sched_group_barrier(0x002, PV * ((16 + KS - 1) / KS), 0);  // chunk 0 softmax share
     }
-    if (__any(ps0 > RESCALE_LIMIT)) ps0 = prefill_chunk_slow<DT, D>(a, s0, st, p0);
+    if (__any(ps0 > RESCALE_LIMIT)) ps0 = prefill_chunk_slow<DT, D, LO>(a, s0, st, p0, l0);
     st.l += ps0;
     // phase 3: chunk 0's P.V with chunk 1's softmax between the MFMAs
     const float m1 = st.m;
@@ -447,24 +485,24 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
             const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p));
             const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + 8 * T::RB));
             const V8 vf = __builtin_bit_cast(V8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            st.o[d] = pf_mfma<DT>(vf, p0[h], st.o[d]);
-            const int r0 = E3 * (T::DB * h + d);
+            st.o[d] = pf_pv<DT, LO>(vf, p0[h], l0[h], st.o[d]);
+            const int t = T::DB * h + d;
 #pragma unroll
-            for (int r = r0; r < r0 + E3; ++r) {
+            for (int r = e3(t); r < e3(t + 1); ++r) {
                 const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(pf_score<DT>(s1[r]), c, -m1));
                 ps1 += pv;
-                p1[r >> 3][r & 7] = (E)pv;
+                pf_set<DT, LO>(p1[r >> 3], l1[r >> 3], r & 7, pv);
             }
         }
     // V^T fragment reads (two per MFMA) run two MFMAs ahead
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
     for (int t = 0; t < NM; ++t) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // P.V MFMA (chunk 0)
+        __builtin_amdgcn_sched_group_barrier(0x008, LO ? 2 : 1, 0);  // P.V MFMA (chunk 0)
         if (t < NM - 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 3 * E3, 0);  // chunk 1 softmax share
+        __builtin_amdgcn_sched_group_barrier(0x002, PV * ((16 + NM - 1) / NM), 0);  // chunk 1 softmax share
     }
-    if (__any(ps1 > RESCALE_LIMIT)) ps1 = prefill_chunk_slow<DT, D>(a, s1, st, p1);
+    if (__any(ps1 > RESCALE_LIMIT)) ps1 = prefill_chunk_slow<DT, D, LO>(a, s1, st, p1, l1);
     st.l += ps1;
     // phase 4: chunk 1's P.V
 #pragma unroll
@@ -475,21 +513,70 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
             const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p));
             const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(p + 8 * T::RB));
             const V8 vf = __builtin_bit_cast(V8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            st.o[d] = pf_mfma<DT>(vf, p1[h], st.o[d]);
+            st.o[d] = pf_pv<DT, LO>(vf, p1[h], l1[h], st.o[d]);
         }
     __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
     for (int t = 0; t < NM; ++t) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, LO ? 2 : 1, 0);
         if (t < NM - 3) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
 }
 
+// The padded kernels' outputs where an infinity or NaN of V met a P of zero (a masked key
+// of a computed tile, or P's low half): 0 * inf is NaN in the MFMA, while the general
+// kernel, which served these head dims before, never reads a masked key's row.  Such rows
+// (a finite row sum, some output not finite) are summed again here, key by key over the
+// visible keys [k_lo, k_hi), in f32, against the same reference m; the lane's dims are
+// 32d + 8 rb + 4 g .. + 3.  Never taken on finite values.
+template <int DT, int D, int NO>
+__device__ __forceinline__ void prefill_redo(const PrefillArgs &a, const void *qrow, const void *kbase,
+                                             const void *vbase, int64_t krs, int dim, int qi, int g, int k_lo,
+                                             int k_hi, float m, f32x16 (&o)[NO]) {
+    using T = typename Elem<DT>::T;
+    const T *const Q = static_cast<const T *>(qrow);
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d) o[d] = (f32x16){};
+    for (int k = k_lo; k < k_hi; ++k) {
+        const T *const K = static_cast<const T *>(kbase) + k * krs;
+        const T *const V = static_cast<const T *>(vbase) + k * krs;
+        float dot = 0.0f;
+        for (int x = 0; x < dim; ++x) dot += Elem<DT>::load(Q[x]) * Elem<DT>::load(K[x]);
+        if constexpr (DT == PUTER_F16) dot = (float)(_Float16)dot;
+        dot += a.alibi_s * (float)(k - qi);
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(dot, a.scale_log2, -m));
+#pragma unroll
+        for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int c = 32 * d + 8 * (r >> 2) + 4 * g + (r & 3);
+                if (c < dim) o[d][r] += p * Elem<DT>::load(V[c]);
+            }
+    }
+}
+// whether a lane's O holds an infinity or NaN
+template <int D, int NO> __device__ __forceinline__ bool prefill_spoiled(const f32x16 (&o)[NO]) {
+    float t = 0.0f;
+#pragma unroll
+    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) t = __builtin_fmaf(o[d][r], 0.0f, t);
+    return t != 0.0f;   // 0 * x is NaN for an infinite or NaN x
+}
+// the keys of [0, seq_k) that query qi sees: [first, last)
+__device__ __forceinline__ int prefill_first_key(const PrefillArgs &a, int qi) {
+    return a.window > 0 ? max(0, qi - a.window + 1) : 0;
+}
+__device__ __forceinline__ int prefill_last_key(const PrefillArgs &a, int qi) {
+    return a.causal ? min(qi + a.shift + 1, a.seq_k) : a.seq_k;
+}
+
 // GEN: a sliding window (a.window > 0) or an ALiBi slope is set; without either
 // that code compiles away.  With ALiBi every tile takes the masked step, which
-// adds the bias.
-template <int DT, int D, bool GEN>
-__global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
+// adds the bias.  PAD: the head dim is below D and read from the arguments (per-lane copy
+// offsets that the exact kernels derive from one register cost the f32 one spills).
+template <int DT, int D, bool GEN, bool PAD>
+__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillArgs a) {
     using namespace fa;
     using T = PfDim<D>;
     using V8 = typename PfFormat<DT>::V8;
@@ -530,10 +617,11 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
     }
     const int kvh = h / (a.heads / a.kv_heads);
     const int q0 = qt * BM;
-    const int64_t qrs = (int64_t)a.heads * D, krs = (int64_t)a.kv_heads * D;
-    const uint16_t *qbase = a.q + (int64_t)b * a.seq_q * qrs + (int64_t)h * D;
-    const uint16_t *kbase = a.k + (int64_t)b * a.seq_k * krs + (int64_t)kvh * D;
-    const uint16_t *vbase = a.v + (int64_t)b * a.seq_k * krs + (int64_t)kvh * D;
+    const int dim = PAD ? a.dim : D;
+    const int64_t qrs = (int64_t)a.heads * dim, krs = (int64_t)a.kv_heads * dim;
+    const uint16_t *qbase = a.q + (int64_t)b * a.seq_q * qrs + (int64_t)h * dim;
+    const uint16_t *kbase = a.k + (int64_t)b * a.seq_k * krs + (int64_t)kvh * dim;
+    const uint16_t *vbase = a.v + (int64_t)b * a.seq_k * krs + (int64_t)kvh * dim;
 
     // this lane's query and its Q^T operand fragments (KS k-steps of 16 dims)
     const int qfirst = q0 + 32 * wave;
@@ -544,7 +632,9 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
         const int qload = min(qi, a.seq_q - 1);  // rows past the end compute garbage, never stored
 #pragma unroll
         for (int t = 0; t < T::KS; ++t)
-            qf[t] = __builtin_bit_cast(V8, *reinterpret_cast<const uint4 *>(qbase + (int64_t)qload * qrs + 16 * t + 8 * g));
+            qf[t] = 16 * t + 8 * g < dim   // dims past the head dim: zeros
+                        ? __builtin_bit_cast(V8, *reinterpret_cast<const uint4 *>(qbase + (int64_t)qload * qrs + 16 * t + 8 * g))
+                        : (V8){};
     }
 
     // key tiles of the block: [tlo, ntiles); tiles [tfree, nfree) need no mask for
@@ -568,13 +658,15 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
     // byte offsets of this lane's tile copies (source side, swizzled) ...
     int kg[T::NI], vg[T::NI];
     {
-        const int rs2 = a.kv_heads * D * 2;
+        // chunks past the head dim: an offset past the buffer's range, read as zeros
+        const int rs2 = a.kv_heads * dim * 2;
         const int pos = lane % T::NC;
 #pragma unroll
         for (int i = 0; i < T::NI; ++i) {
             const int row = 4 * T::RPI * i + T::RPI * wave + lane / T::NC;
-            kg[i] = row * rs2 + ((pos ^ T::kswz(row)) << 4);
-            vg[i] = row * rs2 + ((pos ^ T::vswz(row)) << 4);
+            const int kc = pos ^ T::kswz(row), vc = pos ^ T::vswz(row);
+            kg[i] = 8 * kc < dim ? row * rs2 + (kc << 4) : OOB;
+            vg[i] = 8 * vc < dim ? row * rs2 + (vc << 4) : OOB;
         }
     }
     // ... and of its fragment reads: K row l32 (+32c), chunk (2t + g) ^ kswz(l32);
@@ -600,7 +692,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
 
     // tile t lives in buffer t % 2
     if (tlo < ntiles)
-        prefill_copy_tile<D>(a, kbase, vbase, tlo * BN, kg, vg, (tlo & 1) ? k1s : k0s, (tlo & 1) ? v1s : v0s, wave);
+        prefill_copy_tile<D, PAD>(a, kbase, vbase, tlo * BN, kg, vg, (tlo & 1) ? k1s : k0s, (tlo & 1) ? v1s : v0s, wave);
     wait_tile_copies();
     __syncthreads();
     // One tile: copy the next tile into the other buffers, compute this one, then
@@ -613,7 +705,7 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
         // the next tile's copy runs inside the step (past the last tile: an empty one
         // into the free buffers, so the step has no branch around it)
         const int kvn = it + 1 < ntiles ? (it + 1) * BN : a.seq_k;
-        prefill_step_pipelined<DT, D>(a, kc, vc, qf, st, ka, va, kbase, vbase, kvn, kg, vg, kn, vn, wave);
+        prefill_step_pipelined<DT, D, PAD>(a, kc, vc, qf, st, ka, va, kbase, vbase, kvn, kg, vg, kn, vn, wave);
         wait_tile_copies();
         __syncthreads();
     };
@@ -621,11 +713,11 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
         const int kv0 = it * BN;
         const bool odd = it & 1;
         if (it + 1 < ntiles)
-            prefill_copy_tile<D>(a, kbase, vbase, kv0 + BN, kg, vg, odd ? k0s : k1s, odd ? v0s : v1s, wave);
+            prefill_copy_tile<D, PAD>(a, kbase, vbase, kv0 + BN, kg, vg, odd ? k0s : k1s, odd ? v0s : v1s, wave);
         // waves whose queries all precede this tile, or whose windows all start
         // past it, skip it
         if ((!a.causal || kv0 <= qlast + a.shift) && (!GEN || a.window <= 0 || kv0 + BN - 1 >= qfirst - a.window + 1))
-            prefill_step<DT, D, GEN>(a, odd ? k1s : k0s, odd ? v1s : v0s, qf, st, qi, kv0, ka, va, g, true);
+            prefill_step<DT, D, GEN, PAD>(a, odd ? k1s : k0s, odd ? v1s : v0s, qf, st, qi, kv0, ka, va, g, true);
         wait_tile_copies();
         __syncthreads();
     };
@@ -648,15 +740,29 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
     // normalise and store: lane holds O[qi][32d + 8*(r/4) + 4g + r%4]
     const float ltot = swap_halves_sum(st.l);
     const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
+    if constexpr (PAD) {
+        if (ltot > 0.0f && qi < a.seq_q && prefill_spoiled<D>(st.o))
+            prefill_redo<DT, D>(a, qbase + (int64_t)qi * qrs, kbase, vbase, krs, dim, qi, g, prefill_first_key(a, qi),
+                                prefill_last_key(a, qi), st.m, st.o);
+        // a NaN row sum (a NaN score): zeros, or NaN from FlashAttention, as the general kernels
+        if (!(ltot > 0.0f)) {
+            const float z = a.nan_rows ? ltot : 0.0f;
+#pragma unroll
+            for (int d = 0; d < T::DB; ++d)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st.o[d][r] = z;
+        }
+    }
     if (qi < a.seq_q) {
-        uint16_t *orow = a.o + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)h * D;
+        uint16_t *orow = a.o + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)h * dim;
 #pragma unroll
         for (int d = 0; d < T::DB; ++d)
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb) {
+                if (32 * d + 8 * rb >= dim) continue;   // dim % 8 == 0: an 8-dim run is whole or absent
                 V4 v;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = (E)(st.o[d][4 * rb + i] * inv);
+                for (int i = 0; i < 4; ++i) v[i] = (E)(PAD && !(ltot > 0.0f) ? st.o[d][4 * rb + i] : st.o[d][4 * rb + i] * inv);
                 *reinterpret_cast<V4 *>(orow + 32 * d + 8 * rb + 4 * g) = v;
             }
     }
@@ -680,11 +786,11 @@ __global__ __launch_bounds__(256, 2) void prefill_kernel(PrefillArgs a) {
 //     keeps column d at d ^ 32 (k / 4 % 2), so the two half-waves, rows k and k + 4,
 //     read opposite halves of the bank line).
 template <int D> struct PfF32Dim {
-    static_assert(D == 128 || D == 64, "head dim 128 or 64");
+    static_assert(D == 256 || D == 128 || D == 96 || D == 64, "head dim 256, 128, 96 or 64");
     static constexpr int BN = 32;               // keys per tile
-    static constexpr int RB = D * 4;            // row bytes
+    static constexpr int RB = D > 128 ? 1024 : D > 64 ? 512 : 256;   // row bytes (the power of two that holds D)
     static constexpr int NC = RB / 16;          // 16-byte chunks per row
-    static constexpr int TILE = BN * RB;        // 16 or 8 KB
+    static constexpr int TILE = BN * RB;        // 32, 16 or 8 KB
     static constexpr int KG = D / 8;            // 4-step groups over d
     static constexpr int DB = D / 32;           // O^T blocks of 32 dims
     static constexpr int RPI = 64 / NC;         // rows per copy instruction
@@ -693,8 +799,8 @@ template <int D> struct PfF32Dim {
     static constexpr int vswz(int r) { return ((r >> 2) & 1) << 3; }   // in chunks (8 = 32 floats)
 };
 
-template <int D, bool GEN>
-__global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
+template <int D, bool GEN, bool PAD>
+__global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(PrefillArgs a) {
     using T = PfF32Dim<D>;
     constexpr int BM = fa::BM, BN = T::BN;
     __shared__ __attribute__((aligned(1024))) char k0s[T::TILE];
@@ -728,10 +834,11 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
     const float *const qp = reinterpret_cast<const float *>(a.q);
     const float *const kp = reinterpret_cast<const float *>(a.k);
     const float *const vp = reinterpret_cast<const float *>(a.v);
-    const int64_t qrs = (int64_t)a.heads * D, krs = (int64_t)a.kv_heads * D;
-    const float *qbase = qp + (int64_t)b * a.seq_q * qrs + (int64_t)hd * D;
-    const float *kbase = kp + (int64_t)b * a.seq_k * krs + (int64_t)kvh * D;
-    const float *vbase = vp + (int64_t)b * a.seq_k * krs + (int64_t)kvh * D;
+    const int dim = PAD ? a.dim : D;
+    const int64_t qrs = (int64_t)a.heads * dim, krs = (int64_t)a.kv_heads * dim;
+    const float *qbase = qp + (int64_t)b * a.seq_q * qrs + (int64_t)hd * dim;
+    const float *kbase = kp + (int64_t)b * a.seq_k * krs + (int64_t)kvh * dim;
+    const float *vbase = vp + (int64_t)b * a.seq_k * krs + (int64_t)kvh * dim;
 
     // this lane's query and its Q^T operands: qf[g] = Q[qi][8 g + 4 h .. + 3]
     const int qfirst = q0 + 32 * wave;
@@ -742,7 +849,9 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
         const int qload = min(qi, a.seq_q - 1);   // rows past the end compute garbage, never stored
 #pragma unroll
         for (int g = 0; g < T::KG; ++g)
-            qf[g] = *reinterpret_cast<const f32x4 *>(qbase + (int64_t)qload * qrs + 8 * g + 4 * h);
+            qf[g] = 8 * g + 4 * h < dim   // dims past the head dim: zeros
+                        ? *reinterpret_cast<const f32x4 *>(qbase + (int64_t)qload * qrs + 8 * g + 4 * h)
+                        : (f32x4){};
     }
 
     int kend = a.seq_k;
@@ -762,22 +871,24 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
     }
 
     // copy offsets (source side, swizzled): wave w fills rows 4 RPI i + RPI w + lane / NC
-    int kg[4], vg[4];
+    int kg[8], vg[8];
     {
-        const int rs4 = a.kv_heads * D * 4;
+        // chunks past the head dim: an offset past the buffer's range, read as zeros
+        const int rs4 = a.kv_heads * dim * 4;
         const int pos = lane % T::NC;
 #pragma unroll
         for (int i = 0; i < T::NI; ++i) {
             const int row = 4 * T::RPI * i + T::RPI * wave + lane / T::NC;
-            kg[i] = row * rs4 + ((pos ^ T::kswz(row)) << 4);
-            vg[i] = row * rs4 + ((pos ^ T::vswz(row)) << 4);
+            const int kc = pos ^ T::kswz(row), vc = pos ^ T::vswz(row);
+            kg[i] = 4 * kc < dim ? row * rs4 + (kc << 4) : fa::OOB;
+            vg[i] = 4 * vc < dim ? row * rs4 + (vc << 4) : fa::OOB;
         }
     }
     auto copy_tile = [&](int kv0, char *kdst, char *vdst) __attribute__((always_inline)) {
-        const int rs4 = a.kv_heads * D * 4;
+        const int rs4 = a.kv_heads * dim * 4;
         const int rows = min(a.seq_k - kv0, BN);
-        const int bytes = (rows - 1) * rs4 + D * 4;
-        const int64_t base = (int64_t)kv0 * a.kv_heads * D;
+        const int bytes = (rows - 1) * rs4 + dim * 4;
+        const int64_t base = (int64_t)kv0 * a.kv_heads * dim;
         const __amdgpu_buffer_rsrc_t kd =
             __builtin_amdgcn_make_buffer_rsrc((void *)(kbase + base), (short)0, bytes, fa::BUF_WORD3);
         const __amdgpu_buffer_rsrc_t vd =
@@ -785,12 +896,12 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
         // (constant trip counts with a guard: a loop bound that depends on the template
         // arguments inside a lambda loses the kernel's host stub)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
             if (i < T::NI)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(kd, (lds_void *)(kdst + (4 * T::RPI * i + T::RPI * wave) * T::RB),
                                                          16, kg[i], 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
             if (i < T::NI)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(vd, (lds_void *)(vdst + (4 * T::RPI * i + T::RPI * wave) * T::RB),
                                                          16, vg[i], 0, 0, 0);
@@ -798,20 +909,20 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
     // fragment reads: K row l32, group g at chunk (2 g + h) ^ kswz(l32); V row
     // 8 g + 4 h + s, column (32 db + l32) ^ 32 h (vswz(row) = 8 chunks iff h = 1)
     const int kr = l32 * T::RB;
-    int vr[4];
+    int vr[8];
 #pragma unroll
-    for (int db = 0; db < 4; ++db) vr[db] = 4 * h * T::RB + (((32 * db + l32) ^ (32 * h)) << 2);
+    for (int db = 0; db < T::DB; ++db) vr[db] = 4 * h * T::RB + (((32 * db + l32) ^ (32 * h)) << 2);
 
-    f32x16 o[4];
+    f32x16 o[8];
 #pragma unroll
-    for (int db = 0; db < 4; ++db) o[db] = (f32x16){};
+    for (int db = 0; db < T::DB; ++db) o[db] = (f32x16){};
     float m = -INFINITY, l = 0.0f;
     const float c = a.scale_log2;
 
     auto step = [&](const char *ks, const char *vs, int kv0, bool masked) __attribute__((always_inline)) {
         f32x16 sacc = (f32x16){};
 #pragma unroll
-        for (int g = 0; g < 16; ++g) {
+        for (int g = 0; g < 32; ++g) {
             if (g >= T::KG) break;
             const f32x4 kv = *reinterpret_cast<const f32x4 *>(ks + kr + (((2 * g + h) ^ T::kswz(l32)) << 4));
 #pragma unroll
@@ -846,7 +957,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
             m = mnew;
             l *= alpha;
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
+            for (int db = 0; db < 8; ++db) {
                 if (db >= T::DB) break;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
@@ -856,10 +967,32 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
         float psum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            sacc[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[r], c, -mref));
+            float e = __builtin_fmaf(sacc[r], c, -mref);
+            if constexpr (PAD) e = __builtin_fmaf(sacc[r], a.scale_log2_lo, e);
+            sacc[r] = __builtin_amdgcn_exp2f(e);
             psum += sacc[r];
         }
         l += psum;
+        if constexpr (PAD) {
+            // (the general kernel, which served these head dims before, sums the keys in
+            // short runs: each tile's product starts from zero here and is added to O once,
+            // so the error stays below its own)
+#pragma unroll
+            for (int db = 0; db < 8; ++db) {
+                if (db >= T::DB) break;
+                f32x16 t = (f32x16){};
+#pragma unroll
+                for (int g = 0; g < BN / 8; ++g)
+#pragma unroll
+                    for (int s4 = 0; s4 < 4; ++s4) {
+                        const float vv = *reinterpret_cast<const float *>(vs + (8 * g + s4) * T::RB + vr[db]);
+                        t = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, sacc[4 * g + s4], t, 0, 0, 0);
+                    }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[db][r] += t[r];
+            }
+            return;
+        }
         // O^T += V^T . P^T, step (g, s4): V row 8 g + 4 h + s4, P^T register 4 g + s4; a
         // scheduling barrier per group keeps one group's V reads live at a time
 #pragma unroll
@@ -867,7 +1000,7 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
 #pragma unroll
             for (int s4 = 0; s4 < 4; ++s4)
 #pragma unroll
-                for (int db = 0; db < 4; ++db) {
+                for (int db = 0; db < 8; ++db) {
                     if (db >= T::DB) break;
                     const float vv = *reinterpret_cast<const float *>(vs + (8 * g + s4) * T::RB + vr[db]);
                     o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, sacc[4 * g + s4], o[db], 0, 0, 0);
@@ -906,17 +1039,28 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
     if (it < thi) tile(it, k0s, v0s, k1s, v1s);
 
     const float ltot = swap_halves_sum(l);
+    if constexpr (PAD) {
+        if (ltot > 0.0f && qi < a.seq_q && prefill_spoiled<D>(o))
+            prefill_redo<PUTER_F32, D>(a, qbase + (int64_t)qi * qrs, kbase, vbase, krs, dim, qi, h,
+                                       max(prefill_first_key(a, qi), tlo * BN), min(prefill_last_key(a, qi), thi * BN), m, o);
+        if (!(ltot > 0.0f)) {   // a NaN score: zeros, as the general kernel
+#pragma unroll
+            for (int db = 0; db < 8; ++db)
+                if (db < T::DB) o[db] = (f32x16){};
+        }
+    }
     if (a.part_ml) {
         // split: the row's (max, sum) and unnormalised output to the partials
         if (qi < a.seq_q) {
             const int64_t prow = (((int64_t)blockIdx.y * a.batch + b) * a.seq_q + qi) * a.heads + hd;
             if (h == 0) a.part_ml[prow] = make_float2(m, ltot);
-            float *orow = a.part_o + prow * D;
+            float *orow = a.part_o + prow * dim;
 #pragma unroll
-            for (int db = 0; db < 4; ++db) {
+            for (int db = 0; db < 8; ++db) {
                 if (db >= T::DB) break;
 #pragma unroll
                 for (int rb = 0; rb < 4; ++rb) {
+                    if (32 * db + 8 * rb + 4 * h >= dim) continue;
                     f32x4 v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[i] = o[db][4 * rb + i];
@@ -929,12 +1073,13 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
     // normalise and store: lane holds O[qi][32 db + 8 (r/4) + 4 h + r%4]
     const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
     if (qi < a.seq_q) {
-        float *orow = reinterpret_cast<float *>(a.o) + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)hd * D;
+        float *orow = reinterpret_cast<float *>(a.o) + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)hd * dim;
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
+        for (int db = 0; db < 8; ++db) {
             if (db >= T::DB) break;
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb) {
+                if (32 * db + 8 * rb + 4 * h >= dim) continue;   // dim % 4 == 0
                 f32x4 v;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] = o[db][4 * rb + i] * inv;
@@ -948,38 +1093,61 @@ __global__ __launch_bounds__(256, 2) void prefill_f32_kernel(PrefillArgs a) {
 // lanes over the head dims; the splits are folded in order with weights
 // exp2(m_s - M) (m in the scaled log2 domain), O = sum w_s O_s / sum w_s l_s; a row
 // with no visible key (every m = -inf) is 0, as in the unsplit kernel.
-template <int D>
 __global__ __launch_bounds__(256) void prefill_f32_combine_kernel(PrefillArgs a, int splits, int64_t rows) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int lane = threadIdx.x & 63;
     float M = -INFINITY;
     for (int s = 0; s < splits; ++s) M = fmaxf(M, a.part_ml[s * rows + row].x);
-    float acc[D / 64] = {}, lsum = 0.0f;
+    float acc[4] = {}, lsum = 0.0f;   // dims lane, lane + 64, ..
     if (M != -INFINITY) {
         for (int s = 0; s < splits; ++s) {
             const float2 ml = a.part_ml[s * rows + row];
             const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
             lsum += w * ml.y;
-            const float *po = a.part_o + (s * rows + row) * D;
+            const float *po = a.part_o + (s * rows + row) * a.dim;
 #pragma unroll
-            for (int j = 0; j < D / 64; ++j) acc[j] += w * po[64 * j + lane];
+            for (int j = 0; j < 4; ++j)
+                if (64 * j + lane < a.dim) acc[j] += w * po[64 * j + lane];
         }
     }
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
-    // row = (batch, query, head): the output row of the same index, D floats
-    float *out = reinterpret_cast<float *>(a.o) + row * D;
+    // row = (batch, query, head): the output row of the same index, dim floats
+    float *out = reinterpret_cast<float *>(a.o) + row * a.dim;
 #pragma unroll
-    for (int j = 0; j < D / 64; ++j) out[64 * j + lane] = acc[j] * inv;
+    for (int j = 0; j < 4; ++j)
+        if (64 * j + lane < a.dim) out[64 * j + lane] = acc[j] * inv;
 }
 
-// f32 MultiHeadAttention on prefill_f32_kernel: head dim 128 or 64, at least 16 query
+// The head dim D of the kernel that serves a head dim: the least that holds it.  A dim of
+// 96 runs on the kernel of 96 (6 of 8 k-steps, 3 of 4 output blocks) rather than padded
+// to 128; between 129 and 255 the padding of 256 still beats the general kernel.  Bound
+// by the S, softmax and P.V phases of a tile as at 128, plus the P low halves' MFMAs; before,
+// the general kernel (a thread per key, row-strided 2-byte loads, no MFMA): f16 2 x 700 of
+// 1500 x 16 heads of 96 causal 9680 -> 33 us, bf16 1014 -> 34, f32 1473 -> 150; 2 x 512 x 8
+// of 256 f16 2068 -> 34, bf16 221 -> 34, f32 333 -> 135; FlashAttention 1000 x 1000 of 80
+// f16 929 -> 22, bf16 639 -> 22.  Errors against float64 are no larger than the general
+// kernel's in any of them (f16 2.1e-4, bf16 1.7e-3, f32 2.2e-7 -> 1.5e-7).
+template <int D_, bool PAD_> struct PfHeadDim {
+    static constexpr int D = D_;
+    static constexpr bool PAD = PAD_;
+};
+template <typename F> static void with_head_dim(int64_t dim, F f) {
+    if (dim == 64) f(PfHeadDim<64, false>{});
+    else if (dim == 128) f(PfHeadDim<128, false>{});
+    else if (dim < 64) f(PfHeadDim<64, true>{});
+    else if (dim <= 96) f(PfHeadDim<96, true>{});
+    else if (dim < 128) f(PfHeadDim<128, true>{});
+    else f(PfHeadDim<256, true>{});
+}
+
+// f32 MultiHeadAttention on prefill_f32_kernel: head dims of 4 n up to 256, at least 16 query
 // rows, causal or not, with or without a sliding window and ALiBi.
 static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
-    if (m.dim != 128 && m.dim != 64) return false;
+    if (m.dim % 4 || m.dim > 256) return false;
     if (m.seq_q < 16) return false;
     if (m.seq_q > 0x3FFFFFFF || m.seq_k > 0x3FFFFFFF || m.shift > 0x3FFFFFFF || m.shift < -0x3FFFFFFF) return false;
-    if (m.kv_heads > 32768) return false;   // a 32-row K/V tile spans < 2^31 bytes
+    if (m.kv_heads * m.dim > 32768 * 128) return false;   // a 32-row K/V tile spans < 2^30 bytes
     const uintptr_t mask = 15;
     if ((reinterpret_cast<uintptr_t>(m.q) | reinterpret_cast<uintptr_t>(m.k) |
          reinterpret_cast<uintptr_t>(m.v) | reinterpret_cast<uintptr_t>(m.o)) & mask)
@@ -994,6 +1162,8 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     a.seq_k = (int)m.seq_k;
     a.heads = (int)m.heads;
     a.kv_heads = (int)m.kv_heads;
+    a.dim = (int)m.dim;
+    a.nan_rows = m.nan_rows;
     a.qtiles = (int)((m.seq_q + fa::BM - 1) / fa::BM);
     a.causal = m.causal;
     a.shift = (int)m.shift;
@@ -1003,6 +1173,14 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     a.alibi_s = m.alibi != 0.0f ? m.alibi / m.scale : 0.0f;
     a.xcd_map = ((a.batch * a.kv_heads) % 8 == 0) ? 1 : 0;
     a.scale_log2 = m.scale * 1.4426950408889634f;
+    if (m.dim != 64 && m.dim != 128) {
+        // the padded kernels add the scale's low part; it is kept positive, so a masked
+        // score's -inf stays -inf through both products
+        const double exact = (double)m.scale * 1.4426950408889634;
+        a.scale_log2 = (float)exact;
+        if ((double)a.scale_log2 >= exact) a.scale_log2 = std::nextafter(a.scale_log2, 0.0f);
+        a.scale_log2_lo = (float)(exact - (double)a.scale_log2);
+    }
     const bool gen = a.window > 0 || a.alibi_s != 0.0f;   // the kernel with the window / ALiBi code
     const int64_t blocks = (int64_t)a.qtiles * a.batch * a.heads;
     if (blocks > 0x7FFFFFFF) return false;
@@ -1017,6 +1195,11 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     // (43 unsplit), 640 x 4 x 64 47.5 against 22.1.  From 24 blocks this kernel wins
     // unsplit too (384 x 8 x 64: 32.9 against 36.0, 4 x 128 x 8 x 64: 15.0 against 24.5)
     if (blocks < 24 && (!a.causal || ktiles < 8 || capturing)) return false;
+    // other head dims than 64 and 128: from 2048 rows (batch x queries x heads) on, where the
+    // general kernel's one block per row needs more than one round (2 x 21 x 12 rows over
+    // 173 keys of 96: 10.6 there against 24.9 here; 2 x 60 x 8 over 1500 keys of 256: 218
+    // against 107, 2 x 200 x 16 over 200 keys of 40: 75 against 21)
+    if (m.dim != 64 && m.dim != 128 && m.batch * m.seq_q * m.heads < 2048 && ktiles < 16) return false;
     // Small grids split each block's key range over blockIdx.y, partials in the
     // library's scratch: the longest block's key loop, the critical path, shrinks with
     // the split count.  Causal grids of under two blocks per CU aim at four blocks per
@@ -1032,6 +1215,12 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     else if (!a.causal && blocks < cus)
         splits = std::max<int64_t>(1, std::min<int64_t>((2 * cus + blocks - 1) / blocks, ktiles / 16));
     if (capturing) splits = 1;
+    auto launch = [&](dim3 grid) {
+        with_head_dim(m.dim, [&](auto d) {
+            if (gen) prefill_f32_kernel<d.D, true, d.PAD><<<grid, 256, 0, s>>>(a);
+            else prefill_f32_kernel<d.D, false, d.PAD><<<grid, 256, 0, s>>>(a);
+        });
+    };
     if (splits > 1) {
         a.split_tiles = (int)((ktiles + splits - 1) / splits);
         splits = (ktiles + a.split_tiles - 1) / a.split_tiles;
@@ -1047,39 +1236,26 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
         a.part_ml = reinterpret_cast<float2 *>(a.part_o + splits * rows * m.dim);
         const dim3 grid((unsigned)blocks, (unsigned)splits);
         const unsigned cblocks = (unsigned)((rows + 3) / 4);
-        if (m.dim == 128) {
-            if (gen) prefill_f32_kernel<128, true><<<grid, 256, 0, s>>>(a);
-            else prefill_f32_kernel<128, false><<<grid, 256, 0, s>>>(a);
-            prefill_f32_combine_kernel<128><<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
-        } else {
-            if (gen) prefill_f32_kernel<64, true><<<grid, 256, 0, s>>>(a);
-            else prefill_f32_kernel<64, false><<<grid, 256, 0, s>>>(a);
-            prefill_f32_combine_kernel<64><<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
-        }
+        launch(grid);
+        prefill_f32_combine_kernel<<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
         const int rc = check_launch("prefill f32 mfma split");
         const int fin = lease.finish();
         *status = rc ? rc : fin;
         return true;
     }
-    if (m.dim == 128) {
-        if (gen) prefill_f32_kernel<128, true><<<(unsigned)blocks, 256, 0, s>>>(a);
-        else prefill_f32_kernel<128, false><<<(unsigned)blocks, 256, 0, s>>>(a);
-    } else {
-        if (gen) prefill_f32_kernel<64, true><<<(unsigned)blocks, 256, 0, s>>>(a);
-        else prefill_f32_kernel<64, false><<<(unsigned)blocks, 256, 0, s>>>(a);
-    }
+    launch(dim3((unsigned)blocks));
     *status = check_launch("prefill f32 mfma");
     return true;
 }
 
 bool launch_prefill_mfma(const MhaArgs &m, int dtype, hipStream_t s, int *status) {
     if (dtype == PUTER_F32) return launch_prefill_f32(m, s, status);
-    if ((dtype != PUTER_BF16 && dtype != PUTER_F16) || (m.dim != 128 && m.dim != 64)) return false;
-    if (m.dim == 64 && m.seq_q == 1) return false;   // one query row: the general kernel (no 127 padding rows)
+    if ((dtype != PUTER_BF16 && dtype != PUTER_F16) || m.dim % 8 || m.dim > 256) return false;
+    if (m.dim != 128 && m.seq_q == 1) return false;   // one query row: the general kernel (no 127 padding rows)
     if (m.seq_q > 0x3FFFFFFF || m.seq_k > 0x3FFFFFFF || m.shift > 0x3FFFFFFF || m.shift < -0x3FFFFFFF)
         return false;
-    // 32-bit buffer offsets: one 64-row tile of K/V must span < 2^31 bytes
-    if (m.kv_heads > 65536) return false;
+    // 32-bit buffer offsets: one 64-row tile of K/V must span at most 2^30 bytes
+    if (m.kv_heads * m.dim > 65536 * 128) return false;
     const uintptr_t mask = 15;
     if ((reinterpret_cast<uintptr_t>(m.q) | reinterpret_cast<uintptr_t>(m.k) |
          reinterpret_cast<uintptr_t>(m.v) | reinterpret_cast<uintptr_t>(m.o)) & mask)
@@ -1094,6 +1270,8 @@ bool launch_prefill_mfma(const MhaArgs &m, int dtype, hipStream_t s, int *status
     a.seq_k = (int)m.seq_k;
     a.heads = (int)m.heads;
     a.kv_heads = (int)m.kv_heads;
+    a.dim = (int)m.dim;
+    a.nan_rows = m.nan_rows;
     a.qtiles = (int)((m.seq_q + fa::BM - 1) / fa::BM);
     a.causal = m.causal;
     a.shift = (int)m.shift;
@@ -1107,23 +1285,15 @@ bool launch_prefill_mfma(const MhaArgs &m, int dtype, hipStream_t s, int *status
     if (blocks > 0x7FFFFFFF) return false;
     const bool bf = dtype == PUTER_BF16, win = a.window > 0 || a.alibi_s != 0.0f;
     const dim3 grid((unsigned)blocks);
-    if (m.dim == 128) {
+    with_head_dim(m.dim, [&](auto d) {
         if (win) {
-            if (bf) prefill_kernel<PUTER_BF16, 128, true><<<grid, 256, 0, s>>>(a);
-            else prefill_kernel<PUTER_F16, 128, true><<<grid, 256, 0, s>>>(a);
+            if (bf) prefill_kernel<PUTER_BF16, d.D, true, d.PAD><<<grid, 256, 0, s>>>(a);
+            else prefill_kernel<PUTER_F16, d.D, true, d.PAD><<<grid, 256, 0, s>>>(a);
         } else {
-            if (bf) prefill_kernel<PUTER_BF16, 128, false><<<grid, 256, 0, s>>>(a);
-            else prefill_kernel<PUTER_F16, 128, false><<<grid, 256, 0, s>>>(a);
+            if (bf) prefill_kernel<PUTER_BF16, d.D, false, d.PAD><<<grid, 256, 0, s>>>(a);
+            else prefill_kernel<PUTER_F16, d.D, false, d.PAD><<<grid, 256, 0, s>>>(a);
         }
-    } else {
-        if (win) {
-            if (bf) prefill_kernel<PUTER_BF16, 64, true><<<grid, 256, 0, s>>>(a);
-            else prefill_kernel<PUTER_F16, 64, true><<<grid, 256, 0, s>>>(a);
-        } else {
-            if (bf) prefill_kernel<PUTER_BF16, 64, false><<<grid, 256, 0, s>>>(a);
-            else prefill_kernel<PUTER_F16, 64, false><<<grid, 256, 0, s>>>(a);
-        }
-    }
+    });
     *status = check_launch("prefill mfma");
     return true;
 }

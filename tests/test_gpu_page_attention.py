@@ -363,6 +363,68 @@ def test_mha_random_shapes(backend, dt, case):
         assert_close(got[i], ref, TOL[dt], elem_tol=None, what=f"random mha {case} batch {i}")
 
 
+@pytest.mark.parametrize("dt", [O.BF16, O.F16, O.F32])
+@pytest.mark.parametrize("d,sq,sk,h,kvh,causal,window,alibi", [
+    (8, 140, 200, 12, 3, True, 0, 0.0),       # one chunk of a 64-dim row
+    (40, 130, 70, 12, 12, True, 0, 0.0),      # seqK < seqQ: rows that see no key
+    (72, 257, 300, 8, 2, False, 0, 0.0),      # the kernel of 96: a partly filled k-step
+    (80, 200, 500, 16, 4, True, 60, 0.0),
+    (96, 190, 330, 16, 16, True, 0, 0.0),     # the kernel of 96, filled
+    (112, 128, 128, 24, 24, False, 0, 0.0625),
+    (136, 129, 260, 12, 4, True, 0, 0.0),     # the least dim of the kernel of 256
+    (256, 300, 321, 12, 3, True, 100, -0.125),
+    (256, 384, 130, 8, 8, False, 0, 0.0),
+])
+def test_mha_other_head_dims(backend, dt, d, sq, sk, h, kvh, causal, window, alibi):
+    """Head dims other than 64 and 128 on the MFMA kernels, batched: dims past the head
+    dim are zero chunks of the tile, never the neighbouring head's values, so K, V and Q
+    of the other heads hold NaN where a wrong chunk would read them (batch 1's slabs)."""
+    import puter_amd
+    std = d ** -0.25
+    q = seeded(700 + d, (2, sq, h * d), 0.0, std)
+    k = seeded(701 + d, (2, sk, kvh * d), 0.0, std)
+    v = seeded(702 + d, (2, sk, kvh * d))
+    if kvh > 1:
+        v[1, :, d:] = np.nan     # kv head 0's outputs must stay finite
+    q, k, v = (encode(x, dt) for x in (q, k, v))
+    out = empty_dev((2, sq, h * d), NP[dt])
+    cfg = puter_amd.MultiHeadAttentionConfig(h, d, causal, window, alibi, kvh)
+    backend.MultiHeadAttentionBatched(cfg, to_dev(q), to_dev(k), to_dev(v), out, 2, sq, sk, dt)
+    got = decode(to_host(out, NP[dt]), dt)
+    O.set_threads(8)
+    for i in range(2):
+        ref = decode(O.mha(q[i], k[i], v[i], h, d, causal=causal, kv_heads=kvh, window=window, alibi=alibi,
+                           dtype=dt), dt)
+        n = h // kvh * d if i == 1 and kvh > 1 else h * d
+        assert np.isfinite(got[i][:, :n]).all()
+        assert_close(got[i][:, :n], ref[:, :n], TOL[dt], elem_tol=None, what=f"mha d {d} batch {i}")
+
+
+@pytest.mark.parametrize("dt", [O.BF16, O.F16, O.F32])
+@pytest.mark.parametrize("d", [40, 96, 256])
+def test_mha_other_head_dims_infinite_values(backend, dt, d):
+    """Values that are not finite reach only the rows that see them: a NaN row at the last
+    key (visible to the last query alone, though every query of its tile multiplies it by a
+    zero probability) and an infinity at key 3, dim 5 (an infinity in that dim, whatever
+    the probabilities' low halves are)."""
+    import puter_amd
+    sq = sk = 200
+    h = 12
+    q, k = (encode(seeded(720 + i, (sq, h * d), 0.0, d ** -0.25), dt) for i in range(2))
+    v = seeded(722, (sk, h * d))
+    bad = v.copy()
+    bad[-1], bad[3, 5] = np.nan, np.inf
+    out = empty_dev((sq, h * d), NP[dt])
+    cfg = puter_amd.MultiHeadAttentionConfig(h, d, True, 0, 0.0, h)
+    backend.MultiHeadAttention(cfg, to_dev(q), to_dev(k), to_dev(encode(bad, dt)), out, sq, sk, dt)
+    got = decode(to_host(out, NP[dt]), dt)
+    ref = decode(O.mha(q, k, encode(v, dt), h, d, causal=True, dtype=dt), dt)
+    assert np.isnan(got[-1]).all()
+    assert np.isposinf(got[3:-1, 5]).all()
+    got[3:, 5] = ref[3:, 5]
+    assert_close(got[:-1], ref[:-1], TOL[dt], elem_tol=None, what=f"mha d {d} with NaN and inf values")
+
+
 @pytest.mark.parametrize("dt", [O.BF16, O.F16])
 @pytest.mark.parametrize("b,sk,h,kvh,causal,window", [
     (1, 4096, 32, 8, True, 0),     # configs[4]'s heads at one sequence's full context
