@@ -17,7 +17,9 @@
  *   - the caller owns every buffer (workspaces included, see
  *     puter_hip_paged_decode_workspace_bytes).  The one allocation the library
  *     makes itself is a split-K scratch shared by puter_hip_matmul (16-bit
- *     formats with at most 512 rows or under two rounds of 128x128 tiles, F32
+ *     formats with at most 512 rows or under two rounds of 128x128 tiles, or of
+ *     sizes or alignments that the 16-byte copies cannot take (which run unsplit
+ *     where the scratch has no room), F32
  *     outputs of fewer 128x128 tiles than the device has CUs, when K is split
  *     across blocks rather than inside them) and
  *     puter_hip_multi_head_attention[_batched] with seq_q == 1 (bf16 / f16 at
@@ -377,7 +379,8 @@ PUTER_API int puter_hip_quant(void *dst, const void *src, int64_t count, float s
 /* ------------------------------------------------------------------------ */
 /* out[rows, cols] = left[rows, inner] . right[inner, cols], row-major, in F32, F64,
  * BF16 or F16 (16-bit formats accumulate in f32 and round once).  BF16 / F16 with
- * cols % 8 == 0, inner % 8 == 0 and 16-byte aligned buffers run on MFMA; with at
+ * at least 8 columns run on MFMA, whatever their sizes and alignment (fastest with
+ * cols % 8 == 0, inner % 8 == 0 and 16-byte aligned buffers); with at
  * most 512 rows they split `inner` across blocks and keep f32 partials in the
  * library's per-device scratch (calls on different streams are ordered on the
  * device by an event); so does F32 when the output has fewer than 256 64x64

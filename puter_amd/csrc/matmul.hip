@@ -34,8 +34,10 @@
 // to XCDs in 4 x 8 groups (consecutive block ids run round-robin over the 8
 // XCDs), so the blocks an XCD runs at once share their A and B panels in its L2.
 // Requirements of the MFMA path: N % 8 == 0, K % 8 == 0, 16-byte aligned
-// buffers, 256 * K * 2 and BK * N * 2 below 2^31; other shapes take the generic
-// kernel (one thread per output, f32 accumulation in index order).
+// buffers, 256 * K * 2 and BK * N * 2 below 2^31; at most 32 rows, and the shapes
+// and alignments these exclude, take the rows kernel (16-byte loads into registers
+// at any element); fewer than 8 columns the generic kernel (one thread per output, f32
+// accumulation in index order).
 //
 // f32: small outputs of moderate depth take the small kernel (32 x 32 or 16 x 16
 // tiles, K split over the 8 waves of each block on the f32 MFMA); other shapes with K
@@ -741,6 +743,210 @@ __global__ __launch_bounds__(512) void matmul16_small_kernel(uint16_t *__restric
     }
 }
 
+// ------------------------------------------- a few rows, or any shape, 16-bit --
+// The rows kernel: at most 32 rows (a decode step's projections and output head), and
+// every shape and alignment that the 16-byte copies of the other MFMA kernels cannot take.
+// Bound by streaming `right` once.  A 256-thread block takes 128 columns, 16 MT rows and a
+// run of K; its 4 waves take the 32-deep tiles w, w + 4, .. of the run and add their sums
+// in LDS.  Nothing is staged: in a tile lane l = 16 q + i loads the 8 x 8 elements of rows
+// 8 q .. + 7, columns 8 i .. + 7 as eight 16-byte loads (each instruction whole 256-byte row
+// pieces; 64-byte pieces, which would let a block of 32 columns take all of K, stream at
+// half the rate: reading 117 MB 34 us against 18), pairs the rows' halves with v_perm (32
+// for 64 elements) and feeds column 8 i + j to v_mfma_f32_16x16x32 number j as lane l's
+// k-run; the other operand is a row of `left` at the same k's, one 16-byte load a tile and
+// 16 rows.  One tile's loads in flight at 106 registers (four blocks a CU) beat two at 192
+// (1 x 4096 x 4096 9.7 us against 24).  Global loads of 16 bytes need no alignment on
+// gfx950, so any N >= 8 and any K, and buffers at any element, run here: a lane whose
+// columns would pass N takes the last 8 (columns that two lanes share get the same sums),
+// rows past K are replaced by zeros.  Misaligned rows stream at about 0.8 of the aligned
+// rate (1 x 4096 x 32001 61 us, 4.3 TB/s; the generic kernel took 33 x 4096 x 32001 in
+// 3810 us, 64.6 now, and 2000 x 4096 x 14337 runs at 300 TFLOP/s).
+// Runs: up to 16, so that small matrices fill the chip too (see rows_chunks).  A block
+// writes its sums to the split-K scratch with device-scope stores and counts itself in; the
+// last of a tile's blocks adds the runs in order (so the result does not depend on which
+// came last) and stores the rounded result: no second launch (whose gap and start cost 4 us).
+// No cache is written back or invalidated for this (a fence per block did, and cost 15 to
+// 230 us): the sums are stored and loaded past the L2s of the XCDs (sc1), where the counter's
+// atomics are performed too, and each wave waits for its stores to be there before its
+// block counts itself in.
+typedef float rw_f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kRwCols = 128, kRwDepth = 32, kRwWaves = 4, kRwRows = 16, kRwPad = kRwCols + 4;
+constexpr int kRwMaxTiles = 16384;   // column tiles of a split launch, at most
+// per device: the column tiles' arrival counters, zero between launches (the last block's
+// atomicInc wraps to zero): one set beside the growable scratch, one beside the no-alloc
+// entry point's array, each used by one launch at a time like the scratch it stands by
+static __device__ unsigned rw_arrived[2][kRwMaxTiles];
+
+__device__ __forceinline__ uint4 ld16(const uint16_t *p) {   // 16 bytes at any element
+    uint4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+typedef unsigned int rw_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 ld16_stream(const uint16_t *p) {
+    const rw_u32x4 v = __builtin_nontemporal_load(reinterpret_cast<const rw_u32x4 *>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+// 8 elements of a row from k on, zeros from K on
+__device__ __forceinline__ uint4 ld16_tail(const uint16_t *row, int64_t k, int64_t K) {
+    if (k + 8 <= K) return ld16(row + k);
+    uint32_t w[4] = {};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (k + i < K) w[i >> 1] |= (uint32_t)row[k + i] << (16 * (i & 1));
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+template <int DT>
+__device__ __forceinline__ rw_f32x4 rw_mfma(uint4 a, uint4 b, rw_f32x4 c) {
+    if constexpr (DT == PUTER_BF16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(mm_bf16x8, a), __builtin_bit_cast(mm_bf16x8, b), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(mm_f16x8, a), __builtin_bit_cast(mm_f16x8, b), c, 0, 0, 0);
+}
+
+struct RwArgs {
+    uint16_t *out;
+    const uint16_t *a, *b;
+    float *ws;       // [tile, row tile][chunk][rows][128] sums when split
+    int M, tiles, chunks, mtiles, set;
+    int64_t K, N, kc;   // kc: K per chunk, a multiple of kRwWaves * kRwDepth
+};
+
+template <int DT, int MT>
+__global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void matmul_rows_kernel(RwArgs p) {
+    __shared__ float part[kRwWaves][kRwRows][kRwPad];
+    __shared__ int is_last;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i = lane & 15, q = lane >> 4;
+    // consecutive blocks go round-robin over the XCDs: the row tiles of one column tile
+    // run one after another on one XCD, whose L2 keeps their columns of `right`
+    const unsigned id = blockIdx.x, mt0 = (id >> 3) % p.mtiles;
+    const unsigned u = (id >> 3) / p.mtiles * 8 + (id & 7);
+    if (u >= (unsigned)p.tiles * p.chunks) return;
+    const int tile = u % p.tiles, chunk = u / p.tiles;
+    const int m0 = mt0 * (kRwRows * MT), rows = std::min(p.M - m0, kRwRows * MT);
+    const int64_t K = p.K, N = p.N, n0 = (int64_t)tile * kRwCols;
+    const int64_t kb = (int64_t)chunk * p.kc, ke = std::min(K, kb + p.kc);
+    const uint16_t *const wp = p.b + std::min<int64_t>(n0 + 8 * i, N - 8);
+    const uint16_t *xp[MT];   // rows past M: computed, not stored
+#pragma unroll
+    for (int t = 0; t < MT; ++t) xp[t] = p.a + (int64_t)std::min(m0 + 16 * t + i, p.M - 1) * K;
+
+    struct Tile {
+        uint4 w[8], x[MT];
+    };
+    rw_f32x4 acc[MT][8];
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[t][j] = (rw_f32x4){};
+    auto compute = [&](const Tile &t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            uint32_t lo[4], hi[4];   // columns 2 d and 2 d + 1: the low and high halves of the 8 rows
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const uint32_t v0 = (&t.w[2 * h].x)[d], v1 = (&t.w[2 * h + 1].x)[d];
+                lo[h] = __builtin_amdgcn_perm(v1, v0, 0x05040100u);
+                hi[h] = __builtin_amdgcn_perm(v1, v0, 0x07060302u);
+            }
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                acc[m][2 * d] = rw_mfma<DT>(t.x[m], make_uint4(lo[0], lo[1], lo[2], lo[3]), acc[m][2 * d]);
+                acc[m][2 * d + 1] = rw_mfma<DT>(t.x[m], make_uint4(hi[0], hi[1], hi[2], hi[3]), acc[m][2 * d + 1]);
+            }
+        }
+    };
+    // one tile's loads in flight per wave, four or five blocks a CU
+    constexpr int64_t STEP = kRwWaves * kRwDepth;
+    int64_t k0 = kb + wave * kRwDepth;
+    const int64_t kfull = std::min(ke, K - (K % kRwDepth));   // ends of the whole tiles
+    const uint16_t *w = wp + (k0 + 8 * q) * N;
+    for (; k0 < kfull; k0 += STEP, w += STEP * N) {
+        Tile t;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) t.x[m] = ld16(xp[m] + k0 + 8 * q);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) t.w[r] = ld16_stream(w + r * N);
+        compute(t);
+    }
+    if (k0 < ke) {   // the tile that K cuts, the last of one wave
+        Tile t;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) t.x[m] = ld16_tail(xp[m], k0 + 8 * q, K);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+            const int64_t k = k0 + 8 * q + r;
+            const uint4 v = ld16(wp + std::min<int64_t>(k, K - 1) * N);
+            t.w[r] = k < K ? v : make_uint4(0, 0, 0, 0);
+        }
+        compute(t);
+    }
+    // four columns of a row per thread
+    auto put = [&](int o, float4 t) __attribute__((always_inline)) {
+        const int m = o >> 5, col = (o & 31) * 4;
+        uint16_t *dst = p.out + (int64_t)(m0 + m) * N + std::min<int64_t>(n0 + (col & ~7), N - 8) + (col & 7);
+        const uint32_t h0 = Elem<DT>::store(t.x), h1 = Elem<DT>::store(t.y), h2 = Elem<DT>::store(t.z), h3 = Elem<DT>::store(t.w);
+        const uint2 v = make_uint2(h0 | (h1 << 16), h2 | (h3 << 16));
+        __builtin_memcpy(dst, &v, 8);
+    };
+    const int total = rows * (kRwCols / 4);   // float4s
+    // this tile's sums, [chunk][row][128]: stored and loaded at the agent's coherence point
+    // (sc1), past the XCDs' own L2s
+    constexpr int SC1 = 16;
+    const int slot = tile * p.mtiles + mt0;
+    const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(p.ws + (int64_t)slot * p.chunks * (std::min(p.M, kRwRows * MT) * kRwCols)), (short)0, p.chunks * total * 16, mm::BUF_WORD3);
+    // lane (i, q), register r of acc[t][j]: row 16 t + 4 q + r, column 8 i + j of the tile
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        if (16 * t >= rows) break;
+        if (t) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (16 * t + 4 * q + r < rows) {
+                float *dst = &part[wave][4 * q + r][8 * i];
+                *reinterpret_cast<float4 *>(dst) = make_float4(acc[t][0][r], acc[t][1][r], acc[t][2][r], acc[t][3][r]);
+                *reinterpret_cast<float4 *>(dst + 4) = make_float4(acc[t][4][r], acc[t][5][r], acc[t][6][r], acc[t][7][r]);
+            }
+        __syncthreads();
+        const int n = std::min(rows - 16 * t, 16) * (kRwCols / 4);
+        for (int o = tid; o < n; o += 256) {
+            const float *src = &part[0][o >> 5][(o & 31) * 4];
+            float4 v = *reinterpret_cast<const float4 *>(src);
+#pragma unroll
+            for (int w = 1; w < kRwWaves; ++w) {
+                const float4 u = *reinterpret_cast<const float4 *>(src + w * kRwRows * kRwPad);
+                v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
+            }
+            const int at = o + 16 * t * (kRwCols / 4);
+            if (p.chunks == 1) put(at, v);
+            else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(mm_u32x4, v), ws, (chunk * total + at) * 16, 0, SC1);
+        }
+    }
+    if (p.chunks == 1) return;
+    __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's sums are at the coherence point
+    __syncthreads();
+    if (tid == 0) is_last = atomicInc(&rw_arrived[p.set][slot], (unsigned)p.chunks - 1) == (unsigned)p.chunks - 1;
+    __syncthreads();
+    if (!is_last) return;
+    for (int o = tid; o < total; o += 256) {
+        float4 t = make_float4(0, 0, 0, 0);
+        for (int z0 = 0; z0 < p.chunks; z0 += 8) {   // eight runs' loads in flight, added in order
+            float4 v[8];
+#pragma unroll
+            for (int z = 0; z < 8; ++z)   // (past the last run: past the buffer, zeros)
+                v[z] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(ws, ((z0 + z) * total + o) * 16, 0, SC1));
+#pragma unroll
+            for (int z = 0; z < 8; ++z) {
+                t.x += v[z].x; t.y += v[z].y; t.z += v[z].z; t.w += v[z].w;
+            }
+        }
+        put(o, t);
+    }
+}
+
 // ------------------------------------ skinny (M <= 512) and small outputs --
 // Decode-time projections (a few rows against a large weight matrix) are bound by
 // streaming `right` once; the kernel also serves outputs too small to fill the
@@ -977,6 +1183,19 @@ static int scratch_acquire(SplitScratch &sc, size_t need, hipStream_t s) {
     return PUTER_OK;
 }
 
+// Whether s is recording a graph (or cannot be asked), and the bytes its device's scratch
+// holds, which is all a capture can use.
+static bool scratch_capturing(hipStream_t s, size_t *held) {
+    int dev = 0;
+    bool capturing = true;
+    *held = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return true;
+    std::lock_guard<std::mutex> g(g_split_scratch[dev].mu);
+    if (stream_capturing(s, &capturing) != PUTER_OK) return true;
+    *held = g_split_scratch[dev].bytes;
+    return capturing;
+}
+
 ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
@@ -1056,6 +1275,82 @@ struct PartialsTarget {
     float *fixed = nullptr;
 };
 
+// Runs of K of the rows kernel: toward one block per CU (200 of 256 is near enough: 16 x
+// 4096 x 14336, 112 tiles, 24.9 us in 2 runs, 25.5 in 4; 32 tiles 11.2 in 8, 14.3 in 4), each
+// run two 128-deep steps or more, or one step in at most 8 runs (1 x 768 x 768 5.4 -> 4.5).
+static int64_t rows_chunks(int64_t blocks, int64_t K) {
+    const int64_t steps = (K + kRwWaves * kRwDepth - 1) / (kRwWaves * kRwDepth);
+    int64_t c = 1;
+    while (c < 16 && c * blocks < 200) c *= 2;
+    return std::min<int64_t>(c, std::max<int64_t>(steps / 2, std::min<int64_t>(steps, 8)));
+}
+
+// Runs that the skinny kernel would use (see launch_skinny).
+static int64_t skinny_chunks(int64_t M, int64_t K, int64_t N, int64_t min_depth) {
+    const int64_t tiles = ((N + sk::BN - 1) / sk::BN) * ((M + sk::BM - 1) / sk::BM);
+    const int64_t slices = (K + sk::BK - 1) / sk::BK;
+    int64_t chunks = std::min<int64_t>(std::max<int64_t>(512 / tiles, 1), slices);
+    chunks = std::min<int64_t>(chunks, 8);
+    if (min_depth > 0) chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, K / min_depth));
+    const int64_t per = (slices + chunks - 1) / chunks;
+    return (slices + per - 1) / per;
+}
+
+// general: the shape or alignment is one that only the generic kernel (which needs no
+// scratch) would take otherwise, so a split that finds no room runs unsplit; else, under
+// stream capture, the call is held to what the skinny kernel asked of the scratch: it fails
+// where that did not fit, and otherwise takes as many runs as fit.
+template <int DT, int MT>
+static int launch_rows_mt(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s,
+                          PartialsTarget tgt, bool general) {
+    const int64_t tiles = (N + kRwCols - 1) / kRwCols, mtiles = (M + kRwRows * MT - 1) / (kRwRows * MT);
+    constexpr int64_t STEP = kRwWaves * kRwDepth;
+    const int64_t steps = (K + STEP - 1) / STEP;
+    if ((tiles * 16 + 8) * mtiles > 0x7FFFFFFF || M > 0x3FFFFFFF) return 1;
+    const int64_t unit = tiles * mtiles * std::min<int64_t>(M, kRwRows * MT) * kRwCols * (int64_t)sizeof(float);   // sums of one run
+    int64_t chunks = tiles * mtiles <= kRwMaxTiles ? rows_chunks(tiles * mtiles, K) : 1;
+    chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, (int64_t)noalloc::kScratchBytes / unit));
+    if (chunks > 1 && !tgt.fixed) {
+        size_t held = 0;
+        if (scratch_capturing(s, &held) && held < (size_t)(chunks * unit)) {
+            const int64_t old = skinny_chunks(M, K, N, 0);
+            const size_t need = old > 1 ? (size_t)(old * M * N) * sizeof(float) : 0;
+            if (general || held >= need) chunks = std::max<int64_t>(1, (int64_t)held / unit);
+        }
+    }
+    const int64_t per = (steps + chunks - 1) / chunks;
+    chunks = (steps + per - 1) / per;
+    RwArgs p{static_cast<uint16_t *>(out), static_cast<const uint16_t *>(left), static_cast<const uint16_t *>(right), tgt.fixed,
+             (int)M, (int)tiles, (int)chunks, (int)mtiles, tgt.fixed ? 1 : 0, K, N, per * STEP};
+    auto launch = [&] {
+        const int64_t blocks = (tiles * p.chunks + 7) / 8 * 8 * mtiles;
+        matmul_rows_kernel<DT, MT><<<(unsigned)blocks, 256, 0, s>>>(p);
+        return check_launch("matmul rows");
+    };
+    if (chunks == 1 || tgt.fixed) return launch();
+    ScratchLease lease((size_t)(chunks * unit), s);
+    if (lease.status()) {
+        if (!general) return lease.status();
+        p.chunks = 1;
+        p.kc = steps * STEP;
+        return launch();
+    }
+    p.ws = static_cast<float *>(lease.ptr());
+    const int rc = launch();
+    const int fin = lease.finish();
+    return rc ? rc : fin;
+}
+
+// Row tiles of 16, 32 or 64.  Returns 1 when the shape is not one of the rows kernel's.
+template <int DT>
+static int launch_rows(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s,
+                       PartialsTarget tgt, bool general) {
+    if (N < 8) return 1;
+    if (M <= 16) return launch_rows_mt<DT, 1>(out, left, right, M, K, N, s, tgt, general);
+    if (M <= 32) return launch_rows_mt<DT, 2>(out, left, right, M, K, N, s, tgt, general);
+    return launch_rows_mt<DT, 4>(out, left, right, M, K, N, s, tgt, general);
+}
+
 // min_depth > 0: chunks of K at least min_depth deep (fewer chunks otherwise).
 template <int DT>
 static int launch_skinny(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N,
@@ -1067,11 +1362,8 @@ static int launch_skinny(void *out, const void *left, const void *right, int64_t
     // as many chunks as keep the grid within one wave of 512 blocks (2 per CU): a
     // partial second wave would run at a fraction of the bandwidth; at most 8, as
     // the partials written and summed grow with the chunk count (against at most
-    // 64: 64x4096x4096 18.1 -> 14.7 us, 32x2048x2048 17.2 -> 8.2, 1x4096x4096
-    // 11.0 -> 10.1; 4 lost on 64x14336x4096, 41.4 against 29.0)
-    int64_t chunks = std::min<int64_t>(std::max<int64_t>(512 / (tiles_m * tiles_n), 1), slices);
-    chunks = std::min<int64_t>(chunks, 8);
-    if (min_depth > 0) chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, K / min_depth));
+    // 64: 64x4096x4096 18.1 -> 14.7 us; 4 lost on 64x14336x4096, 41.4 against 29.0)
+    int64_t chunks = skinny_chunks(M, K, N, min_depth);
     const int64_t per = (slices + chunks - 1) / chunks;  // slices per chunk
     chunks = (slices + per - 1) / per;
     SkArgs p{static_cast<const uint16_t *>(left), static_cast<const uint16_t *>(right), static_cast<uint16_t *>(out),
@@ -1133,7 +1425,16 @@ static bool mfma_small_tiles(int64_t M, int64_t N) {
 template <int DT>
 static int launch_matmul16(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N,
                            hipStream_t s, PartialsTarget tgt) {
-    if (N % 8 == 0 && K % 8 == 0 && aligned16(out) && aligned16(left) && aligned16(right)) {
+    // A few rows (a decode step's projections) take the rows kernel: against the skinny
+    // kernel and its reduce launch 1 x 4096 x 4096 14.1 -> 9.5 us, 1 x 4096 x 14336 25.2 ->
+    // 22.7, 16 x 14336 x 4096 35.0 -> 24.0, 32 x 4096 x 4096 15.4 -> 13.6; at 64 rows the
+    // skinny kernel wins (64 x 4096 x 14336: 33.1 against 35.3)
+    const bool fits = N % 8 == 0 && K % 8 == 0 && aligned16(out) && aligned16(left) && aligned16(right);
+    if (!fits || M <= 32) {
+        const int rc = launch_rows<DT>(out, left, right, M, K, N, s, tgt, !fits);
+        if (rc != 1) return rc;
+    }
+    if (fits) {
         // small outputs of moderate depth with a small right operand: K split inside
         // each block (as for f32; 128x512x512 7.5 -> 6.3 us, 256x1024x1024 17.5 ->
         // 10.0).  Its B reads are 2-byte gathers, so a few rows against a large

@@ -352,6 +352,62 @@ def test_matmul_f32_small_unaligned_left(backend):
     assert_close(got_u, O.matmul_f32(a, b), TOL[O.F32], elem_tol=1e-3, what="f32 matmul, unaligned A")
 
 
+@pytest.mark.parametrize("dt", [O.BF16, O.F16])
+@pytest.mark.parametrize("rows,inner,cols,shift", [
+    (1, 1, 9, 0), (1, 8, 8, 0), (2, 31, 129, 1), (4, 32, 4097, 0),
+    (16, 100, 127, 0), (16, 768, 1024, 3),     # one row tile of 16: the last columns shifted back, K cut
+    (17, 129, 128, 1), (32, 4104, 136, 0),     # 32: two column tiles in many runs of K
+    (33, 77, 1001, 0), (64, 31, 8, 1), (65, 260, 257, 5), (200, 1000, 333, 0),   # 64: several row tiles
+    (8, 14336, 64, 0), (31, 4096, 1025, 2),
+])
+def test_matmul_16bit_rows_kernel_exact(backend, dt, rows, inner, cols, shift):
+    """The rows kernel (at most 32 rows, or a shape or alignment the 16-byte copies of the
+    other kernels cannot take), bit for bit: integer operands keep every sum exact, so each
+    output is the exact product narrowed once.  Buffers start `shift` elements past a
+    16-byte boundary and end where an allocation of their own would: guard elements of the
+    output must stay.  Several calls in a row with other operands: the split-K sums and
+    arrival counters of one call are never seen by the next."""
+    import torch
+    for rep in range(4):
+        rng = np.random.default_rng(rows + 7 * inner + 3 * cols + rep)
+        ai = rng.integers(-2, 3, (rows, inner)).astype(np.float32)
+        bi = rng.integers(-2, 3, (inner, cols)).astype(np.float32)
+        want = O.from_f32((ai @ bi).astype(np.float32), dt)
+
+        def place(x):
+            buf = torch.zeros(x.size + shift, dtype=torch.int16, device="cuda")
+            buf[shift:] = to_dev(O.from_f32(x, dt)).view(-1)
+            return buf[shift:]
+        out = torch.full((rows * cols + shift + 8,), 0x7E55, dtype=torch.int16, device="cuda")
+        backend.Matmul(out[shift:], place(ai), place(bi), rows, inner, cols, dt)
+        got = to_host(out, np.uint16)
+        assert (got[:shift] == 0x7E55).all() and (got[shift + rows * cols:] == 0x7E55).all()
+        assert np.array_equal(got[shift:shift + rows * cols].reshape(rows, cols), want), (dt, rows, inner, cols, rep)
+
+
+def test_matmul_unaligned_captured_without_scratch(backend):
+    """A shape that only the rows kernel takes was never refused under stream capture (the
+    generic kernel needs no scratch): captured, it splits K only as far as the scratch held
+    allows, and its replays with new operands are exact."""
+    import torch
+    rows, inner, cols = 3, 4000, 1001
+    rng = np.random.default_rng(5)
+    a, b = (torch.zeros(n, dtype=torch.int16, device="cuda") for n in (rows * inner, inner * cols))
+    out = torch.empty(rows * cols, dtype=torch.int16, device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        backend.Matmul(out, a, b, rows, inner, cols, O.BF16)
+    for step in range(3):
+        ai = rng.integers(-2, 3, (rows, inner)).astype(np.float32)
+        bi = rng.integers(-2, 3, (inner, cols)).astype(np.float32)
+        a.copy_(to_dev(O.from_f32(ai, O.BF16)).view(-1))
+        b.copy_(to_dev(O.from_f32(bi, O.BF16)).view(-1))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(to_host(out, np.uint16).reshape(rows, cols), O.from_f32(ai @ bi, O.BF16)), step
+        (torch.randn(1 << 20, device="cuda") * 2).sum().item()
+
+
 @pytest.mark.parametrize("dt,np_dt", [(O.BF16, np.uint16), (O.F32, np.float32), (O.F64, np.float64)])
 def test_matmul_empty_inner_is_zero(backend, dt, np_dt):
     rows, cols = 5, 7   # odd element count
