@@ -12,10 +12,12 @@
 // written once (for the fused op, 8 B/elem of HBM traffic in bf16):
 //   - norm_row_kernel: a block per row, 1-8 16-byte vectors per thread per
 //     tensor (long rows, many rows);
-//   - norm_wave_kernel: one wave64 per row, 4 rows per 256-thread block, the row
-//     as VPL 16-byte vectors per lane (lane l owns vectors j*64 + l, so each
-//     wave-wide load is one contiguous 1 KiB burst); register-only butterflies.
-// Any other shape or alignment uses the generic block-per-row kernel, which
+//   - norm_wave_kernel (fused norms): one wave64 per row, 4 rows per 256-thread block, the
+//     row as VPL 16-byte vectors per lane (lane l owns vectors j*64 + l, so each
+//     wave-wide load is one contiguous 1 KiB burst); register-only butterflies;
+//   - norm_line_kernel: a block per row for few rows and for any other length and
+//     alignment.
+// Rows too long for a block's registers use the generic block-per-row kernel, which
 // re-reads the row from memory for each pass.
 #include "common.hpp"
 
@@ -99,7 +101,7 @@ __device__ __forceinline__ float apply_one(float h, float mean, float inv, float
 // SHARE (fused gated residual + RMSNorm/LayerNorm, the block's 4 rows in one
 // modulation batch): the gate row, gamma (and beta) are staged once per block
 // in LDS instead of being re-read from L2 by every wave.
-template <int DT, int OP, bool GR, int VPL, bool SHARE = false>
+template <int DT, int OP, int VPL, bool SHARE>
 __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
 #pragma clang fp contract(off)
     constexpr int N = Vec<DT>::N;
@@ -114,54 +116,48 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
     const int64_t batch = (live ? row : 0) / a.rows_per_batch;
 
     uint4 hv[VPL];
-    if constexpr (GR) {
-        const uint4 *res = reinterpret_cast<const uint4 *>(a.x) + row_vec;
-        const uint4 *br = reinterpret_cast<const uint4 *>(a.branch) + row_vec;
-        const uint4 *gate = reinterpret_cast<const uint4 *>(a.mod) +
-                            (size_t)(batch * a.mod_cols + a.gate_off) / N;
-        uint4 rv[VPL], bv[VPL], gv[VPL];
+    const uint4 *res = reinterpret_cast<const uint4 *>(a.x) + row_vec;
+    const uint4 *br = reinterpret_cast<const uint4 *>(a.branch) + row_vec;
+    const uint4 *gate = reinterpret_cast<const uint4 *>(a.mod) +
+                        (size_t)(batch * a.mod_cols + a.gate_off) / N;
+    uint4 rv[VPL], bv[VPL], gv[VPL];
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            rv[j] = ld_stream(res + j * 64 + lane);
-            bv[j] = ld_stream(br + j * 64 + lane);
-            if constexpr (!SHARE) gv[j] = gate[j * 64 + lane];
+    for (int j = 0; j < VPL; ++j) {
+        rv[j] = ld_stream(res + j * 64 + lane);
+        bv[j] = ld_stream(br + j * 64 + lane);
+        if constexpr (!SHARE) gv[j] = gate[j * 64 + lane];
+    }
+    if constexpr (SHARE) {
+        // the row loads above are in flight while the block fills the table
+        const int64_t b0 = ((int64_t)blockIdx.x * 4) / a.rows_per_batch;
+        const uint4 *g0 = reinterpret_cast<const uint4 *>(a.mod) + (size_t)(b0 * a.mod_cols + a.gate_off) / N;
+        const uint4 *gm = reinterpret_cast<const uint4 *>(a.scale);
+        const uint4 *bt = reinterpret_cast<const uint4 *>(a.bias);
+        for (int i = threadIdx.x; i < ROWV; i += 256) {
+            tbl[i] = g0[i];
+            tbl[ROWV + i] = gm[i];
+            if constexpr (OP == OP_LN) tbl[2 * ROWV + i] = bt[i];
         }
-        if constexpr (SHARE) {
-            // the row loads above are in flight while the block fills the table
-            const int64_t b0 = ((int64_t)blockIdx.x * 4) / a.rows_per_batch;
-            const uint4 *g0 = reinterpret_cast<const uint4 *>(a.mod) + (size_t)(b0 * a.mod_cols + a.gate_off) / N;
-            const uint4 *gm = reinterpret_cast<const uint4 *>(a.scale);
-            const uint4 *bt = reinterpret_cast<const uint4 *>(a.bias);
-            for (int i = threadIdx.x; i < ROWV; i += 256) {
-                tbl[i] = g0[i];
-                tbl[ROWV + i] = gm[i];
-                if constexpr (OP == OP_LN) tbl[2 * ROWV + i] = bt[i];
-            }
-            __syncthreads();
-            if (!live) return;
+        __syncthreads();
+        if (!live) return;
 #pragma unroll
-            for (int j = 0; j < VPL; ++j) gv[j] = tbl[j * 64 + lane];
-        }
-        uint4 *hid = reinterpret_cast<uint4 *>(a.hidden) + row_vec;
+        for (int j = 0; j < VPL; ++j) gv[j] = tbl[j * 64 + lane];
+    }
+    uint4 *hid = reinterpret_cast<uint4 *>(a.hidden) + row_vec;
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) {
-            float r[N], b[N], g[N], o[N];
-            unpack_vec<DT>(rv[j], r);
-            unpack_vec<DT>(bv[j], b);
-            unpack_vec<DT>(gv[j], g);
+    for (int j = 0; j < VPL; ++j) {
+        float r[N], b[N], g[N], o[N];
+        unpack_vec<DT>(rv[j], r);
+        unpack_vec<DT>(bv[j], b);
+        unpack_vec<DT>(gv[j], g);
 #pragma unroll
-            for (int i = 0; i < N; ++i) o[i] = r[i] + g[i] * b[i];
-            hv[j] = pack_vec<DT>(o);
-            st_stream(hv[j], hid + j * 64 + lane);
-        }
-    } else {
-        const uint4 *x = reinterpret_cast<const uint4 *>(a.x) + row_vec;
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) hv[j] = ld_stream(x + j * 64 + lane);
+        for (int i = 0; i < N; ++i) o[i] = r[i] + g[i] * b[i];
+        hv[j] = pack_vec<DT>(o);
+        st_stream(hv[j], hid + j * 64 + lane);
     }
 
     float mean = 0.0f, inv;
-    if constexpr (OP == OP_RMS || OP == OP_ADAPTIVE) {
+    if constexpr (OP == OP_RMS) {
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPL; ++j) {
@@ -200,14 +196,9 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
     if constexpr (SHARE) {
         gp = tbl + ROWV;
         if constexpr (OP == OP_LN) bp = tbl + 2 * ROWV;
-    } else if constexpr (OP == OP_RMS || OP == OP_LN) {
+    } else {
         gp = reinterpret_cast<const uint4 *>(a.scale);
         if constexpr (OP == OP_LN) bp = reinterpret_cast<const uint4 *>(a.bias);
-    } else {
-        const uint4 *m = reinterpret_cast<const uint4 *>(a.mod) +
-                         (size_t)(batch * a.mod_cols + a.mod_off) / N;
-        if constexpr (OP == OP_ADAPTIVE) { gp = m; bp = m + H / N; }      // scale, shift
-        else { bp = m; gp = m + H / N; }                                  // shift, scale
     }
     uint4 *out = reinterpret_cast<uint4 *>(a.out) + row_vec;
 #pragma unroll
@@ -381,6 +372,176 @@ __global__ __launch_bounds__(1024) void norm_row_kernel(NormArgs a) {
     }
 }
 
+// ----------------------------------------------------------- any-row path --
+// A block per row for rows that the two kernels above cannot hold in whole vectors of
+// their fixed counts (3072, 5120, .., odd lengths, buffers at any element) and for few
+// rows, whose time is the chain of one row: thread t owns the vectors j T + t (j < V), the
+// last one cut by the row's end.  Every tensor is read once and written once with 16-byte
+// accesses (at any element when !AL: gfx950's global accesses need no alignment; the row's
+// last H % N elements go one by one), and the per-column rows (gamma, beta, modulation)
+// are loaded beside the input, not after the reduction.
+typedef unsigned int nm_u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+
+template <int DT, bool AL>
+__device__ __forceinline__ uint4 line_load(const void *base, int64_t e, int n, bool stream) {
+    using T = typename Elem<DT>::T;
+    constexpr int N = Vec<DT>::N;
+    const T *p = reinterpret_cast<const T *>(base) + e;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (n == N) {
+        if constexpr (AL) {
+            v = stream ? ld_stream(reinterpret_cast<const uint4 *>(p)) : *reinterpret_cast<const uint4 *>(p);
+        } else {
+            const nm_u32x4 *q = reinterpret_cast<const nm_u32x4 *>(p);
+            const nm_u32x4 u = stream ? __builtin_nontemporal_load(q) : *q;
+            v = make_uint4(u.x, u.y, u.z, u.w);
+        }
+    } else if (!AL && n > 0) {
+        uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < N - 1; ++i)
+            if (i < n) {
+                if constexpr (sizeof(T) == 4) w[i] = __float_as_uint(p[i]);
+                else w[i >> 1] |= (uint32_t)p[i] << (16 * (i & 1));
+            }
+        v = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    return v;
+}
+template <int DT, bool AL>
+__device__ __forceinline__ void line_store(uint4 v, void *base, int64_t e, int n) {
+    using T = typename Elem<DT>::T;
+    constexpr int N = Vec<DT>::N;
+    T *p = reinterpret_cast<T *>(base) + e;
+    if (n == N) {
+        if constexpr (AL) st_stream(v, reinterpret_cast<uint4 *>(p));
+        else {
+            const nm_u32x4 u = {v.x, v.y, v.z, v.w};
+            __builtin_nontemporal_store(u, reinterpret_cast<nm_u32x4 *>(p));
+        }
+    } else if (!AL && n > 0) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < N - 1; ++i)
+            if (i < n) {
+                if constexpr (sizeof(T) == 4) p[i] = __uint_as_float(w[i]);
+                else p[i] = (T)(w[i >> 1] >> (16 * (i & 1)));
+            }
+    }
+}
+
+template <int DT, int OP, bool GR, int V, bool AL>
+__global__ __launch_bounds__(1024) void norm_line_kernel(NormArgs a) {
+#pragma clang fp contract(off)
+    constexpr int N = Vec<DT>::N;
+    constexpr bool BIAS = OP != OP_RMS;   // a second per-column row
+    __shared__ float red[2][16];
+    const int T = blockDim.x, t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = T >> 6;
+    const int64_t H = a.H, off = (int64_t)blockIdx.x * H;
+    // (rows fit 31 bits, and rows_per_batch divides them)
+    const int64_t batch = (GR || OP == OP_ADAPTIVE || OP == OP_MODULATED) ? blockIdx.x / (uint32_t)a.rows_per_batch : 0;
+    int64_t e[V];   // first element of each vector, and how many of the row it holds
+    int n[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        e[j] = (int64_t)(j * T + t) * N;
+        n[j] = (int)min((int64_t)N, max((int64_t)0, H - e[j]));
+    }
+    auto total = [&](float v, int slot) __attribute__((always_inline)) -> float {
+        v = wave_sum(v);
+        if (nw == 1) return v;
+        if (lane == 0) red[slot][wave] = v;
+        __syncthreads();
+        float s = 0.0f;
+        for (int w = 0; w < nw; ++w) s += red[slot][w];
+        return s;
+    };
+    using E = typename Elem<DT>::T;
+    const E *gp, *bp = nullptr;
+    if constexpr (OP == OP_RMS || OP == OP_LN) {
+        gp = reinterpret_cast<const E *>(a.scale);
+        if constexpr (OP == OP_LN) bp = reinterpret_cast<const E *>(a.bias);
+    } else {
+        const E *m = reinterpret_cast<const E *>(a.mod) + batch * a.mod_cols + a.mod_off;
+        gp = OP == OP_ADAPTIVE ? m : m + H;   // adaptive: scale, shift; modulated: shift, scale
+        bp = OP == OP_ADAPTIVE ? m + H : m;
+    }
+    uint4 hv[V], gv[V], bv[V];
+    auto tables = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            gv[j] = line_load<DT, AL>(gp, e[j], n[j], false);
+            if constexpr (BIAS) bv[j] = line_load<DT, AL>(bp, e[j], n[j], false);
+        }
+    };
+    if constexpr (GR) {
+        uint4 br[V], gt[V];
+        const E *gate = reinterpret_cast<const E *>(a.mod) + batch * a.mod_cols + a.gate_off;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            hv[j] = line_load<DT, AL>(a.x, off + e[j], n[j], true);
+            br[j] = line_load<DT, AL>(a.branch, off + e[j], n[j], true);
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) gt[j] = line_load<DT, AL>(gate, e[j], n[j], false);
+        tables();
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            float x[N], b[N], g[N], o[N];
+            unpack_vec<DT>(hv[j], x);
+            unpack_vec<DT>(br[j], b);
+            unpack_vec<DT>(gt[j], g);
+#pragma unroll
+            for (int i = 0; i < N; ++i) o[i] = i < n[j] ? x[i] + g[i] * b[i] : 0.0f;
+            hv[j] = pack_vec<DT>(o);
+            line_store<DT, AL>(hv[j], a.hidden, off + e[j], n[j]);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < V; ++j) hv[j] = line_load<DT, AL>(a.x, off + e[j], n[j], true);
+        tables();
+    }
+    float mean = 0.0f, inv, s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        float h[N];
+        unpack_vec<DT>(hv[j], h);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {   // (zeros past the row)
+            if constexpr (OP == OP_RMS || OP == OP_ADAPTIVE) s += h[i] * h[i];
+            else s += h[i];
+        }
+    }
+    s = total(s, 0);
+    if constexpr (OP == OP_RMS || OP == OP_ADAPTIVE) {
+        inv = rms_inverse<DT, OP>(s, H, a.eps);
+    } else {
+        mean = ln_mean<DT, OP>(s, H);
+        float sq = 0.0f;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            float h[N];
+            unpack_vec<DT>(hv[j], h);
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float d = i < n[j] ? h[i] - mean : 0.0f;
+                sq += d * d;
+            }
+        }
+        inv = ln_inverse<DT, OP>(total(sq, 1), H, a.eps);
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        float h[N], g[N], b[N], o[N];
+        unpack_vec<DT>(hv[j], h);
+        unpack_vec<DT>(gv[j], g);
+        if constexpr (BIAS) unpack_vec<DT>(bv[j], b);
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = apply_one<DT, OP>(h[i], mean, inv, g[i], BIAS ? b[i] : 0.0f);
+        line_store<DT, AL>(pack_vec<DT>(o), a.out, off + e[j], n[j]);
+    }
+}
+
 // ---------------------------------------------------------- generic path --
 __device__ __forceinline__ float block_sum(float v, float *smem) {
     v = wave_sum(v);
@@ -476,6 +637,38 @@ __global__ __launch_bounds__(256) void gated_residual_vec_kernel(NormArgs a) {
 }
 
 // --------------------------------------------------------------- launch --
+// The any-row kernel; false when the row is longer than a block holds.
+template <int DT, int OP, bool GR>
+static bool launch_line(const NormArgs &a, hipStream_t s, bool vec_ok) {
+    constexpr int N = Vec<DT>::N;
+    const int64_t U = (a.H + N - 1) / N;
+    // vectors per thread: one for few rows (a row's chain of latencies is the time: 1 x 4096
+    // bf16 RMSNorm 2.71 us, 2.76 with two, 2.96 with four); else two, or four where that
+    // leaves no more lanes of the block idle or two would take over 512 threads (LayerNorm
+    // 4608 x 3072, 384 vectors: 13.9 with two, 14.5 with four; 16384 x 1536, 192: 22.6 and
+    // 20.3; 4608 x 5120, 640: 23.3 and 22.0; eight spill)
+    auto threads = [&](int64_t v) { return ((U + v - 1) / v + 63) / 64 * 64; };
+    int64_t V = 2;
+    if (a.rows < 512 && U <= 512) V = 1;
+    else if (a.rows >= 512 && (U > 512 || threads(4) * 4 <= threads(2) * 2)) V = 4;
+    else if (U > 2048) V = 4;
+    if (threads(V) > 1024) return false;
+    const unsigned T = (unsigned)threads(V), blocks = (unsigned)a.rows;
+    const bool al = vec_ok && a.H % N == 0;
+#define PUTER_LINE(VV)                                                          \
+    case VV:                                                                    \
+        if (al) norm_line_kernel<DT, OP, GR, VV, true><<<blocks, T, 0, s>>>(a); \
+        else norm_line_kernel<DT, OP, GR, VV, false><<<blocks, T, 0, s>>>(a);   \
+        break;
+    switch (V) {
+        PUTER_LINE(1)
+        PUTER_LINE(2)
+        PUTER_LINE(4)
+    }
+#undef PUTER_LINE
+    return true;
+}
+
 template <int DT, int OP, bool GR>
 static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
     constexpr int N = Vec<DT>::N;
@@ -489,7 +682,13 @@ static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
     // rows against V = 1), V = 8 for the two-reduction LayerNorm, whose barriers
     // cost less over fewer waves (4096 columns, 64 threads: 4667 -> 5638 / 5014 ->
     // 5999; 8192, 128 threads: 5352 -> 5659 / 5641 -> 5799 against 512 threads).
-    // Fewer rows (latency-bound) and shorter rows keep the wave per row.
+    // The fused norms of 512 rows and more keep the wave per row on shorter rows
+    // (1024 x 2048 RMSNorm 5.1 us against 5.3 on the any-row kernel, 1024 x 8192 12.6
+    // against 13.3).  All others, few rows and every other length and alignment,
+    // take the any-row kernel (1 x 4096 RMSNorm 3.8 -> 2.7 us, 256 x 4096 4.9 -> 3.7,
+    // 1024 x 8192 LayerNorm 11.0 -> 8.8, all against the wave per row; ModulatedLayerNorm
+    // 4608 x 3072 44.2 -> 14.1, GatedResidual+RMSNorm 16384 x 2560 152 -> 58, RMSNorm 2540 x
+    // 6361 42.5 -> 19.7 against the generic kernel's three passes of single elements).
     const int64_t U = a.H / N;
     constexpr bool two_pass = OP == OP_LN || OP == OP_MODULATED;
     if (vec_ok && a.H % (64 * N) == 0 && a.rows >= 4096 && U >= 512) {
@@ -508,29 +707,27 @@ static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
             return check_launch("norm");
         }
     }
-    if (vec_ok && a.H % (64 * N) == 0) {
-        const int64_t vpl = a.H / (64 * N);
-        const unsigned blocks = (unsigned)((a.rows + 3) / 4);
-        if constexpr (GR && (OP == OP_RMS || OP == OP_LN)) {
-            if (a.rows_per_batch % 4 == 0) {   // a block's 4 rows share one gate row
-                const size_t lds = (size_t)a.H * sizeof(typename Elem<DT>::T) * (OP == OP_LN ? 3 : 2);
-                switch (vpl) {
-                case 2: norm_wave_kernel<DT, OP, GR, 2, true><<<blocks, 256, lds, s>>>(a); return check_launch("norm");
-                case 4: norm_wave_kernel<DT, OP, GR, 4, true><<<blocks, 256, lds, s>>>(a); return check_launch("norm");
-                case 8: norm_wave_kernel<DT, OP, GR, 8, true><<<blocks, 256, lds, s>>>(a); return check_launch("norm");
-                case 16: norm_wave_kernel<DT, OP, GR, 16, true><<<blocks, 256, lds, s>>>(a); return check_launch("norm");
-                default: break;
-                }
+    if constexpr (GR) {
+        if (vec_ok && a.H % (64 * N) == 0 && a.rows >= 512) {
+            const bool share = a.rows_per_batch % 4 == 0;   // a block's 4 rows share one gate row
+            const unsigned blocks = (unsigned)((a.rows + 3) / 4);
+            const size_t lds = share ? (size_t)a.H * sizeof(typename Elem<DT>::T) * (OP == OP_LN ? 3 : 2) : 0;
+#define PUTER_WAVE(VPL)                                                                           \
+    case VPL:                                                                                     \
+        if (share) norm_wave_kernel<DT, OP, VPL, true><<<blocks, 256, lds, s>>>(a);               \
+        else norm_wave_kernel<DT, OP, VPL, false><<<blocks, 256, lds, s>>>(a);                    \
+        return check_launch("norm");
+            switch (a.H / (64 * N)) {
+                PUTER_WAVE(2)
+                PUTER_WAVE(4)
+                PUTER_WAVE(8)
+                PUTER_WAVE(16)
+            default: break;
             }
-        }
-        switch (vpl) {
-        case 2: norm_wave_kernel<DT, OP, GR, 2><<<blocks, 256, 0, s>>>(a); return check_launch("norm");
-        case 4: norm_wave_kernel<DT, OP, GR, 4><<<blocks, 256, 0, s>>>(a); return check_launch("norm");
-        case 8: norm_wave_kernel<DT, OP, GR, 8><<<blocks, 256, 0, s>>>(a); return check_launch("norm");
-        case 16: norm_wave_kernel<DT, OP, GR, 16><<<blocks, 256, 0, s>>>(a); return check_launch("norm");
-        default: break;
+#undef PUTER_WAVE
         }
     }
+    if (launch_line<DT, OP, GR>(a, s, vec_ok)) return check_launch("norm");
     norm_block_kernel<DT, OP, GR><<<(unsigned)a.rows, 256, 0, s>>>(a, 1);
     return check_launch("norm(generic)");
 }

@@ -215,3 +215,58 @@ def test_norms_block_per_row(backend, dt, h):
             assert_close(got_h, hid_ref, TOL[dt], REDUCE_ELEM_TOL[dt], what="hidden")
         assert_close(decode(to_host(out, NP[dt]), dt), decode(y_ref, dt), TOL[dt], REDUCE_ELEM_TOL[dt],
                      what=f"fused {kind}")
+
+
+@pytest.mark.parametrize("dt", [O.F32, O.BF16, O.F16])
+@pytest.mark.parametrize("rows,h,rpb,shift", [
+    (1, 1, 1, 0), (3, 5, 1, 1), (2, 63, 2, 0), (4, 513, 2, 0), (511, 1016, 511, 0),
+    (512, 1025, 256, 3), (6, 3072, 3, 0), (600, 3080, 300, 0),   # one, two and four vectors a thread
+    (514, 8200, 257, 0), (2, 16385, 1, 0), (2, 34000, 2, 0),     # two blocks' worth of vectors; too long: generic
+])
+def test_norms_any_row(backend, dt, rows, h, rpb, shift):
+    """The any-row kernel against the oracle: row lengths that leave the last vector, wave
+    or block partly filled, few rows and many (512 changes the vectors per thread), buffers
+    `shift` elements past a 16-byte boundary.  Guard elements before and after each output
+    stay; the gated residual runs in place (hidden == residual)."""
+    import torch
+    import puter_amd
+    npd, eps = NP[dt], 1e-5
+    x = encode(seeded(8000 + rows + h, (rows, h)), dt)
+    br = encode(seeded(8100 + h, (rows, h)), dt)
+    mod = encode(seeded(8200 + h, (rows // rpb, 6 * h), 0.0, 0.5), dt)
+    g = encode(seeded(8300 + h, (h,), 1.0, 0.02), dt)
+    b = encode(seeded(8400 + h, (h,), 0.0, 0.02), dt)
+    guard = 8
+
+    def place(a=None):
+        buf = torch.full((shift + rows * h + guard,), 7, device="cuda",
+                         dtype=torch.float32 if dt == O.F32 else torch.int16)
+        if a is not None:
+            buf[shift:shift + a.size] = to_dev(a).view(-1)
+        return buf
+
+    def check(buf, ref, what):
+        got = to_host(buf, npd)
+        assert (got[:shift] == 7).all() and (got[shift + rows * h:] == 7).all(), what
+        assert_close(decode(got[shift:shift + rows * h].reshape(rows, h), dt), decode(ref, dt), TOL[dt],
+                     REDUCE_ELEM_TOL[dt], what=what)
+    dx, dm, dg, db = (place(a)[shift:] if a is not mod else to_dev(mod) for a in (x, mod, g, b))
+    cfg = puter_amd.RMSNormConfig(eps)
+    out = place()
+    backend.RMSNorm(cfg, dx, dg, out[shift:], rows, h, dt)
+    check(out, O.rmsnorm(x, g, eps, dt), "rms")
+    backend.LayerNorm(dx, dg, db, out[shift:], rows, h, dt)
+    check(out, O.layernorm(x, g, b, dt), "ln")
+    backend.AdaptiveRMSNorm(cfg, dx, dm, out[shift:], rows, h, rpb, 6 * h, dt)
+    check(out, O.adaptive_rmsnorm(x, mod, rpb, eps, dt), "adaptive")
+    backend.ModulatedLayerNorm(puter_amd.ModulatedLayerNormConfig(eps, 1), dx, dm, out[shift:], rows, h, rpb, 6 * h, dt)
+    check(out, O.modulated_layernorm(x, mod, rpb, eps, 1, dt), "modulated")
+    hid_ref = O.gated_residual(x, br, mod, rpb, 0, dt)
+    for kind in ("rms", "ln"):
+        hid, dbr = place(x), place(br)[shift:]
+        if kind == "rms":
+            backend.GatedResidualRMSNorm(cfg, hid[shift:], dbr, dm, dg, hid[shift:], out[shift:], rows, h, rpb, 6 * h, 0, dt)
+        else:
+            backend.GatedResidualLayerNorm(hid[shift:], dbr, dm, dg, db, hid[shift:], out[shift:], rows, h, rpb, 6 * h, 0, dt)
+        check(hid, hid_ref, "hidden " + kind)
+        check(out, O.rmsnorm(hid_ref, g, eps, dt) if kind == "rms" else O.layernorm(hid_ref, g, b, dt), "fused " + kind)
