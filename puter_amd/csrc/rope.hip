@@ -10,6 +10,7 @@
 // element is read and written once (4 B/elem in bf16); the float64 work is
 // D/2 sincos per position, not per element.  input may alias output.
 #include "common.hpp"
+#include <algorithm>
 
 namespace puter {
 
@@ -22,6 +23,10 @@ struct RopeArgs {
     int64_t orig_ctx;
     int mode, scaling;
     int ppb;  // positions per block
+    // MultiAxisRoPE: seq counts the rows of all batches; a row's token is its index modulo
+    // tokens, the first text_len tokens are text, the rest a side-wide image
+    int tokens, text_len, side, axis_count;
+    int starts[5];   // first pair of each axis, then the pair count
 };
 
 __device__ __forceinline__ double rope_inv_freq(const RopeArgs &a, int64_t pair) {
@@ -37,6 +42,27 @@ __device__ __forceinline__ double rope_inv_freq(const RopeArgs &a, int64_t pair)
     if (wavelength < highW) return inv;
     const double smooth = ((double)a.orig_ctx / wavelength - a.low) / (a.high - a.low);
     return (1.0 - smooth) * (inv / a.factor) + smooth * inv;
+}
+
+// MultiAxisRoPE, compute.go:195-330: a pair belongs to one axis; text tokens stand at their
+// index on the text axis (the last of four, the first of fewer), image tokens at their row
+// on axis 1 and column on axis 2, and at 0 on every other axis.
+__device__ __forceinline__ int rope_axis(const RopeArgs &a, int pair) {
+    int axis = 0;
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+        if (k < a.axis_count && pair >= a.starts[k]) axis = k;
+    return axis;
+}
+__device__ __forceinline__ double rope_axis_inv_freq(const RopeArgs &a, int pair) {
+    const int axis = rope_axis(a, pair);
+    const double axis_dim = 2.0 * (double)(a.starts[axis + 1] - a.starts[axis]);
+    return pow(a.base, -2.0 * (double)(pair - a.starts[axis]) / axis_dim);
+}
+__device__ __forceinline__ int rope_axis_position(const RopeArgs &a, int axis, int token) {
+    if (token < a.text_len) return axis == (a.axis_count == 4 ? 3 : 0) ? token : 0;
+    const int img = token - a.text_len;
+    return axis == 1 ? img / a.side : axis == 2 ? img % a.side : 0;
 }
 
 constexpr int kRopeLds = 8192;  // max (cos, sin) entries per block (64 KiB of LDS)
@@ -56,7 +82,10 @@ constexpr int kRopeMaxBlocks = 2048; // 8 blocks per CU on MI355X's 256 CUs
 // waits for LDS only; with no branch around any load or store the compiler
 // waits for exactly the current group's loads instead of draining every
 // outstanding access (which would also wait for the stores just issued).
-template <int DT, int MODE, bool FAST>
+// AXES: MultiAxisRoPE (interleaved pairs), whose tables differ only in the positions and
+// the axes' own frequencies.  Against a thread per pair (a float64 pow and sincos for
+// every head, 4-byte accesses) 4608 tokens x 24 heads x 128 bf16 107 -> 14 us.
+template <int DT, int MODE, bool FAST, bool AXES = false>
 __global__ __launch_bounds__(256) void rope_reg_kernel(RopeArgs a) {
 #pragma clang fp contract(off)
     extern __shared__ float2 cs[];  // [2][ppb * half] tables, then half doubles
@@ -126,7 +155,10 @@ __global__ __launch_bounds__(256) void rope_reg_kernel(RopeArgs a) {
         const int n = (int)min((int64_t)ppb, a.seq - p0) * half;
         for (int e = tid; e < n; e += 256) {
             const int p = e / half, pair = e - p * half;
-            const double theta = (double)(p0 + p + a.start) * invf[pair];
+            double theta;
+            if constexpr (AXES)
+                theta = (double)rope_axis_position(a, rope_axis(a, pair), (int)((uint32_t)(p0 + p) % (uint32_t)a.tokens)) * invf[pair];
+            else theta = (double)(p0 + p + a.start) * invf[pair];
             double sn, cn;
             sincos(theta, &sn, &cn);
             t[e] = make_float2((float)cn, (float)sn);
@@ -173,7 +205,7 @@ __global__ __launch_bounds__(256) void rope_reg_kernel(RopeArgs a) {
     if (g >= ngroups) return;  // block-uniform: the whole block leaves together
     uint4 lo[ITEMS], hi[ITEMS];
     load(g, lo, hi);
-    for (int pair = tid; pair < half; pair += 256) invf[pair] = rope_inv_freq(a, pair);
+    for (int pair = tid; pair < half; pair += 256) invf[pair] = AXES ? rope_axis_inv_freq(a, pair) : rope_inv_freq(a, pair);
     __syncthreads();
     table(g, cs);
     __syncthreads();
@@ -303,7 +335,8 @@ __global__ __launch_bounds__(256) void rope_scalar_kernel(RopeArgs a) {
     }
 }
 
-// MultiAxisRoPE compute.go:195-330: one thread per pair, angle in float64.
+// MultiAxisRoPE compute.go:195-330 for the shapes and alignments that rope_reg_kernel does
+// not take: one thread per pair, angle in float64.
 struct MultiAxisArgs {
     const void *in;
     void *out;
@@ -403,8 +436,10 @@ __global__ __launch_bounds__(256) void rope_pairs_kernel(float *__restrict__ out
     }
 }
 
-template <int DT>
-static int launch_rope(RopeArgs a, hipStream_t s) {
+// The register-resident kernel; false when a position does not fit a block's registers or
+// the vectors the buffers.
+template <int DT, bool AXES>
+static bool launch_rope_reg(RopeArgs a, hipStream_t s) {
     constexpr int N = Vec<DT>::N;
     const int64_t half = a.dim / 2;
     const int64_t slab = a.heads * a.dim;
@@ -422,15 +457,26 @@ static int launch_rope(RopeArgs a, hipStream_t s) {
         const size_t lds = 2 * (size_t)(ppb * half) * sizeof(float2) + (size_t)half * sizeof(double);
         constexpr int items = 256 * kRopeVpt;  // vectors a group can hold
         const bool fast = a.seq % ppb == 0 && ppb * slab_vec == items;
-        if (a.mode == 0) {
-            if (fast) rope_reg_kernel<DT, 0, true><<<blocks, 256, lds, s>>>(a);
-            else rope_reg_kernel<DT, 0, false><<<blocks, 256, lds, s>>>(a);
+        if (AXES || a.mode == 0) {
+            if (fast) rope_reg_kernel<DT, 0, true, AXES><<<blocks, 256, lds, s>>>(a);
+            else rope_reg_kernel<DT, 0, false, AXES><<<blocks, 256, lds, s>>>(a);
         } else {
             if (fast) rope_reg_kernel<DT, 1, true><<<blocks, 256, lds, s>>>(a);
             else rope_reg_kernel<DT, 1, false><<<blocks, 256, lds, s>>>(a);
         }
-        return check_launch("rope");
+        return true;
     }
+    return false;
+}
+
+template <int DT>
+static int launch_rope(RopeArgs a, hipStream_t s) {
+    constexpr int N = Vec<DT>::N;
+    if (launch_rope_reg<DT, false>(a, s)) return check_launch("rope");
+    const int64_t half = a.dim / 2;
+    const int64_t slab = a.heads * a.dim;
+    const bool vec = aligned16(a.in) && aligned16(a.out) && slab % N == 0 &&
+                     (a.mode == 0 ? (a.dim % N == 0) : (half % N == 0));
     // ~4096 elements of work per block, bounded by the LDS table
     int64_t ppb = slab >= 4096 ? 1 : 4096 / slab;
     if (ppb * half > kRopeLds) ppb = kRopeLds / half;
@@ -472,7 +518,7 @@ int puter_hip_rope(const puter_rope_config *config, const void *input, void *out
     if (!input || !output) return fail(PUTER_ERR_NIL, "rope: nil buffer");
     RopeArgs a{input, output, seq_len, num_heads, head_dim, c.start_position, c.base_freq,
                c.scaling_factor, c.low_freq_factor, c.high_freq_factor, c.original_context,
-               c.mode, c.scaling, 1};
+               c.mode, c.scaling, 1, 0, 0, 0, 0, {0, 0, 0, 0, 0}};
     hipStream_t s = as_stream(stream);
     switch (dtype) {
     case PUTER_F32: return launch_rope<PUTER_F32>(a, s);
@@ -528,10 +574,21 @@ int puter_hip_multi_axis_rope(const puter_multi_axis_rope_config *config, const 
     MultiAxisArgs a{input, output, batch, seq_len, num_heads, head_dim, c.base_freq,
                     c.latent_seq_len, c.latent_side, c.axis_count, {0, 0, 0, 0, 0}};
     for (int k = 0; k < c.axis_count; ++k) a.starts[k + 1] = a.starts[k] + c.axis_dims[k] / 2;
+    hipStream_t s = as_stream(stream);
+    // rows and positions fit 31 bits in the register-resident kernel
+    if (batch * seq_len <= 0x7FFFFFFF && c.latent_side <= 0x7FFFFFFF && head_dim / 2 <= kRopeGroupLds) {
+        RopeArgs r{input, output, batch * seq_len, num_heads, head_dim, 0, c.base_freq, 1.0, 0.0, 0.0, 0, 0, 0, 1,
+                   (int)seq_len, (int)std::max<int64_t>(seq_len - c.latent_seq_len, 0), (int)c.latent_side, c.axis_count,
+                   {0, 0, 0, 0, 0}};
+        for (int k = 0; k < c.axis_count; ++k) r.starts[k + 1] = (int)a.starts[k + 1];
+        const bool done = dtype == PUTER_F32   ? launch_rope_reg<PUTER_F32, true>(r, s)
+                          : dtype == PUTER_BF16 ? launch_rope_reg<PUTER_BF16, true>(r, s)
+                                                : launch_rope_reg<PUTER_F16, true>(r, s);
+        if (done) return check_launch("multi-axis rope");
+    }
     const int64_t pairs = batch * seq_len * num_heads * (head_dim / 2);
     int64_t blocks = (pairs + 255) / 256;
     if (blocks > 16384) blocks = 16384;
-    hipStream_t s = as_stream(stream);
     switch (dtype) {
     case PUTER_F32: multi_axis_rope_kernel<PUTER_F32><<<(unsigned)blocks, 256, 0, s>>>(a); break;
     case PUTER_BF16: multi_axis_rope_kernel<PUTER_BF16><<<(unsigned)blocks, 256, 0, s>>>(a); break;

@@ -60,6 +60,32 @@ def test_multi_axis_rope(backend, dt, b, s, h, base, latent, side, dims):
     assert_close(decode(to_host(out, NP[dt]), dt), ref, TOL[dt], what="multi-axis")
 
 
+@pytest.mark.parametrize("dt", [O.F32, O.BF16, O.F16])
+@pytest.mark.parametrize("b,s,h,latent,side,dims", [
+    (1, 1, 1, 1, 1, [8]),                       # one row
+    (3, 37, 5, 20, 7, [16, 24, 24]),            # groups of rows that cross batches; a ragged image row
+    (2, 130, 24, 128, 16, [32, 32, 32, 32]),    # two rows to a group, as a full-size image block
+    (1, 50, 8, 80, 9, [16, 56, 56]),            # more latent positions than tokens: no text
+    (2, 65, 3, 64, 8, [4, 6, 6, 4]),            # 20-element heads: 16-byte vectors do not fit f16 / bf16
+    (1, 40, 300, 36, 6, [32, 32]),              # a row past a block's registers: the per-pair kernel
+])
+def test_multi_axis_rope_groups(backend, dt, b, s, h, latent, side, dims):
+    """MultiAxisRoPE on the register-resident kernel (groups of rows over all batches) and
+    where that does not fit, against the oracle."""
+    import puter_amd
+    d = sum(dims)
+    x = encode(seeded(640 + s, (b, s, h, d)), dt)
+    full = dims + [0] * (4 - len(dims))
+    ref = decode(O.multi_axis_rope(x, 1e4, latent, side, dims, dt), dt)
+    cfg = puter_amd.MultiAxisRoPEConfig(1e4, latent, side, len(dims), *full)
+    dx = to_dev(x)
+    out = empty_dev((b, s, h, d), NP[dt])
+    backend.MultiAxisRoPE(cfg, dx, out, b, s, h, d, dt)
+    assert_close(decode(to_host(out, NP[dt]), dt), ref, TOL[dt], what="multi-axis rope")
+    backend.MultiAxisRoPE(cfg, dx, dx, b, s, h, d, dt)   # in place
+    assert np.array_equal(to_host(dx, NP[dt]).view(np.uint8), to_host(out, NP[dt]).view(np.uint8))
+
+
 GATES = ["SwiGLU", "GeGLU", "GeGLUTanh", "SiGLU", "GLU", "ReGLU", "LinGLU", "SeGLU"]
 
 
