@@ -26,7 +26,8 @@
  *     head dim 128 without ALiBi, or any row over more than 768 keys) or in F32
  *     with at least 16 query rows, a head dim that is a multiple of 4, and
  *     fewer 128-query blocks than two per CU (causal) or one per CU (not
- *     causal): one buffer per device, allocated on first use and grown on
+ *     causal): two buffers per device (the default stream's, and one for all
+ *     other streams), each allocated on first use and grown on
  *     demand (Matmul: at most 16 MiB; one-row attention: the paged decode
  *     workspace size, or batch x heads x ceil(seq_k / 256) x (head_dim + 2)
  *     floats; F32 attention: key splits x batch x seq_q x heads x (head_dim +

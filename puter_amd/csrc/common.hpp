@@ -22,7 +22,8 @@ inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s);
 int device_cus();
 
 // The library's scratch buffer on the current device (split-K partials of Matmul
-// and of one-row attention), held for one call's launches: the constructor orders
+// and of one-row attention; one buffer for the default stream, one for all others),
+// held for one call's launches: the constructor orders
 // the call's stream after the buffer's last user on another stream and grows the
 // buffer if needed; finish() records the call's completion on its stream.  The
 // device's lock is held from construction to destruction.  On a stream that is
@@ -37,6 +38,7 @@ public:
     ScratchLease &operator=(const ScratchLease &) = delete;
     int status() const { return status_; }
     void *ptr() const { return ptr_; }
+    int set() const { return set_; }  // 0: the default stream's buffer, 1: the other streams'
     int finish();  // call once, after the launches that use ptr()
 private:
     SplitScratch *sc_ = nullptr;
@@ -45,6 +47,7 @@ private:
     void *ptr_ = nullptr;
     int status_ = 0;
     bool captured_ = false;
+    int set_ = 0;
 };
 
 inline bool is_float_dtype(int dt) { return dt >= PUTER_F32 && dt <= PUTER_F8E5M2; }

@@ -773,9 +773,10 @@ typedef float rw_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRwCols = 128, kRwDepth = 32, kRwWaves = 4, kRwRows = 16, kRwPad = kRwCols + 4;
 constexpr int kRwMaxTiles = 16384;   // column tiles of a split launch, at most
 // per device: the column tiles' arrival counters, zero between launches (the last block's
-// atomicInc wraps to zero): one set beside the growable scratch, one beside the no-alloc
-// entry point's array, each used by one launch at a time like the scratch it stands by
-static __device__ unsigned rw_arrived[2][kRwMaxTiles];
+// atomicInc wraps to zero): a set beside each of the two growable scratch buffers and one
+// beside the no-alloc entry point's array, each used by one launch at a time like the
+// scratch it stands by
+static __device__ unsigned rw_arrived[3][kRwMaxTiles];
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) {   // 16 bytes at any element
     uint4 v;
@@ -1116,18 +1117,22 @@ __global__ __launch_bounds__(256) void matmul_splitk_reduce_kernel(uint16_t *c, 
     }
 }
 
-// Split-K partials: one scratch buffer per device, kept for the life of the
-// process and grown on demand.  A call on another stream than the buffer's last
-// user first waits (on the device, hipStreamWaitEvent) for that user's
-// completion event, so calls on different streams never overlap on the buffer.
-// Nothing waits on the host: a growth frees the old buffer and allocates the new
+// Split-K partials: two scratch buffers per device, kept for the life of the process
+// and grown on demand: one for the default (null) stream, whose own order keeps its
+// calls apart, and one for all other streams.  On the latter a call on another stream
+// than the buffer's last user first waits (on the device, hipStreamWaitEvent) for that
+// user's completion event, so calls on different streams never overlap on the buffer.
+// (The event's record costs 3.2 us of device time a call: seven split Matmuls of a
+// decoder layer at batch 1, on one buffer with events for every stream, 152.8 us; without
+// them 130.)  Nothing waits on the host: a growth frees the old buffer and allocates the new
 // one in stream order on the calling stream (hipFreeAsync / hipMallocAsync),
 // after the last user's work.  The mutex is held from acquisition until the
 // call's launches and event are enqueued.
 //
 // Under stream capture (a HIP graph being recorded) a call allocates, frees,
-// waits on and records nothing: it uses the buffer it finds when that is large
-// enough and otherwise fails with PUTER_ERR_INVALID before any launch.  The
+// waits on and records nothing: it uses whichever buffer it finds large enough (the
+// capturing stream's or the default stream's, where the call before the capture may have
+// sized it) and otherwise fails with PUTER_ERR_INVALID before any launch.  The
 // graph keeps the buffer's address, so a buffer a capture has used is never
 // freed: a later growth retires it (kept until the process ends) and allocates
 // the new one beside it.  Replays of such a graph share the buffer with eager
@@ -1143,7 +1148,7 @@ struct SplitScratch {
     bool pinned = false;        // a captured graph holds ptr
     std::vector<void *> retired;  // pinned buffers replaced by a growth
 };
-static SplitScratch g_split_scratch[64];
+static SplitScratch g_split_scratch[64][2];   // [device][0: the default stream, 1: all others]
 
 // Whether s is recording a graph (an invalidated capture counts: it must not
 // allocate either).
@@ -1156,7 +1161,7 @@ static int stream_capturing(hipStream_t s, bool *capturing) {
 }
 
 static int scratch_acquire(SplitScratch &sc, size_t need, hipStream_t s) {
-    if (!sc.done && hipEventCreateWithFlags(&sc.done, hipEventDisableTiming) != hipSuccess)
+    if (s && !sc.done && hipEventCreateWithFlags(&sc.done, hipEventDisableTiming) != hipSuccess)
         return fail(PUTER_ERR_UNAVAILABLE, "matmul: cannot create the split-K event");
     if (sc.used && sc.last != s && hipStreamWaitEvent(s, sc.done, 0) != hipSuccess)
         return fail(PUTER_ERR_LAUNCH, "matmul: cannot order the split-K scratch");
@@ -1190,10 +1195,13 @@ static bool scratch_capturing(hipStream_t s, size_t *held) {
     bool capturing = true;
     *held = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return true;
-    std::lock_guard<std::mutex> g(g_split_scratch[dev].mu);
     if (stream_capturing(s, &capturing) != PUTER_OK) return true;
-    *held = g_split_scratch[dev].bytes;
-    return capturing;
+    if (!capturing) return false;
+    for (SplitScratch &sc : g_split_scratch[dev]) {
+        std::lock_guard<std::mutex> g(sc.mu);
+        *held = std::max(*held, sc.bytes);
+    }
+    return true;
 }
 
 ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
@@ -1202,11 +1210,23 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
         status_ = fail(PUTER_ERR_UNAVAILABLE, "scratch: no device");
         return;
     }
-    sc_ = &g_split_scratch[dev];
-    lock_ = std::unique_lock<std::mutex>(sc_->mu);
     bool capturing = false;
     if ((status_ = stream_capturing(s, &capturing)) != PUTER_OK) return;
+    set_ = s ? 1 : 0;
+    sc_ = &g_split_scratch[dev][set_];
+    lock_ = std::unique_lock<std::mutex>(sc_->mu);
     if (capturing) {
+        if (sc_->bytes < bytes) {   // the other buffer, if it is large enough
+            SplitScratch &other = g_split_scratch[dev][1 - set_];
+            lock_.unlock();
+            lock_ = std::unique_lock<std::mutex>(other.mu);
+            if (other.bytes >= bytes) {
+                sc_ = &other;
+                set_ = 1 - set_;
+            } else {
+                lock_ = std::unique_lock<std::mutex>(sc_->mu);
+            }
+        }
         if (sc_->bytes < bytes) {
             status_ = fail(PUTER_ERR_INVALID,
                            "scratch: %zu bytes needed under stream capture, %zu held; the library's scratch "
@@ -1226,7 +1246,7 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
 
 int ScratchLease::finish() {
     if (status_ != PUTER_OK) return status_;
-    if (captured_) return PUTER_OK;
+    if (captured_ || set_ == 0) return PUTER_OK;   // the default stream orders its own calls
     if (hipEventRecord(sc_->done, s_) != hipSuccess) return fail(PUTER_ERR_LAUNCH, "scratch: cannot record the event");
     sc_->last = s_;
     sc_->used = true;
@@ -1321,7 +1341,7 @@ static int launch_rows_mt(void *out, const void *left, const void *right, int64_
     const int64_t per = (steps + chunks - 1) / chunks;
     chunks = (steps + per - 1) / per;
     RwArgs p{static_cast<uint16_t *>(out), static_cast<const uint16_t *>(left), static_cast<const uint16_t *>(right), tgt.fixed,
-             (int)M, (int)tiles, (int)chunks, (int)mtiles, tgt.fixed ? 1 : 0, K, N, per * STEP};
+             (int)M, (int)tiles, (int)chunks, (int)mtiles, 2, K, N, per * STEP};
     auto launch = [&] {
         const int64_t blocks = (tiles * p.chunks + 7) / 8 * 8 * mtiles;
         matmul_rows_kernel<DT, MT><<<(unsigned)blocks, 256, 0, s>>>(p);
@@ -1336,6 +1356,7 @@ static int launch_rows_mt(void *out, const void *left, const void *right, int64_
         return launch();
     }
     p.ws = static_cast<float *>(lease.ptr());
+    p.set = lease.set();
     const int rc = launch();
     const int fin = lease.finish();
     return rc ? rc : fin;

@@ -385,6 +385,48 @@ def test_matmul_16bit_rows_kernel_exact(backend, dt, rows, inner, cols, shift):
         assert np.array_equal(got[shift:shift + rows * cols].reshape(rows, cols), want), (dt, rows, inner, cols, rep)
 
 
+def test_matmul_default_and_side_streams_keep_apart(backend):
+    """Split-K calls on the default stream and on two side streams, interleaved without
+    synchronisation: the default stream's partials are in a buffer of its own (no events
+    order it with the others), so every result must match the same call made alone; then
+    the default stream's calls size the scratch that a capture on another stream uses."""
+    import torch
+    shapes = [(1, 4096, 1024), (64, 4096, 1024), (16, 4096, 512), (128, 8192, 2048)]
+    ins, alone = [], []
+    for i, (m, k, n) in enumerate(shapes):
+        rng = np.random.default_rng(970 + i)
+        a = to_dev(O.from_f32(rng.integers(-2, 3, (m, k)).astype(np.float32), O.BF16))
+        b = to_dev(O.from_f32(rng.integers(-2, 3, (k, n)).astype(np.float32), O.BF16))
+        out = empty_dev((m, n), np.uint16)
+        backend.Matmul(out, a, b, m, k, n, O.BF16)
+        ins.append((a, b))
+        alone.append(to_host(out, np.uint16))
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for rep in range(4):
+        outs = [[empty_dev((m, n), np.uint16) for m, k, n in shapes] for _ in streams]
+        torch.cuda.synchronize()
+        for i, (m, k, n) in enumerate(shapes):
+            for j, st in enumerate(streams):
+                with torch.cuda.stream(st):
+                    backend.Matmul(outs[j][i], *ins[i], m, k, n, O.BF16)
+        torch.cuda.synchronize()
+        for row in outs:
+            for got, want in zip(row, alone):
+                assert np.array_equal(to_host(got, np.uint16), want), rep
+    (a, b), (m, k, n) = ins[3], shapes[3]
+    out = empty_dev((m, n), np.uint16)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        backend.Matmul(out, a, b, m, k, n, O.BF16)
+    for rep in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(to_host(out, np.uint16), alone[3]), rep
+        (torch.randn(1 << 20, device="cuda") * 2).sum().item()
+
+
 def test_matmul_unaligned_captured_without_scratch(backend):
     """A shape that only the rows kernel takes was never refused under stream capture (the
     generic kernel needs no scratch): captured, it splits K only as far as the scratch held
