@@ -31,7 +31,8 @@
  *     demand (Matmul: at most 16 MiB; one-row attention: the paged decode
  *     workspace size, or batch x heads x ceil(seq_k / 256) x (head_dim + 2)
  *     floats; F32 attention: key splits x batch x seq_q x heads x (head_dim +
- *     2) floats, at most about 100 MB).  A growth is stream-ordered on the calling
+ *     2) floats, at most about 100 MB; scaled-dot-product attention: see there).
+ *     A growth is stream-ordered on the calling
  *     stream (hipFreeAsync of the old buffer after its last user, then
  *     hipMallocAsync): it never blocks the host.  On a stream that is capturing
  *     a HIP graph these calls allocate, free, wait on and record nothing: they
@@ -320,7 +321,10 @@ typedef struct puter_flash_config {
 /* ScaledDotProductAttention(config, q, k, v, out, seqQ, seqK, depth, valueDim, format)
  * interface.go:104-109: one head, Q [seqQ, depth], K [seqK, depth], V [seqK, valueDim],
  * O [seqQ, valueDim]; online softmax through FastExp32 (cpu/attention/typed_compute.go:31-97).
- * depth <= 8192, valueDim <= 1024 (beyond: PUTER_ERR_INVALID). */
+ * depth <= 8192, valueDim <= 1024 (beyond: PUTER_ERR_INVALID).  F32 and the 16-bit
+ * head sizes past the MFMA prefill kernel's keep up to 64 MiB of scores (and f32
+ * copies of V and of the output where needed) in the library's scratch, for 64 to
+ * 16384 keys; under stream capture only if the scratch held has that room. */
 PUTER_API int puter_hip_scaled_dot_product_attention(const puter_flash_config *config,
                                            const void *query, const void *key, const void *value,
                                            void *output, int64_t seq_q, int64_t seq_k,

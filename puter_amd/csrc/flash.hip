@@ -18,6 +18,7 @@
 // on the MFMA prefill kernel with one head and shift 0 (hardware exp2 in place of
 // FastExp32; the difference is far below bf16 / f16 resolution).
 #include "attention.hpp"
+#include <algorithm>
 
 namespace puter {
 
@@ -91,6 +92,256 @@ __global__ __launch_bounds__(64) void flash_generic_kernel(FlashArgs a) {
     }
 }
 
+// ------------------------------------------------- three-pass form (MFMA) --
+// f32, and the 16-bit head sizes that the MFMA prefill kernel does not take: the scores of
+// a block of query rows in the library's scratch, the rows turned into weights, the weights
+// times V.  The general kernel above walks one row's keys one at a time (2048 x 2048 x 64
+// f32 1246 us); here the two products run on v_mfma_f32_32x32x2_f32 and a row's keys are
+// spread over a block.  The exponentials are the reference's own, each evaluated at the
+// same argument: with M_j the running maximum after key j and alpha_j = exp(M_(j-1) - M_j)
+// the reference's rescale, key j ends up with the weight
+//     exp(s_j - M_j) * product of alpha_i over i > j,
+// so a prefix maximum and a suffix product over the row give the weights in any order of
+// evaluation (only the rounding of the products and of the sum differs).  Measured, the
+// error against float64 unchanged in each: f32 2048 x 2048 x 64 1249 -> 48 us (scores 17, weights
+// 13.5, product 18.5; the three are bound by their passes over the 16 MB of scores, which
+// the L2s and the last-level cache serve, and the float32 MFMA rate), 1000 x 1000 x 512 f32
+// 2488 -> 67, bf16 2334 -> 92; 64 x 64 x 64 38 -> 19; below 64 keys the general kernel runs.
+
+// S[r, k] = Q[q0 + r] . K[k] for 32 query rows and 4 x 64 keys a block: wave w owns keys
+// 64 w .. + 63 of the block's as two 32 x 32 accumulators.  A lane's operands for four
+// MFMA steps are 4 consecutive elements of its row (half h = lane / 32 takes d = 8 g + 4 h
+// .. + 3), read straight from memory: Q and K of one head stay in the caches.  VEC: rows
+// are whole 4-element pieces at their natural alignment.
+typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
+
+template <int DT, bool VEC>
+__device__ __forceinline__ float4 flash_load4(const void *row, int64_t d, int64_t depth) {
+    using T = typename Elem<DT>::T;
+    const T *p = static_cast<const T *>(row) + d;
+    if constexpr (VEC) {
+        if (d >= depth) return make_float4(0, 0, 0, 0);
+        if constexpr (DT == PUTER_F32) return *reinterpret_cast<const float4 *>(p);
+        else {
+            const uint2 v = *reinterpret_cast<const uint2 *>(p);
+            return make_float4(Elem<DT>::load((T)v.x), Elem<DT>::load((T)(v.x >> 16)), Elem<DT>::load((T)v.y),
+                               Elem<DT>::load((T)(v.y >> 16)));
+        }
+    } else {
+        float f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = d + i < depth ? Elem<DT>::load(p[i]) : 0.0f;
+        return make_float4(f[0], f[1], f[2], f[3]);
+    }
+}
+
+template <int DT, bool VEC>
+__global__ __launch_bounds__(256) void flash_score_kernel(FlashArgs a, float *S, int64_t ld, int64_t q0, int64_t rows) {
+    using T = typename Elem<DT>::T;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, h = lane >> 5;
+    const int64_t r0 = (int64_t)blockIdx.y * 32, k0 = ((int64_t)blockIdx.x * 4 + wave) * 64;
+    // (causal: keys past the block's last row are masked in all of it)
+    if (k0 >= a.seq_k || (a.causal && k0 > q0 + std::min(r0 + 31, rows - 1))) return;
+    const int64_t depth = a.depth;
+    const T *q = static_cast<const T *>(a.q) + (q0 + std::min(r0 + l32, rows - 1)) * depth;
+    const T *k[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) k[n] = static_cast<const T *>(a.k) + std::min(k0 + 32 * n + l32, a.seq_k - 1) * depth;
+    fl_f32x16 acc[2] = {(fl_f32x16){}, (fl_f32x16){}};
+    constexpr int U = 4;   // groups of 8 d's in flight
+    for (int64_t d0 = 0; d0 < depth; d0 += 8 * U) {
+        float4 qv[U], kv[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t d = d0 + 8 * u + 4 * h;
+            qv[u] = flash_load4<DT, VEC>(q, d, depth);
+#pragma unroll
+            for (int n = 0; n < 2; ++n) kv[u][n] = flash_load4<DT, VEC>(k[n], d, depth);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+                    acc[n] = __builtin_amdgcn_mfma_f32_32x32x2f32((&qv[u].x)[i], (&kv[u][n].x)[i], acc[n], 0, 0, 0);
+    }
+    // register j of lane (l32, h): row 8 (j / 4) + 4 h + j % 4, key l32
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        const int64_t key = k0 + 32 * n + l32;
+        if (key >= a.seq_k) continue;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int64_t r = r0 + 8 * (j >> 2) + 4 * h + (j & 3);
+            if (r < rows) S[r * ld + key] = acc[n][j];
+        }
+    }
+}
+
+// Row r of S becomes its normalised weights, zeros on masked keys and on the columns
+// [seq_k, ld).  One block per row; thread t holds the E keys E t .. + E - 1 (E T >= ld).
+template <int DT, int E>
+__global__ __launch_bounds__(1024) void flash_weights_kernel(FlashArgs a, float *S, int64_t ld, int64_t q0) {
+    __shared__ float part[3][16];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
+    float *row = S + (int64_t)blockIdx.x * ld;
+    const int64_t k0 = (int64_t)t * E;
+    const int64_t k_hi = a.causal ? min(a.seq_k, q0 + (int64_t)blockIdx.x + 1) : a.seq_k;
+    float s[E];
+#pragma unroll
+    for (int j = 0; j < E; j += 4) {   // ld % 4 == 0
+        const float4 v = k0 + j < k_hi ? *reinterpret_cast<const float4 *>(row + k0 + j) : make_float4(0, 0, 0, 0);
+        s[j] = v.x; s[j + 1] = v.y; s[j + 2] = v.z; s[j + 3] = v.w;
+    }
+    // the running maximum before this thread's keys (NaN scores never raise it)
+    float top = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        s[j] = round_reduction<DT>(s[j]) * a.scale;
+        if (k0 + j < k_hi && s[j] > top) top = s[j];
+    }
+    float incl = top;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const float up = __shfl_up(incl, o, kWave);
+        if (lane >= o) incl = fmaxf(incl, up);
+    }
+    if (lane == 63) part[0][wave] = incl;
+    __syncthreads();
+    float m = __shfl_up(incl, 1, kWave);
+    if (lane == 0) m = -INFINITY;
+    for (int w = 0; w < wave; ++w) m = fmaxf(m, part[0][w]);
+    // this thread's keys in order: weight against the running maximum, then the later
+    // rescales of its own keys (alpha is 1 wherever the maximum stays)
+    float alpha[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        const bool seen = k0 + j < k_hi;
+        const float old = m;
+        if (seen && s[j] > m) m = s[j];
+        const bool rescale = seen && (old != m || m == -INFINITY);
+        alpha[j] = 1.0f;
+        if (__any(rescale)) alpha[j] = rescale ? flash_exp(old - m) : 1.0f;
+        s[j] = seen ? flash_exp(s[j] - m) : 0.0f;
+    }
+    float after = 1.0f;
+#pragma unroll
+    for (int j = E - 1; j >= 0; --j) {
+        s[j] *= after;
+        after *= alpha[j];
+    }
+    // the rescales of all later threads: a suffix product
+    float suf = after;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const float dn = __shfl_down(suf, o, kWave);
+        if (lane + o < 64) suf *= dn;
+    }
+    if (lane == 0) part[1][wave] = suf;
+    float later = __shfl_down(suf, 1, kWave);
+    if (lane == 63) later = 1.0f;
+    __syncthreads();
+    float all = 1.0f;   // the product of every rescale, which the empty sum at the start gets
+    for (int w = 0; w < nw; ++w) {
+        all *= part[1][w];
+        if (w > wave) later *= part[1][w];
+    }
+    float l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        s[j] *= later;
+        l += s[j];
+    }
+    l = wave_sum(l);
+    if (lane == 0) part[2][wave] = l;
+    __syncthreads();
+    l = 0.0f * all;
+    for (int w = 0; w < nw; ++w) l += part[2][w];
+    const float inv = l != 0.0f ? 1.0f / l : 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; j += 4)
+        if (k0 + j < ld) *reinterpret_cast<float4 *>(row + k0 + j) = make_float4(s[j] * inv, s[j + 1] * inv, s[j + 2] * inv, s[j + 3] * inv);
+}
+
+// V as f32 with zero rows up to a multiple of 4 keys.
+template <int DT>
+__global__ __launch_bounds__(256) void flash_values_kernel(float *dst, const void *v, int64_t n, int64_t padded) {
+    using T = typename Elem<DT>::T;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < padded; i += (int64_t)gridDim.x * 256)
+        dst[i] = i < n ? Elem<DT>::load(static_cast<const T *>(v)[i]) : 0.0f;
+}
+
+// Narrows the f32 product (16-bit formats; from null: o holds f32 already), and sums again,
+// key by key, every causal row with an infinity or NaN in it: a masked key's zero weight
+// times an infinite value is NaN in the product, while its row is never read here.
+template <int DT>
+__global__ __launch_bounds__(64) void flash_finish_kernel(FlashArgs a, const float *W, const float *from, int64_t ld,
+                                                          int64_t q0) {
+    using T = typename Elem<DT>::T;
+    const int64_t r = blockIdx.x, vd = a.value_dim;
+    const int lane = threadIdx.x;
+    T *O = static_cast<T *>(a.o) + (q0 + r) * vd;
+    const T *V = static_cast<const T *>(a.v);
+    for (int64_t d = lane; d < vd; d += kWave) {
+        float x = from ? from[r * vd + d] : Elem<DT>::load(O[d]);
+        if (a.causal && x * 0.0f != 0.0f) {
+            x = 0.0f;
+            const int64_t k_hi = min(a.seq_k, q0 + r + 1);
+            for (int64_t k = 0; k < k_hi; ++k) x += W[r * ld + k] * Elem<DT>::load(V[k * vd + d]);
+            O[d] = Elem<DT>::store(x);
+        } else if (from) O[d] = Elem<DT>::store(x);
+    }
+}
+
+constexpr int64_t kFlashScores = (int64_t)64 << 20;   // bytes of scores held at once
+constexpr int64_t kFlashMaxKeys = 16384;              // a row's keys in one block's registers
+
+// Returns false when the general kernel is to run: few keys, rows past a block, or a
+// stream capture whose scratch has no room.
+template <int DT>
+static bool run_flash_passes(const FlashArgs &a, hipStream_t s, int *status) {
+    if (a.seq_k < 64 || a.seq_k > kFlashMaxKeys) return false;
+    const int64_t ld = (a.seq_k + 3) / 4 * 4, vd = a.value_dim;
+    const int64_t chunk = std::min<int64_t>(a.seq_q, std::max<int64_t>(32, kFlashScores / (ld * 4) / 32 * 32));
+    const bool widen = DT != PUTER_F32 || ld != a.seq_k, narrow = DT != PUTER_F32;
+    auto up = [](int64_t floats) { return (floats + 63) / 64 * 64; };
+    const int64_t n_s = up(chunk * ld), n_v = widen ? up(ld * vd) : 0, n_o = narrow ? up(chunk * vd) : 0;
+    const size_t part = matmul_f32_scratch_bytes(chunk, ld, vd);
+    const size_t need = (size_t)(n_s + n_v + n_o) * sizeof(float) + part;
+    size_t held = 0;
+    if (scratch_capturing(s, &held) && held < need) return false;
+    ScratchLease lease(need, s);
+    if (lease.status()) return false;
+    float *S = static_cast<float *>(lease.ptr()), *vf = S + n_s, *of = vf + n_v, *mm = of + n_o;
+    if (widen) {
+        const int64_t padded = ld * vd;
+        flash_values_kernel<DT><<<(unsigned)std::min<int64_t>((padded + 255) / 256, 2048), 256, 0, s>>>(vf, a.v, a.seq_k * vd, padded);
+    }
+    const uintptr_t align = DT == PUTER_F32 ? 15 : 7;
+    const bool vec = a.depth % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k)) & align) == 0;
+    int rc = PUTER_OK;
+    for (int64_t q0 = 0; q0 < a.seq_q && rc == PUTER_OK; q0 += chunk) {
+        const int64_t rows = std::min(chunk, a.seq_q - q0);
+        const dim3 grid((unsigned)((a.seq_k + 255) / 256), (unsigned)((rows + 31) / 32));
+        if (vec) flash_score_kernel<DT, true><<<grid, 256, 0, s>>>(a, S, ld, q0, rows);
+        else flash_score_kernel<DT, false><<<grid, 256, 0, s>>>(a, S, ld, q0, rows);
+        const int E = ld <= 256 * 4 ? 4 : ld <= 1024 * 8 ? 8 : 16;
+        const unsigned T = (unsigned)((ld + E - 1) / E + 63) / 64 * 64;
+        if (E == 4) flash_weights_kernel<DT, 4><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
+        else if (E == 8) flash_weights_kernel<DT, 8><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
+        else flash_weights_kernel<DT, 16><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
+        float *o = narrow ? of : static_cast<float *>(a.o) + q0 * vd;
+        rc = matmul_f32_in_scratch(o, S, widen ? vf : static_cast<const float *>(a.v), rows, ld, vd, s, mm, part);
+        if (narrow || a.causal)
+            flash_finish_kernel<DT><<<(unsigned)rows, 64, 0, s>>>(a, S, narrow ? of : nullptr, ld, q0);
+    }
+    if (rc == PUTER_OK) rc = check_launch("flash attention");
+    const int fin = lease.finish();
+    *status = rc ? rc : fin;
+    return true;
+}
+
 static int run_flash(const puter_flash_config *config, const void *q, const void *k,
                      const void *v, void *o, int64_t seq_q, int64_t seq_k, int64_t depth,
                      int64_t value_dim, int dtype, hipStream_t s) {
@@ -115,6 +366,13 @@ static int run_flash(const puter_flash_config *config, const void *q, const void
     }
     FlashArgs a{q, k, v, o, seq_q, seq_k, depth, value_dim, config->causal ? 1 : 0, scale};
     const size_t lds = sizeof(float) * (size_t)depth;
+    {
+        int status = PUTER_OK;
+        const bool done = dtype == PUTER_F32   ? run_flash_passes<PUTER_F32>(a, s, &status)
+                          : dtype == PUTER_BF16 ? run_flash_passes<PUTER_BF16>(a, s, &status)
+                                                : run_flash_passes<PUTER_F16>(a, s, &status);
+        if (done) return status;
+    }
     switch (dtype) {
     case PUTER_F32: flash_generic_kernel<PUTER_F32><<<(unsigned)seq_q, kWave, lds, s>>>(a); break;
     case PUTER_BF16: flash_generic_kernel<PUTER_BF16><<<(unsigned)seq_q, kWave, lds, s>>>(a); break;

@@ -695,6 +695,52 @@ def test_scaled_dot_product_attention(backend, dt, sq, sk, d, vd, causal):
                      elem_tol=1e-3 if dt == O.F32 else None, what="sdpa")
 
 
+@pytest.mark.parametrize("dt", [O.F32, O.F16, O.BF16])
+@pytest.mark.parametrize("sq,sk,d,vd,causal", [
+    (64, 64, 4, 4, False),          # the fewest keys of the three-pass form
+    (33, 65, 7, 5, True),           # rows of odd elements; seqK > seqQ, one key past a multiple of 64
+    (100, 1021, 40, 24, False),     # padded key columns; 4 keys a thread
+    (700, 1027, 20, 12, True),      # 8 keys a thread, causal rows that end in every wave
+    (40, 8193, 16, 8, False),       # 16 keys a thread
+    (1100, 16384, 8, 4, True),      # the most keys; two blocks of query rows
+    (70, 300, 512, 512, True),      # a head size past the MFMA prefill kernel's
+])
+def test_scaled_dot_product_attention_passes(backend, dt, sq, sk, d, vd, causal):
+    """The three-pass form (scores, weights, product) against the oracle's key-by-key
+    recurrence: the same exponentials, so f32 stays within its bar."""
+    import puter_amd
+    std = 1.0 / np.sqrt(d) if dt != O.F32 else 0.25
+    q = encode(seeded(530 + sq, (sq, d), 0.0, 4 * std), dt)   # spread scores: several new maxima a row
+    k = encode(seeded(531 + sk, (sk, d), 0.0, std), dt)
+    v = encode(seeded(532 + sk, (sk, vd)), dt)
+    ref = decode(O.flash_attention(q, k, v, causal=causal, dtype=dt), dt)
+    out = empty_dev((sq, vd), NP[dt])
+    backend.FlashAttention(puter_amd.FlashAttentionConfig(64, causal), to_dev(q), to_dev(k), to_dev(v), out, sq, sk,
+                           d, vd, dt)
+    assert_close(decode(to_host(out, NP[dt]), dt), ref, TOL[dt], elem_tol=1e-3 if dt == O.F32 else None, what="sdpa passes")
+
+
+def test_flash_f32_values_not_finite(backend):
+    """A NaN row of V at the last key reaches the last causal row alone (the general kernel
+    never reads a masked key), an infinity at key 2 every row from 2 on; a NaN in Q its row."""
+    import puter_amd
+    s, d = 150, 32
+    q, k, v = (seeded(560 + i, (s, d), 0.0, 0.3) for i in range(3))
+    ref = O.flash_attention(q, k, v, causal=True, dtype=O.F32)
+    q2, v2 = q.copy(), v.copy()
+    q2[70, 0] = np.nan
+    v2[-1], v2[2, 7] = np.nan, np.inf
+    out = empty_dev((s, d), np.float32)
+    backend.FlashAttention(puter_amd.FlashAttentionConfig(64, True), to_dev(q2), to_dev(k), to_dev(v2), out, s, s, d, d,
+                           O.F32)
+    got = to_host(out, np.float32)
+    assert np.isnan(got[-1]).all() and np.isnan(got[70]).all()
+    rows = [r for r in range(s - 1) if r != 70]
+    assert np.isposinf(got[rows][2:, 7]).all()
+    got[2:, 7] = ref[2:, 7]
+    assert_close(got[rows], ref[rows], TOL[O.F32], elem_tol=1e-3, what="flash with NaN and inf")
+
+
 def out_dtype(kv_dt):
     """Query and output format of a paged decode: the pool's for f16 / bf16
     pools, bf16 for fp8 pools."""
