@@ -21,7 +21,7 @@
 // rows target one (page, slot) the last one wins (page_generic.go:23-27).  The
 // rows are copied in parallel here, and a row skips its store when a later row
 // targets the same slot.  Each block (1024 threads; 256 for calls of at most
-// 8192 rows) takes R consecutive rows (R a power of two, 8 to 1024, about
+// 8192 rows) takes R consecutive rows (R a power of two, 8 to 1024, 2 for calls of at most 1024 rows, about
 // value_rows / 512 so that a large call has about 512 blocks, two per CU,
 // resident at once), puts their (page id, slot) keys in an
 // LDS hash table (a key's entry keeps the highest
@@ -330,20 +330,60 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) vo
     }
 }
 
-// fp8 quantising write: R rows per block as for the plain write, each winning
-// row taken by one wave; a lane handles 16 consecutive elements at a time (one
-// 16-byte fp8 store; head = element / head_dim).
+// fp8 quantising write: R rows per block as for the plain write.  The block's rows are one
+// run of 8-element units (one 8-byte fp8 store each; pool rows are whole units); the
+// thread's first unit is loaded ahead of the table work and each next one ahead of its
+// store.  Values are read 16 bytes at a time at any element alignment, and a unit divides
+// once for its head, whose scale is loaded with the values.  A 64-row decode step of 8 x 128
+// bf16 is bound by its chain of latencies: 17 us with 2-byte loads and a 64-bit division an
+// element, 9.8 with these units, 5.6 with the scales loaded ahead and two rows to a block.
+template <int DT> struct QuantUnit {
+    static constexpr int NV = 8 / Vec<DT>::N;   // 16-byte vectors of values
+    uint4 v[NV];
+    int64_t head, left;   // the first element's head, and its elements from there on
+    float s;              // and scale
+    // the unit that starts at element e0 of the row at `row`: one division finds its head
+    __device__ __forceinline__ void load(const void *values, int64_t row, int64_t e0, const float *__restrict__ scales,
+                                         int64_t head_dim) {
+        const typename Elem<DT>::T *p = reinterpret_cast<const typename Elem<DT>::T *>(values) + row + e0;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) __builtin_memcpy(&v[k], p + k * Vec<DT>::N, 16);
+        const bool small = ((uint64_t)(e0 | head_dim) >> 32) == 0;
+        head = small ? (int64_t)((uint32_t)e0 / (uint32_t)head_dim) : e0 / head_dim;
+        left = (head + 1) * head_dim - e0;
+        s = scales[head];
+    }
+    __device__ __forceinline__ uint2 codes(const float *__restrict__ scales, int64_t head_dim) {
+        uint32_t w[2] = {0, 0};
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            float f[Vec<DT>::N];
+            unpack_vec<DT>(v[k], f);
+#pragma unroll
+            for (int i = 0; i < Vec<DT>::N; ++i) {
+                const int at = k * Vec<DT>::N + i;
+                if (left == 0) {
+                    left = head_dim;
+                    s = scales[++head];
+                }
+                --left;
+                w[at >> 2] |= f32_to_e4m3(__fdiv_rn(f[i], s)) << (8 * (at & 3));
+            }
+        }
+        return make_uint2(w[0], w[1]);
+    }
+};
+
 template <int DT, int THREADS>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) void page_write_fp8_kernel(uint8_t *__restrict__ storage,
-                                                             const void *__restrict__ values,
-                                                             const int32_t *__restrict__ ids,
-                                                             const int32_t *__restrict__ offsets,
-                                                             const float *__restrict__ scales,
-                                                             int64_t page_count, int64_t page_size,
-                                                             int64_t head_dim, int64_t inner, int64_t value_rows,
-                                                             int64_t rows_per_block, int table_bits,
-                                                             int32_t *status) {
-    using T = typename Elem<DT>::T;
+__global__ __launch_bounds__(THREADS) void page_write_fp8_kernel(uint8_t *__restrict__ storage,
+                                                                 const void *__restrict__ values,
+                                                                 const int32_t *__restrict__ ids,
+                                                                 const int32_t *__restrict__ offsets,
+                                                                 const float *__restrict__ scales,
+                                                                 int64_t page_count, int64_t page_size,
+                                                                 int64_t head_dim, int64_t inner, int64_t value_rows,
+                                                                 int64_t rows_per_block, int table_bits,
+                                                                 int32_t *status) {
     extern __shared__ __align__(16) char lds[];
     const int tid = threadIdx.x;
     const int64_t row0 = (int64_t)blockIdx.x * rows_per_block;
@@ -354,40 +394,35 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(8))) vo
         my_id = ids[row0 + tid];
         my_off = offsets[row0 + tid];
     }
+    const int64_t upr = inner / 8, units = nrows * upr, first = row0 * inner;
+    QuantUnit<DT> u;
+    auto row_of = [&](int64_t q) __attribute__((always_inline)) -> int64_t {
+        return units <= 0xFFFFFFFFll ? (int64_t)((uint32_t)q / (uint32_t)upr) : q / upr;
+    };
+    int64_t i = row_of(tid), e0 = (tid - i * upr) * 8;
+    if (tid < units) u.load(values, first + i * inner, e0, scales, head_dim);
     ScanChunk c0;
     scan_load<THREADS>(c0, ids, offsets, row0 + nrows, value_rows);
     write_winners<THREADS>(t, my_id, my_off, c0, ids, offsets, row0, nrows, value_rows, page_count, page_size, status);
-    const int lane = threadIdx.x & 63;
-    for (int i = threadIdx.x >> 6; i < nrows; i += THREADS / 64) {
-        if (!write_wins(t, i)) continue;
-        const int64_t row = row0 + i;
-        uint8_t *dst = storage + write_slot(t, i, page_size) * inner;
-        const T *src = reinterpret_cast<const T *>(values) + row * inner;
-        for (int64_t e0 = (int64_t)lane * 16; e0 < inner; e0 += 64 * 16) {
-            uint32_t w[4] = {0, 0, 0, 0};
-            const int n = (int)min((int64_t)16, inner - e0);
-#pragma unroll
-            for (int k = 0; k < 16; ++k) {
-                if (k < n) {
-                    const int64_t e = e0 + k;
-                    const float q = __fdiv_rn(Elem<DT>::load(src[e]), scales[e / head_dim]);
-                    w[k >> 2] |= f32_to_e4m3(q) << (8 * (k & 3));
-                }
-            }
-            if (n == 16) {
-                *reinterpret_cast<uint4 *>(dst + e0) = make_uint4(w[0], w[1], w[2], w[3]);
-            } else {
-                for (int k = 0; k < n; ++k) dst[e0 + k] = (uint8_t)(w[k >> 2] >> (8 * (k & 3)));
-            }
+    for (int64_t q = tid; q < units; q += THREADS) {
+        QuantUnit<DT> cur = u;
+        const int64_t ci = i, ce = e0;
+        if (q + THREADS < units) {
+            i = row_of(q + THREADS);
+            e0 = (q + THREADS - i * upr) * 8;
+            u.load(values, first + i * inner, e0, scales, head_dim);
         }
+        if (!write_wins(t, (int)ci)) continue;
+        *reinterpret_cast<uint2 *>(storage + write_slot(t, (int)ci, page_size) * inner + ce) = cur.codes(scales, head_dim);
     }
 }
 
-// Rows per write block (a power of two, 8..1024, about rows / 512; at most 16
+// Rows per write block (a power of two, 2 up to 1024 rows, else 8..1024, about rows / 512;
+// at most 16
 // for the 256-thread blocks of calls up to kSmallWriteRows rows, so R never
 // exceeds the block's threads) and log2 of its table size (2R entries).
 static int64_t write_rows_per_block(int64_t rows, int *table_bits) {
-    int64_t r = 8;
+    int64_t r = rows <= 1024 ? 2 : 8;
     while (r < kWriteMaxRows && r * 512 < rows) r <<= 1;
     int bits = 0;
     while (((int64_t)1 << bits) < 2 * r) ++bits;
