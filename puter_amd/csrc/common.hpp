@@ -53,11 +53,6 @@ private:
 // Whether s is recording a graph (or cannot be asked); if so, the bytes that the largest
 // of the device's scratch buffers holds, which is all a lease can get (matmul.hip).
 bool scratch_capturing(hipStream_t s, size_t *held);
-// out = left . right in f32 as puter_hip_matmul, the split-K partials in `scratch`, a
-// part of a lease that the caller holds, of matmul_f32_scratch_bytes(...) bytes.
-size_t matmul_f32_scratch_bytes(int64_t rows, int64_t inner, int64_t cols);
-int matmul_f32_in_scratch(float *out, const float *left, const float *right, int64_t rows, int64_t inner, int64_t cols,
-                          hipStream_t s, float *scratch, size_t bytes);
 
 inline bool is_float_dtype(int dt) { return dt >= PUTER_F32 && dt <= PUTER_F8E5M2; }
 inline bool is_norm_dtype(int dt) { return dt == PUTER_F32 || dt == PUTER_F16 || dt == PUTER_BF16; }

@@ -103,16 +103,19 @@ __global__ __launch_bounds__(64) void flash_generic_kernel(FlashArgs a) {
 //     exp(s_j - M_j) * product of alpha_i over i > j,
 // so a prefix maximum and a suffix product over the row give the weights in any order of
 // evaluation (only the rounding of the products and of the sum differs).  Measured, the
-// error against float64 unchanged in each: f32 2048 x 2048 x 64 1249 -> 48 us (scores 17, weights
-// 13.5, product 18.5; the three are bound by their passes over the 16 MB of scores, which
-// the L2s and the last-level cache serve, and the float32 MFMA rate), 1000 x 1000 x 512 f32
-// 2488 -> 67, bf16 2334 -> 92; 64 x 64 x 64 38 -> 19; below 64 keys the general kernel runs.
+// error against float64 unchanged in each: f32 2048 x 2048 x 64 1249 -> 41 us (scores 16.5,
+// weights 12, product 13.5; the three are bound by their passes over the 16 MB of scores,
+// which are written non-temporally, 44.3 -> 41, and by the float32 MFMA rate, 3.5 us a
+// product), 1000 x 1000 x 512 f32 2488 -> 59, bf16 2334 -> 88; 64 x 64 x 64 38 -> 13; below
+// 64 keys the general kernel runs.  Scores from a tile staged in LDS: 43.5 against 44.3 at
+// depth 64, but 74 against 60 at 1000 x 1000 x 512.
 
 // S[r, k] = Q[q0 + r] . K[k] for 32 query rows and 4 x 64 keys a block: wave w owns keys
 // 64 w .. + 63 of the block's as two 32 x 32 accumulators.  A lane's operands for four
 // MFMA steps are 4 consecutive elements of its row (half h = lane / 32 takes d = 8 g + 4 h
 // .. + 3), read straight from memory: Q and K of one head stay in the caches.  VEC: rows
 // are whole 4-element pieces at their natural alignment.
+typedef float fl_f32x4 __attribute__((ext_vector_type(4)));
 typedef float fl_f32x16 __attribute__((ext_vector_type(16)));
 
 template <int DT, bool VEC>
@@ -174,9 +177,25 @@ __global__ __launch_bounds__(256) void flash_score_kernel(FlashArgs a, float *S,
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
             const int64_t r = r0 + 8 * (j >> 2) + 4 * h + (j & 3);
-            if (r < rows) S[r * ld + key] = acc[n][j];
+            if (r < rows) __builtin_nontemporal_store(acc[n][j], S + r * ld + key);
         }
     }
+}
+
+// flash_exp for x <= 0 or NaN (which passes through the polynomial)
+__device__ __forceinline__ float flash_exp_neg(float x) {
+    const float z = __fmul_rn(x, 1.4426950408889634f);
+    int32_t k = (int32_t)z;
+    if (z < 0) k--;
+    const float f = __fsub_rn(z, (float)k);
+    float p = __fmul_rn(f, 0.00133389f);
+    p = __fmul_rn(f, __fadd_rn(0.00961812f, p));
+    p = __fmul_rn(f, __fadd_rn(0.05550410f, p));
+    p = __fmul_rn(f, __fadd_rn(0.24022650f, p));
+    p = __fmul_rn(f, __fadd_rn(0.69314718f, p));
+    p = __fadd_rn(1.0f, p);
+    const float y = __uint_as_float(__float_as_uint(p) + ((uint32_t)k << 23));
+    return x < -87.33654f ? 0.0f : x != x ? x : y;
 }
 
 // Row r of S becomes its normalised weights, zeros on masked keys and on the columns
@@ -222,8 +241,8 @@ __global__ __launch_bounds__(1024) void flash_weights_kernel(FlashArgs a, float 
         if (seen && s[j] > m) m = s[j];
         const bool rescale = seen && (old != m || m == -INFINITY);
         alpha[j] = 1.0f;
-        if (__any(rescale)) alpha[j] = rescale ? flash_exp(old - m) : 1.0f;
-        s[j] = seen ? flash_exp(s[j] - m) : 0.0f;
+        if (__any(rescale)) alpha[j] = rescale ? flash_exp_neg(old - m) : 1.0f;
+        s[j] = seen ? flash_exp_neg(s[j] - m) : 0.0f;
     }
     float after = 1.0f;
 #pragma unroll
@@ -261,37 +280,81 @@ __global__ __launch_bounds__(1024) void flash_weights_kernel(FlashArgs a, float 
     const float inv = l != 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
     for (int j = 0; j < E; j += 4)
-        if (k0 + j < ld) *reinterpret_cast<float4 *>(row + k0 + j) = make_float4(s[j] * inv, s[j + 1] * inv, s[j + 2] * inv, s[j + 3] * inv);
+        if (k0 + j < ld)
+            __builtin_nontemporal_store((fl_f32x4){s[j] * inv, s[j + 1] * inv, s[j + 2] * inv, s[j + 3] * inv}, reinterpret_cast<fl_f32x4 *>(row + k0 + j));
 }
 
-// V as f32 with zero rows up to a multiple of 4 keys.
+// O[r, d] = sum over k of W[r, k] V[k, d] for 16 rows and 32 dims a block, its 8 waves
+// taking the 16-key groups w, w + 8, .. on v_mfma_f32_16x16x4_f32 and adding their sums in
+// LDS in wave order.  Lane (i = lane % 16, q = lane / 16) holds W[r0 + i][k + 4 q .. + 3] (one
+// 16-byte load a group) and V[k + 4 q + e][2 i, 2 i + 1] (e < 4), and MFMA (e, j) multiplies
+// k + 4 q + e into dim 2 i + j.  A causal block stops at its last row's key; a masked key's
+// zero weight times an infinite value is NaN in its products, while the general kernel
+// never reads that row, so an output that is not finite is summed again over the row's
+// own keys.  (The f32 Matmul in its place, with V widened or padded for it and the result
+// narrowed afterwards: 18.5 us against 13.5 at 2048 x 2048 x 64, 19 -> 13 the whole call at 64.)
 template <int DT>
-__global__ __launch_bounds__(256) void flash_values_kernel(float *dst, const void *v, int64_t n, int64_t padded) {
+__global__ __launch_bounds__(512) void flash_product_kernel(FlashArgs a, const float *W, int64_t ld, int64_t q0, int64_t rows) {
     using T = typename Elem<DT>::T;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < padded; i += (int64_t)gridDim.x * 256)
-        dst[i] = i < n ? Elem<DT>::load(static_cast<const T *>(v)[i]) : 0.0f;
-}
-
-// Narrows the f32 product (16-bit formats; from null: o holds f32 already), and sums again,
-// key by key, every causal row with an infinity or NaN in it: a masked key's zero weight
-// times an infinite value is NaN in the product, while its row is never read here.
-template <int DT>
-__global__ __launch_bounds__(64) void flash_finish_kernel(FlashArgs a, const float *W, const float *from, int64_t ld,
-                                                          int64_t q0) {
-    using T = typename Elem<DT>::T;
-    const int64_t r = blockIdx.x, vd = a.value_dim;
-    const int lane = threadIdx.x;
-    T *O = static_cast<T *>(a.o) + (q0 + r) * vd;
+    __shared__ float part[8][16][33];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
+    const int64_t r0 = (int64_t)blockIdx.x * 16, d0 = (int64_t)blockIdx.y * 32 + 2 * i, vd = a.value_dim;
+    const int64_t kend = a.causal ? std::min(a.seq_k, q0 + std::min(r0 + 16, rows)) : a.seq_k;
+    const float *w = W + std::min(r0 + i, rows - 1) * ld;
     const T *V = static_cast<const T *>(a.v);
-    for (int64_t d = lane; d < vd; d += kWave) {
-        float x = from ? from[r * vd + d] : Elem<DT>::load(O[d]);
-        if (a.causal && x * 0.0f != 0.0f) {
-            x = 0.0f;
-            const int64_t k_hi = min(a.seq_k, q0 + r + 1);
-            for (int64_t k = 0; k < k_hi; ++k) x += W[r * ld + k] * Elem<DT>::load(V[k * vd + d]);
-            O[d] = Elem<DT>::store(x);
-        } else if (from) O[d] = Elem<DT>::store(x);
+    const bool pair = d0 + 1 < vd, one = d0 < vd;
+    fl_f32x4 acc[2] = {(fl_f32x4){}, (fl_f32x4){}};
+    constexpr int U = 4;   // groups in flight
+    for (int64_t k0 = (int64_t)wave * 16; k0 < kend; k0 += 8 * 16 * U) {
+        float4 wv[U];
+        float v[U][4][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t k = k0 + u * 128 + 4 * q;
+            wv[u] = k < kend ? *reinterpret_cast<const float4 *>(w + k) : make_float4(0, 0, 0, 0);   // ld % 4 == 0
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[u][e][0] = v[u][e][1] = 0.0f;
+                if (k + e < kend) {
+                    const T *p = V + (k + e) * vd + d0;
+                    if (pair) {   // (8 or 4 bytes at any element)
+                        T t[2];
+                        __builtin_memcpy(t, p, sizeof(t));
+                        v[u][e][0] = Elem<DT>::load(t[0]);
+                        v[u][e][1] = Elem<DT>::load(t[1]);
+                    } else if (one) v[u][e][0] = Elem<DT>::load(p[0]);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    // (keys past kend: their weights count as zero against zero values)
+                    const float x = k0 + u * 128 + 4 * q + e < kend ? (&wv[u].x)[e] : 0.0f;
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, v[u][e][j], acc[j], 0, 0, 0);
+                }
     }
+    // register g of acc[j]: row 4 q + g, dim 2 i + j
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) part[wave][4 * q + g][2 * i + j] = acc[j][g];
+    __syncthreads();
+    const int row = threadIdx.x >> 5, col = threadIdx.x & 31;
+    float t = part[0][row][col];
+#pragma unroll
+    for (int x = 1; x < 8; ++x) t += part[x][row][col];
+    const int64_t r = r0 + row, d = (int64_t)blockIdx.y * 32 + col;
+    if (r >= rows || d >= vd) return;
+    if (a.causal && t * 0.0f != 0.0f) {
+        t = 0.0f;
+        const int64_t k_hi = std::min(a.seq_k, q0 + r + 1);
+        for (int64_t k = 0; k < k_hi; ++k) t += W[r * ld + k] * Elem<DT>::load(V[k * vd + d]);
+    }
+    static_cast<T *>(a.o)[(q0 + r) * vd + d] = Elem<DT>::store(t);
 }
 
 constexpr int64_t kFlashScores = (int64_t)64 << 20;   // bytes of scores held at once
@@ -302,26 +365,17 @@ constexpr int64_t kFlashMaxKeys = 16384;              // a row's keys in one blo
 template <int DT>
 static bool run_flash_passes(const FlashArgs &a, hipStream_t s, int *status) {
     if (a.seq_k < 64 || a.seq_k > kFlashMaxKeys) return false;
-    const int64_t ld = (a.seq_k + 3) / 4 * 4, vd = a.value_dim;
+    const int64_t ld = (a.seq_k + 3) / 4 * 4;
     const int64_t chunk = std::min<int64_t>(a.seq_q, std::max<int64_t>(32, kFlashScores / (ld * 4) / 32 * 32));
-    const bool widen = DT != PUTER_F32 || ld != a.seq_k, narrow = DT != PUTER_F32;
-    auto up = [](int64_t floats) { return (floats + 63) / 64 * 64; };
-    const int64_t n_s = up(chunk * ld), n_v = widen ? up(ld * vd) : 0, n_o = narrow ? up(chunk * vd) : 0;
-    const size_t part = matmul_f32_scratch_bytes(chunk, ld, vd);
-    const size_t need = (size_t)(n_s + n_v + n_o) * sizeof(float) + part;
+    const size_t need = (size_t)(chunk * ld) * sizeof(float);
     size_t held = 0;
     if (scratch_capturing(s, &held) && held < need) return false;
     ScratchLease lease(need, s);
     if (lease.status()) return false;
-    float *S = static_cast<float *>(lease.ptr()), *vf = S + n_s, *of = vf + n_v, *mm = of + n_o;
-    if (widen) {
-        const int64_t padded = ld * vd;
-        flash_values_kernel<DT><<<(unsigned)std::min<int64_t>((padded + 255) / 256, 2048), 256, 0, s>>>(vf, a.v, a.seq_k * vd, padded);
-    }
+    float *S = static_cast<float *>(lease.ptr());
     const uintptr_t align = DT == PUTER_F32 ? 15 : 7;
     const bool vec = a.depth % 4 == 0 && ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k)) & align) == 0;
-    int rc = PUTER_OK;
-    for (int64_t q0 = 0; q0 < a.seq_q && rc == PUTER_OK; q0 += chunk) {
+    for (int64_t q0 = 0; q0 < a.seq_q; q0 += chunk) {
         const int64_t rows = std::min(chunk, a.seq_q - q0);
         const dim3 grid((unsigned)((a.seq_k + 255) / 256), (unsigned)((rows + 31) / 32));
         if (vec) flash_score_kernel<DT, true><<<grid, 256, 0, s>>>(a, S, ld, q0, rows);
@@ -331,12 +385,9 @@ static bool run_flash_passes(const FlashArgs &a, hipStream_t s, int *status) {
         if (E == 4) flash_weights_kernel<DT, 4><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
         else if (E == 8) flash_weights_kernel<DT, 8><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
         else flash_weights_kernel<DT, 16><<<(unsigned)rows, T, 0, s>>>(a, S, ld, q0);
-        float *o = narrow ? of : static_cast<float *>(a.o) + q0 * vd;
-        rc = matmul_f32_in_scratch(o, S, widen ? vf : static_cast<const float *>(a.v), rows, ld, vd, s, mm, part);
-        if (narrow || a.causal)
-            flash_finish_kernel<DT><<<(unsigned)rows, 64, 0, s>>>(a, S, narrow ? of : nullptr, ld, q0);
+        flash_product_kernel<DT><<<dim3((unsigned)((rows + 15) / 16), (unsigned)((a.value_dim + 31) / 32)), 512, 0, s>>>(a, S, ld, q0, rows);
     }
-    if (rc == PUTER_OK) rc = check_launch("flash attention");
+    const int rc = check_launch("flash attention");
     const int fin = lease.finish();
     *status = rc ? rc : fin;
     return true;

@@ -1291,7 +1291,6 @@ static int address(float **out) {
 // else a lease of the library's growable scratch.
 struct PartialsTarget {
     float *fixed = nullptr;
-    size_t bytes = noalloc::kScratchBytes;   // of fixed
 };
 
 // Runs of K of the rows kernel: toward one block per CU (200 of 256 is near enough: 16 x
@@ -1396,9 +1395,9 @@ static int launch_skinny(void *out, const void *left, const void *right, int64_t
     const size_t need = (size_t)(chunks * M * N) * sizeof(float);
     const int64_t quads = M * N / 4;
     if (tgt.fixed) {
-        if (need > tgt.bytes)
+        if (need > noalloc::kScratchBytes)
             return fail(PUTER_ERR_INVALID, "matmul (no-alloc): split-K partials of %zu bytes exceed the %zu-byte scratch",
-                        need, tgt.bytes);
+                        need, noalloc::kScratchBytes);
         p.ws = tgt.fixed;
         matmul_skinny_kernel<DT><<<grid, 256, 0, s>>>(p);
         matmul_splitk_reduce_kernel<DT><<<(unsigned)std::min<int64_t>((quads + 255) / 256, 4096), 256, 0, s>>>(
@@ -1549,9 +1548,9 @@ static int launch_f32_mfma(float *out, const float *left, const float *right, in
         return check_launch("matmul f32 mfma split-k");
     };
     if (tgt.fixed) {
-        if (need > tgt.bytes)
+        if (need > noalloc::kScratchBytes)
             return fail(PUTER_ERR_INVALID, "matmul (no-alloc): split-K partials of %zu bytes exceed the %zu-byte scratch",
-                        need, tgt.bytes);
+                        need, noalloc::kScratchBytes);
         return launch(tgt.fixed);
     }
     ScratchLease lease(need, s);
@@ -1625,9 +1624,9 @@ static int launch_matmul_f32(float *out, const float *left, const float *right, 
         return check_launch("matmul split-k");
     };
     if (tgt.fixed) {
-        if (need > tgt.bytes)
+        if (need > noalloc::kScratchBytes)
             return fail(PUTER_ERR_INVALID, "matmul (no-alloc): split-K partials of %zu bytes exceed the %zu-byte scratch",
-                        need, tgt.bytes);
+                        need, noalloc::kScratchBytes);
         return launch(tgt.fixed);
     }
     ScratchLease lease(need, s);
@@ -1635,20 +1634,6 @@ static int launch_matmul_f32(float *out, const float *left, const float *right, 
     const int rc = launch(static_cast<float *>(lease.ptr()));
     const int fin = lease.finish();
     return rc ? rc : fin;
-}
-
-// (the split-K launches write at most 16 MiB of partials, and at most 64 chunks of them)
-size_t puter::matmul_f32_scratch_bytes(int64_t rows, int64_t inner, int64_t cols) {
-    if (rows * cols > (int64_t)(noalloc::kScratchBytes / sizeof(float))) return 0;
-    return std::min<size_t>(noalloc::kScratchBytes, (size_t)(64 * rows * cols) * sizeof(float));
-}
-
-int puter::matmul_f32_in_scratch(float *out, const float *left, const float *right, int64_t rows, int64_t inner,
-                                 int64_t cols, hipStream_t s, float *scratch, size_t bytes) {
-    PartialsTarget tgt;
-    tgt.fixed = scratch;
-    tgt.bytes = bytes;
-    return launch_matmul_f32(out, left, right, rows, inner, cols, s, tgt);
 }
 
 static int matmul_entry(void *out, const void *left, const void *right, int64_t rows, int64_t inner,
