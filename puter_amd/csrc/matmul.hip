@@ -223,6 +223,7 @@ typedef __bf16 mm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 mm_f16x8 __attribute__((ext_vector_type(8)));
 typedef short mm_i16x4 __attribute__((ext_vector_type(4)));
 typedef float mm_f32x16 __attribute__((ext_vector_type(16)));
+typedef float mm_f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int mm_u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void mm_lds_void;
 typedef __attribute__((address_space(3))) mm_i16x4 mm_lds_i16x4;
@@ -232,7 +233,17 @@ struct MmArgs {
     uint16_t *c;
     int M, N, K;
     int tiles_m, tiles_n, groups_m;  // groups_m: 4-tile groups along M
+    // two halves of K: the first K of the second half (a multiple of 64), the tile groups of
+    // one half, the pairs' sums ([tile][32][512 threads] float4) and counters
+    int kc, groups, set;
+    float *ws;
 };
+
+// Per scratch buffer and tile of the split 256 x 256 kernel: the blocks that have finished
+// their half (modulo 2), and the halves written and not yet fetched.  Both end each launch
+// as they began it, at zero.
+constexpr int kPairTiles = 384;
+static __device__ unsigned mm_finished[2][kPairTiles], mm_written[2][kPairTiles];
 
 template <int DT>
 __device__ __forceinline__ mm_f32x16 mm_mfma(const mm_i16x4 (&a)[2], const uint4 &b, mm_f32x16 acc) {
@@ -245,7 +256,7 @@ __device__ __forceinline__ mm_f32x16 mm_mfma(const mm_i16x4 (&a)[2], const uint4
                                                       __builtin_bit_cast(mm_f16x8, b), acc, 0, 0, 0);
 }
 
-template <int DT, int NW, int MT, int BK, int S>
+template <int DT, int NW, int MT, int BK, int S, bool PAIR>
 __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(MmArgs p) {
     using namespace mm;
     constexpr int BM = 64 * MT, BN = 64 * NW;   // 2 waves along M of 32 MT rows, NW along N of 64 columns
@@ -274,7 +285,12 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
 
     // block -> output tile: XCD x runs the 4 x 8 tile groups x, x + 8, ...
     const int id = blockIdx.x;
-    const int local = id >> 3, grp = (local >> 5) * 8 + (id & 7), w = local & 31;
+    const int local = id >> 3, w = local & 31;
+    int grp = (local >> 5) * 8 + (id & 7), half = 0;
+    if constexpr (PAIR) {
+        half = grp >= p.groups ? 1 : 0;
+        if (half) grp -= p.groups;
+    }
     const int tm = (grp % p.groups_m) * 4 + (w & 3);
     const int tn = (grp / p.groups_m) * 8 + (w >> 2);
     if (tm >= p.tiles_m || tn >= p.tiles_n) return;
@@ -369,13 +385,13 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
         }
     };
 
-    const int nk = (K + BK - 1) / BK;
+    const int k_lo = half ? p.kc : 0, nk = ((PAIR && !half ? p.kc : K) - k_lo + BK - 1) / BK;
     char *const abuf[4] = {as0, as1, as2, as3};
     char *const bbuf[4] = {bs0, bs1, bs2, bs3};
     // prologue: slices 0 .. S-2 in flight, slice 0 landed
 #pragma unroll
     for (int i = 0; i < S - 1; ++i)
-        if (i < nk) copy_slice(i * BK, abuf[i], bbuf[i]);
+        if (i < nk) copy_slice(k_lo + i * BK, abuf[i], bbuf[i]);
     if (S == 2 || nk < 2) __builtin_amdgcn_s_waitcnt(0x0F70);
     else if (S == 3) __builtin_amdgcn_s_waitcnt(0x0F70 | (APW + BPW));            // vmcnt(one slice)
     else if (nk < 3) __builtin_amdgcn_s_waitcnt(0x0F70 | (APW + BPW));
@@ -385,7 +401,7 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
     // wait for slice kt + 1
     auto slice = [&](int kt, int pos) __attribute__((always_inline)) {
         const int nxt = kt + S - 1;
-        if (nxt < nk) copy_slice(nxt * BK, abuf[(pos + S - 1) % S], bbuf[(pos + S - 1) % S]);
+        if (nxt < nk) copy_slice(k_lo + nxt * BK, abuf[(pos + S - 1) % S], bbuf[(pos + S - 1) % S]);
         // keep the copies ahead of the compute: left alone, the scheduler sinks them
         // to the end of the slice, right before the wait, exposing their latency
         __builtin_amdgcn_sched_barrier(0);
@@ -404,6 +420,53 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < S; ++i)
         if (kt + i < nk) slice(kt + i, i);
+
+    // Two halves: whichever block finishes first leaves its sums in ws and ends; the other
+    // waits for them (their writer is past its last wait, so they come) and adds them to
+    // its own, an addition of two floats that does not depend on the order.  Device-scope
+    // stores, a wait for them and a relaxed counter, as in the rows kernel; the counter of
+    // written halves is taken down by one, so that calls which break the rule on shared
+    // scratch could mix up sums but never wait for good.
+    if constexpr (PAIR) {
+        constexpr int SC1 = 16;
+        __shared__ int second;
+        const int slot = tm * p.tiles_n + tn;
+        const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(p.ws + (int64_t)slot * (BM * BN)), (short)0, BM * BN * 4, BUF_WORD3);
+        if (tid == 0) second = (int)atomicInc(&mm_finished[p.set][slot], 1u);
+        __syncthreads();
+        if (!__builtin_amdgcn_readfirstlane(second)) {
+#pragma unroll
+            for (int j = 0; j < 8 * MT; ++j) {
+                const mm_f32x16 &f = acc[j >> 3][j >> 2 & 1];
+                const mm_f32x4 v = {f[4 * (j & 3)], f[4 * (j & 3) + 1], f[4 * (j & 3) + 2], f[4 * (j & 3) + 3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(mm_u32x4, v), ws, tid * 16, j * (128 * NW * 16), SC1);
+            }
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's sums are at the coherence point
+            __syncthreads();
+            if (tid == 0) atomicAdd(&mm_written[p.set][slot], 1u);
+            return;
+        }
+        if (tid == 0) {
+            for (;;) {
+                const unsigned n = __hip_atomic_load(&mm_written[p.set][slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (n && atomicCAS(&mm_written[p.set][slot], n, n - 1) == n) break;
+                __builtin_amdgcn_s_sleep(2);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j0 = 0; j0 < 8 * MT; j0 += 8) {   // (eight loads in flight: in batches of four 3072 x 8192 x 8192 takes 365 us, not 353)
+            mm_f32x4 v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                v[j] = __builtin_bit_cast(mm_f32x4, __builtin_amdgcn_raw_buffer_load_b128(ws, tid * 16, (j0 + j) * (128 * NW * 16), SC1));
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[j0 >> 3][j >> 2][4 * (j & 3) + e] += v[j][e];
+        }
+    }
 
     // Epilogue.  Lane holds C[m0 + WR wm + 32 mt + l32][n0 + 64 wn + 32 nt + 8 (r/4) +
     // 4 g + r%4]: stored straight from the accumulators, each store instruction would
@@ -467,28 +530,55 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
     }
 }
 
+// The arguments of a tiling by 64 NW columns and 64 MT rows (64-deep slices); false when the
+// shape does not fit the kernel.
+static bool mfma_args(MmArgs &p, int nw, int mt, void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N) {
+    if (256 * K * 2 >= mm::OOB || 64 * N * 2 >= mm::OOB || M > 0x3FFFFFFF || N > 0x3FFFFFFF) return false;
+    p = {};
+    p.a = static_cast<const uint16_t *>(left);
+    p.b = static_cast<const uint16_t *>(right);
+    p.c = static_cast<uint16_t *>(out);
+    p.M = (int)M; p.N = (int)N; p.K = (int)K;
+    p.tiles_m = (int)((M + 64 * mt - 1) / (64 * mt));
+    p.tiles_n = (int)((N + 64 * nw - 1) / (64 * nw));
+    p.groups_m = (p.tiles_m + 3) / 4;
+    const int64_t groups = (int64_t)p.groups_m * ((p.tiles_n + 7) / 8);
+    if ((groups + 7) / 8 * 8 * 32 > 0x7FFFFFFF) return false;
+    p.groups = (int)groups;
+    return true;
+}
+
 // Launches the MFMA kernel with NW waves along N and MT accumulator blocks of 32
 // rows per wave (256 x 256 tiles: NW = 4, MT = 4; 128 x 128: NW = 2, MT = 2), 64-deep
 // slices double buffered; returns 1 when the shape does not fit it.
 template <int DT, int NW, int MT>
 static int launch_mfma(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N,
                        hipStream_t s) {
-    constexpr int BK = 64, S = 2;
-    constexpr int BM = 64 * MT;
-    if (256 * K * 2 >= mm::OOB || BK * N * 2 >= mm::OOB || M > 0x3FFFFFFF || N > 0x3FFFFFFF) return 1;
     MmArgs p;
-    p.a = static_cast<const uint16_t *>(left);
-    p.b = static_cast<const uint16_t *>(right);
-    p.c = static_cast<uint16_t *>(out);
-    p.M = (int)M; p.N = (int)N; p.K = (int)K;
-    p.tiles_m = (int)((M + BM - 1) / BM);
-    p.tiles_n = (int)((N + 64 * NW - 1) / (64 * NW));
-    p.groups_m = (p.tiles_m + 3) / 4;
-    const int64_t groups = (int64_t)p.groups_m * ((p.tiles_n + 7) / 8);
-    const int64_t blocks = (groups + 7) / 8 * 8 * 32;
-    if (blocks > 0x7FFFFFFF) return 1;
-    matmul_mfma_kernel<DT, NW, MT, BK, S><<<(unsigned)blocks, 128 * NW, 0, s>>>(p);
+    if (!mfma_args(p, NW, MT, out, left, right, M, K, N)) return 1;
+    const unsigned blocks = (unsigned)((p.groups + 7) / 8 * 8 * 32);
+    matmul_mfma_kernel<DT, NW, MT, 64, 2, false><<<blocks, 128 * NW, 0, s>>>(p);
     return 0;
+}
+
+// The 256 x 256 tiles with K in two halves, two blocks a tile.  Returns 1 when the shape does
+// not fit or the scratch has no room, which the undivided kernels do not need.
+template <int DT>
+static int launch_mfma_pair(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s) {
+    MmArgs p;
+    if (!mfma_args(p, 4, 4, out, left, right, M, K, N)) return 1;
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+    if (tiles > kPairTiles) return 1;
+    const size_t need = (size_t)tiles * 256 * 256 * sizeof(float);
+    size_t held = 0;
+    if (scratch_capturing(s, &held)) return 1;   // graphs of these shapes may replay side by side
+    ScratchLease lease(need, s);
+    if (lease.status()) return 1;
+    p.kc = (int)((K + 127) / 128 * 64);
+    p.ws = static_cast<float *>(lease.ptr());
+    p.set = lease.set();
+    matmul_mfma_kernel<DT, 4, 4, 64, 2, true><<<(unsigned)((2 * p.groups + 7) / 8 * 8 * 32), 512, 0, s>>>(p);
+    return lease.finish();
 }
 
 // ---------------------------------------------------------- f32 MFMA --
@@ -1180,6 +1270,7 @@ static int scratch_acquire(SplitScratch &sc, size_t need, hipStream_t s) {
         }
         const size_t grown = (need + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
         if (hipMallocAsync(&sc.ptr, grown, s) != hipSuccess) {
+            (void)hipGetLastError();   // (a caller that runs without scratch must not find it)
             sc.ptr = nullptr;
             return fail(PUTER_ERR_UNAVAILABLE, "matmul: split-K scratch of %zu bytes unavailable", grown);
         }
@@ -1441,6 +1532,20 @@ static bool mfma_small_tiles(int64_t M, int64_t N) {
     return 59 * r_small < 100 * r_large;
 }
 
+// 256 x 256 tiles with K in two halves: twice the blocks of half the work, for grids that fill
+// half a round (or one and a half) of them.  In units of 1/100 of a large round: a half round
+// 50, and 30 us (1200 / K of a round) for the sums that change hands; a small round 55, the
+// launch's first and last slices 11 (one small round measured 66, three 165 - 190).
+// 2000 x 14336 x 4096 247 -> 211 us, 2048 x 8192 x 4096 142 -> 125, 2048 x 28672 x 4096 488 ->
+// 388, 3072 x 8192 x 8192 (one and a half) 404 -> 353; where it would lose: 2048 x 4096 x
+// 4096 73.6 against 74.3, 5120 x 4096 x 4096 184 against 192.
+static bool mfma_pair_wins(int64_t M, int64_t K, int64_t N) {
+    const int64_t cus = device_cus();
+    const int64_t large = ((M + 255) / 256) * ((N + 255) / 256), small = ((M + 127) / 128) * ((N + 127) / 128);
+    const int64_t r_large = (large + cus - 1) / cus, r_small = (small + 2 * cus - 1) / (2 * cus), r_pair = (2 * large + cus - 1) / cus;
+    return large <= kPairTiles && K >= 2048 && 50 * r_pair + 120000 / K < std::min(100 * r_large, 55 * r_small + 11);
+}
+
 template <int DT>
 static int launch_matmul16(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N,
                            hipStream_t s, PartialsTarget tgt) {
@@ -1487,6 +1592,10 @@ static int launch_matmul16(void *out, const void *left, const void *right, int64
         if (M <= 512 || few_tiles) {
             const int rc = launch_skinny<DT>(out, left, right, M, K, N, s, tgt, M <= 512 ? 0 : 1024);
             if (rc != 1) return rc;
+        }
+        if (!tgt.fixed && mfma_pair_wins(M, K, N)) {
+            const int rc = launch_mfma_pair<DT>(out, left, right, M, K, N, s);
+            if (rc != 1) return rc ? rc : check_launch("matmul mfma");
         }
         const int rc = mfma_small_tiles(M, N) ? launch_mfma<DT, 2, 2>(out, left, right, M, K, N, s)
                                               : launch_mfma<DT, 4, 4>(out, left, right, M, K, N, s);

@@ -457,3 +457,39 @@ def test_matmul_empty_inner_is_zero(backend, dt, np_dt):
     dummy = to_dev(np.zeros(8, np_dt))
     backend.Matmul(out, dummy, dummy, rows, 0, cols, dt)
     assert not to_host(out, np_dt).any()
+
+
+@pytest.mark.parametrize("dt", [O.BF16, O.F16])
+@pytest.mark.parametrize("rows,inner,cols", [
+    (2041, 8200, 4088),    # half a round of 256 x 256 tiles; ragged rows and columns, the second half of K ragged
+    (1793, 16384, 4096),   # the last row tile of one row
+    (4100, 7752, 4096),    # one and a half rounds, row tiles past a multiple of four
+])
+def test_matmul_16bit_two_halves_of_k_exact(backend, dt, rows, inner, cols):
+    """256 x 256 tiles whose K is divided between two blocks, bit for bit: integer operands keep
+    every sum exact.  On the default stream and on a side stream (each has its own sums and
+    counters) without synchronisation between the calls, and under capture, which takes the
+    undivided kernel."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    t = torch.bfloat16 if dt == O.BF16 else torch.float16
+    xs = [(torch.randint(-2, 3, (rows, inner), device="cuda", generator=g).to(t),
+           torch.randint(-2, 3, (inner, cols), device="cuda", generator=g).to(t)) for _ in range(2)]
+    want = [(a.float() @ b.float()).to(t) for a, b in xs]
+    outs = [torch.full((rows + 1, cols), 7, dtype=t, device="cuda") for _ in range(6)]
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        with torch.cuda.stream(side if i & 1 else torch.cuda.default_stream()):
+            backend.Matmul(o, *xs[i // 2 % 2], rows, inner, cols, dt)
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        assert torch.equal(o[:rows], want[i // 2 % 2]) and (o[rows] == 7).all(), i
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        backend.Matmul(outs[0], *xs[1], rows, inner, cols, dt)
+    for _ in range(3):
+        outs[0].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(outs[0][:rows], want[1])
