@@ -18,17 +18,18 @@
  *     puter_hip_paged_decode_workspace_bytes).  The one allocation the library
  *     makes itself is a split-K scratch shared by puter_hip_matmul (16-bit
  *     formats with at most 512 rows or under two rounds of 128x128 tiles, or of
- *     sizes or alignments that the 16-byte copies cannot take (which run unsplit
- *     where the scratch has no room), F32
+ *     sizes or alignments that the 16-byte copies cannot take, or of grids of
+ *     256x256 tiles that fill about half a round, F32
  *     outputs of fewer 128x128 tiles than the device has CUs, when K is split
  *     across blocks rather than inside them) and
  *     puter_hip_multi_head_attention[_batched] with seq_q == 1 (bf16 / f16 at
  *     head dim 128 without ALiBi, or any row over more than 768 keys) or in F32
  *     with at least 16 query rows, a head dim that is a multiple of 4, and
  *     fewer 128-query blocks than two per CU (causal) or one per CU (not
- *     causal): two buffers per device (the default stream's, and one for all
- *     other streams), each allocated on first use and grown on
- *     demand (Matmul: at most 16 MiB; one-row attention: the paged decode
+ *     causal): four buffers per device (the default stream's and one for all
+ *     other streams, each once for calls that also run on scratch under capture
+ *     and once for those that do not), allocated on first use and grown on
+ *     demand (Matmul: at most 16 MiB, 96 MiB for 256x256 tiles; one-row attention: the paged decode
  *     workspace size, or batch x heads x ceil(seq_k / 256) x (head_dim + 2)
  *     floats; F32 attention: key splits x batch x seq_q x heads x (head_dim +
  *     2) floats, at most about 100 MB; scaled-dot-product attention: see there).
@@ -39,8 +40,10 @@
  *     use the buffer held if it is large enough (the graph keeps its address,
  *     so that buffer is never freed: a later growth keeps it and allocates
  *     beside it) and otherwise return PUTER_ERR_INVALID before launching; make
- *     the same call, or a larger one, outside the capture first (F32 attention
- *     takes its unsplit kernel under capture and uses no scratch).  Replays share
+ *     the same call, or a larger one, outside the capture first (F32 attention,
+ *     scaled-dot-product attention, and Matmul with unaligned 16-bit operands or in
+ *     256x256 tiles use no scratch under capture, and where an eager call of theirs
+ *     finds no room it runs without).  Replays share
  *     the buffer with eager scratch-using calls until such a growth, so the
  *     caller orders them (one stream, or its own events).
  *
@@ -322,9 +325,8 @@ typedef struct puter_flash_config {
  * interface.go:104-109: one head, Q [seqQ, depth], K [seqK, depth], V [seqK, valueDim],
  * O [seqQ, valueDim]; online softmax through FastExp32 (cpu/attention/typed_compute.go:31-97).
  * depth <= 8192, valueDim <= 1024 (beyond: PUTER_ERR_INVALID).  F32 and the 16-bit
- * head sizes past the MFMA prefill kernel's keep up to 64 MiB of scores (and f32
- * copies of V and of the output where needed) in the library's scratch, for 64 to
- * 16384 keys; under stream capture only if the scratch held has that room. */
+ * head sizes past the MFMA prefill kernel's keep up to 64 MiB of scores in the library's
+ * scratch, for 64 to 16384 keys; under stream capture they run without. */
 PUTER_API int puter_hip_scaled_dot_product_attention(const puter_flash_config *config,
                                            const void *query, const void *key, const void *value,
                                            void *output, int64_t seq_q, int64_t seq_k,

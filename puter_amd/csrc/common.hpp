@@ -29,16 +29,19 @@ int device_cus();
 // device's lock is held from construction to destruction.  On a stream that is
 // capturing a graph the lease neither grows, orders nor records: it hands out the
 // buffer it finds (never freed afterwards) or fails with PUTER_ERR_INVALID when
-// that is too small.
+// that is too small.  An eager-only lease is for calls that run without scratch under
+// capture: it takes one of two further buffers, which no graph ever holds, so that such a
+// call on one stream needs no order with the replays of a graph on another.
 struct SplitScratch;
 class ScratchLease {
 public:
-    ScratchLease(size_t bytes, hipStream_t s);
+    ScratchLease(size_t bytes, hipStream_t s, bool eager_only = false);
     ScratchLease(const ScratchLease &) = delete;
     ScratchLease &operator=(const ScratchLease &) = delete;
     int status() const { return status_; }
     void *ptr() const { return ptr_; }
-    int set() const { return set_; }  // 0: the default stream's buffer, 1: the other streams'
+    // 0: the default stream's buffer, 1: the other streams'; 2 and 3: the eager-only ones
+    int set() const { return set_; }
     int finish();  // call once, after the launches that use ptr()
 private:
     SplitScratch *sc_ = nullptr;
@@ -51,8 +54,8 @@ private:
 };
 
 // Whether s is recording a graph (or cannot be asked); if so, the bytes that the largest
-// of the device's scratch buffers holds, which is all a lease can get (matmul.hip).
-bool scratch_capturing(hipStream_t s, size_t *held);
+// of the buffers that a graph may use holds, which is all a lease can get (matmul.hip).
+bool scratch_capturing(hipStream_t s, size_t *held = nullptr);
 
 inline bool is_float_dtype(int dt) { return dt >= PUTER_F32 && dt <= PUTER_F8E5M2; }
 inline bool is_norm_dtype(int dt) { return dt == PUTER_F32 || dt == PUTER_F16 || dt == PUTER_BF16; }

@@ -360,17 +360,16 @@ __global__ __launch_bounds__(512) void flash_product_kernel(FlashArgs a, const f
 constexpr int64_t kFlashScores = (int64_t)64 << 20;   // bytes of scores held at once
 constexpr int64_t kFlashMaxKeys = 16384;              // a row's keys in one block's registers
 
-// Returns false when the general kernel is to run: few keys, rows past a block, or a
-// stream capture whose scratch has no room.
+// Returns false when the general kernel is to run: few keys, rows past a block, a
+// stream capture (graphs of these calls may replay side by side), or no room.
 template <int DT>
 static bool run_flash_passes(const FlashArgs &a, hipStream_t s, int *status) {
     if (a.seq_k < 64 || a.seq_k > kFlashMaxKeys) return false;
     const int64_t ld = (a.seq_k + 3) / 4 * 4;
     const int64_t chunk = std::min<int64_t>(a.seq_q, std::max<int64_t>(32, kFlashScores / (ld * 4) / 32 * 32));
     const size_t need = (size_t)(chunk * ld) * sizeof(float);
-    size_t held = 0;
-    if (scratch_capturing(s, &held) && held < need) return false;
-    ScratchLease lease(need, s);
+    if (scratch_capturing(s)) return false;
+    ScratchLease lease(need, s, true);
     if (lease.status()) return false;
     float *S = static_cast<float *>(lease.ptr());
     const uintptr_t align = DT == PUTER_F32 ? 15 : 7;

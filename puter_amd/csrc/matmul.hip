@@ -243,7 +243,7 @@ struct MmArgs {
 // their half (modulo 2), and the halves written and not yet fetched.  Both end each launch
 // as they began it, at zero.
 constexpr int kPairTiles = 384;
-static __device__ unsigned mm_finished[2][kPairTiles], mm_written[2][kPairTiles];
+static __device__ unsigned mm_finished[2][kPairTiles], mm_written[2][kPairTiles];   // [the default stream, others]
 
 template <int DT>
 __device__ __forceinline__ mm_f32x16 mm_mfma(const mm_i16x4 (&a)[2], const uint4 &b, mm_f32x16 acc) {
@@ -570,13 +570,12 @@ static int launch_mfma_pair(void *out, const void *left, const void *right, int6
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     if (tiles > kPairTiles) return 1;
     const size_t need = (size_t)tiles * 256 * 256 * sizeof(float);
-    size_t held = 0;
-    if (scratch_capturing(s, &held)) return 1;   // graphs of these shapes may replay side by side
-    ScratchLease lease(need, s);
+    if (scratch_capturing(s)) return 1;
+    ScratchLease lease(need, s, true);
     if (lease.status()) return 1;
     p.kc = (int)((K + 127) / 128 * 64);
     p.ws = static_cast<float *>(lease.ptr());
-    p.set = lease.set();
+    p.set = lease.set() & 1;
     matmul_mfma_kernel<DT, 4, 4, 64, 2, true><<<(unsigned)((2 * p.groups + 7) / 8 * 8 * 32), 512, 0, s>>>(p);
     return lease.finish();
 }
@@ -863,10 +862,10 @@ typedef float rw_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRwCols = 128, kRwDepth = 32, kRwWaves = 4, kRwRows = 16, kRwPad = kRwCols + 4;
 constexpr int kRwMaxTiles = 16384;   // column tiles of a split launch, at most
 // per device: the column tiles' arrival counters, zero between launches (the last block's
-// atomicInc wraps to zero): a set beside each of the two growable scratch buffers and one
+// atomicInc wraps to zero): a set beside each of the four growable scratch buffers and one
 // beside the no-alloc entry point's array, each used by one launch at a time like the
 // scratch it stands by
-static __device__ unsigned rw_arrived[3][kRwMaxTiles];
+static __device__ unsigned rw_arrived[5][kRwMaxTiles];
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) {   // 16 bytes at any element
     uint4 v;
@@ -1207,9 +1206,10 @@ __global__ __launch_bounds__(256) void matmul_splitk_reduce_kernel(uint16_t *c, 
     }
 }
 
-// Split-K partials: two scratch buffers per device, kept for the life of the process
+// Split-K partials: four scratch buffers per device, kept for the life of the process
 // and grown on demand: one for the default (null) stream, whose own order keeps its
-// calls apart, and one for all other streams.  On the latter a call on another stream
+// calls apart, and one for all other streams, each twice: the eager-only pair serves calls
+// that take no scratch under capture, so no graph holds it.  On another stream's buffer a call on another stream
 // than the buffer's last user first waits (on the device, hipStreamWaitEvent) for that
 // user's completion event, so calls on different streams never overlap on the buffer.
 // (The event's record costs 3.2 us of device time a call: seven split Matmuls of a
@@ -1238,7 +1238,7 @@ struct SplitScratch {
     bool pinned = false;        // a captured graph holds ptr
     std::vector<void *> retired;  // pinned buffers replaced by a growth
 };
-static SplitScratch g_split_scratch[64][2];   // [device][0: the default stream, 1: all others]
+static SplitScratch g_split_scratch[64][4];   // [device][0: the default stream, 1: all others; 2, 3: eager-only]
 
 // Whether s is recording a graph (an invalidated capture counts: it must not
 // allocate either).
@@ -1282,18 +1282,19 @@ static int scratch_acquire(SplitScratch &sc, size_t need, hipStream_t s) {
 bool scratch_capturing(hipStream_t s, size_t *held) {
     int dev = 0;
     bool capturing = true;
-    *held = 0;
+    if (held) *held = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return true;
     if (stream_capturing(s, &capturing) != PUTER_OK) return true;
     if (!capturing) return false;
-    for (SplitScratch &sc : g_split_scratch[dev]) {
+    for (int set = 0; held && set < 2; ++set) {
+        SplitScratch &sc = g_split_scratch[dev][set];
         std::lock_guard<std::mutex> g(sc.mu);
         *held = std::max(*held, sc.bytes);
     }
     return true;
 }
 
-ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
+ScratchLease::ScratchLease(size_t bytes, hipStream_t s, bool eager_only) : s_(s) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
         status_ = fail(PUTER_ERR_UNAVAILABLE, "scratch: no device");
@@ -1301,7 +1302,11 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
     }
     bool capturing = false;
     if ((status_ = stream_capturing(s, &capturing)) != PUTER_OK) return;
-    set_ = s ? 1 : 0;
+    if (eager_only && capturing) {
+        status_ = fail(PUTER_ERR_INVALID, "scratch: not held for this call under stream capture");
+        return;
+    }
+    set_ = (s ? 1 : 0) + (eager_only ? 2 : 0);
     sc_ = &g_split_scratch[dev][set_];
     lock_ = std::unique_lock<std::mutex>(sc_->mu);
     if (capturing) {
@@ -1335,7 +1340,7 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s) : s_(s) {
 
 int ScratchLease::finish() {
     if (status_ != PUTER_OK) return status_;
-    if (captured_ || set_ == 0) return PUTER_OK;   // the default stream orders its own calls
+    if (captured_ || (set_ & 1) == 0) return PUTER_OK;   // the default stream orders its own calls
     if (hipEventRecord(sc_->done, s_) != hipSuccess) return fail(PUTER_ERR_LAUNCH, "scratch: cannot record the event");
     sc_->last = s_;
     sc_->used = true;
@@ -1406,8 +1411,8 @@ static int64_t skinny_chunks(int64_t M, int64_t K, int64_t N, int64_t min_depth)
 }
 
 // general: the shape or alignment is one that only the generic kernel (which needs no
-// scratch) would take otherwise, so a split that finds no room runs unsplit; else, under
-// stream capture, the call is held to what the skinny kernel asked of the scratch: it fails
+// scratch) would take otherwise, so it runs unsplit under stream capture and where a split
+// finds no room; else, under capture, the call is held to what the skinny kernel asked of the scratch: it fails
 // where that did not fit, and otherwise takes as many runs as fit.
 template <int DT, int MT>
 static int launch_rows_mt(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s,
@@ -1419,25 +1424,26 @@ static int launch_rows_mt(void *out, const void *left, const void *right, int64_
     const int64_t unit = tiles * mtiles * std::min<int64_t>(M, kRwRows * MT) * kRwCols * (int64_t)sizeof(float);   // sums of one run
     int64_t chunks = tiles * mtiles <= kRwMaxTiles ? rows_chunks(tiles * mtiles, K) : 1;
     chunks = std::min<int64_t>(chunks, std::max<int64_t>(1, (int64_t)noalloc::kScratchBytes / unit));
+    if (general && chunks > 1 && !tgt.fixed && scratch_capturing(s)) chunks = 1;
     if (chunks > 1 && !tgt.fixed) {
         size_t held = 0;
         if (scratch_capturing(s, &held) && held < (size_t)(chunks * unit)) {
             const int64_t old = skinny_chunks(M, K, N, 0);
             const size_t need = old > 1 ? (size_t)(old * M * N) * sizeof(float) : 0;
-            if (general || held >= need) chunks = std::max<int64_t>(1, (int64_t)held / unit);
+            if (held >= need) chunks = std::max<int64_t>(1, (int64_t)held / unit);
         }
     }
     const int64_t per = (steps + chunks - 1) / chunks;
     chunks = (steps + per - 1) / per;
     RwArgs p{static_cast<uint16_t *>(out), static_cast<const uint16_t *>(left), static_cast<const uint16_t *>(right), tgt.fixed,
-             (int)M, (int)tiles, (int)chunks, (int)mtiles, 2, K, N, per * STEP};
+             (int)M, (int)tiles, (int)chunks, (int)mtiles, 4, K, N, per * STEP};
     auto launch = [&] {
         const int64_t blocks = (tiles * p.chunks + 7) / 8 * 8 * mtiles;
         matmul_rows_kernel<DT, MT><<<(unsigned)blocks, 256, 0, s>>>(p);
         return check_launch("matmul rows");
     };
     if (chunks == 1 || tgt.fixed) return launch();
-    ScratchLease lease((size_t)(chunks * unit), s);
+    ScratchLease lease((size_t)(chunks * unit), s, general);
     if (lease.status()) {
         if (!general) return lease.status();
         p.chunks = 1;

@@ -1226,22 +1226,21 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
         splits = (ktiles + a.split_tiles - 1) / a.split_tiles;
         const int64_t rows = m.batch * m.seq_q * m.heads;
         const size_t need = (size_t)(splits * rows) * (sizeof(float2) + (size_t)m.dim * sizeof(float));
-        ScratchLease lease(need, s);
-        if (lease.status()) {
-            *status = lease.status();
+        ScratchLease lease(need, s, true);
+        if (!lease.status()) {
+            // outputs first: splits * rows * D floats keep the (max, sum) pairs 16-byte aligned
+            a.part_o = static_cast<float *>(lease.ptr());
+            a.part_ml = reinterpret_cast<float2 *>(a.part_o + splits * rows * m.dim);
+            const dim3 grid((unsigned)blocks, (unsigned)splits);
+            const unsigned cblocks = (unsigned)((rows + 3) / 4);
+            launch(grid);
+            prefill_f32_combine_kernel<<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
+            const int rc = check_launch("prefill f32 mfma split");
+            const int fin = lease.finish();
+            *status = rc ? rc : fin;
             return true;
         }
-        // outputs first: splits * rows * D floats keep the (max, sum) pairs 16-byte aligned
-        a.part_o = static_cast<float *>(lease.ptr());
-        a.part_ml = reinterpret_cast<float2 *>(a.part_o + splits * rows * m.dim);
-        const dim3 grid((unsigned)blocks, (unsigned)splits);
-        const unsigned cblocks = (unsigned)((rows + 3) / 4);
-        launch(grid);
-        prefill_f32_combine_kernel<<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
-        const int rc = check_launch("prefill f32 mfma split");
-        const int fin = lease.finish();
-        *status = rc ? rc : fin;
-        return true;
+        a.split_tiles = 0;   // no room: unsplit
     }
     launch(dim3((unsigned)blocks));
     *status = check_launch("prefill f32 mfma");

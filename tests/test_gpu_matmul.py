@@ -429,8 +429,8 @@ def test_matmul_default_and_side_streams_keep_apart(backend):
 
 def test_matmul_unaligned_captured_without_scratch(backend):
     """A shape that only the rows kernel takes was never refused under stream capture (the
-    generic kernel needs no scratch): captured, it splits K only as far as the scratch held
-    allows, and its replays with new operands are exact."""
+    generic kernel needs no scratch): captured, it does not split K, so graphs of it need no
+    order among themselves, and its replays with new operands are exact."""
     import torch
     rows, inner, cols = 3, 4000, 1001
     rng = np.random.default_rng(5)

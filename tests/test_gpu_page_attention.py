@@ -956,3 +956,35 @@ def test_matmul_f32(backend):
         out = empty_dev((rows, cols), np.float32)
         backend.Matmul(out, to_dev(a), to_dev(b), rows, inner, cols, O.F32)
         assert_close(to_host(out, np.float32), ref, TOL[O.F32], elem_tol=1e-3, what="matmul")
+
+
+def test_flash_f32_captured_beside_eager_calls(backend):
+    """A captured f32 call takes no scratch (it was never refused there): its replays agree with
+    the oracle and need no order with eager calls on another stream, whose scores are in
+    the scratch and stay what they are alone."""
+    import puter_amd
+    import torch
+    s, d = 200, 32
+    q, k, v = (seeded(580 + i, (s, d), 0.0, 0.3) for i in range(3))
+    ref = O.flash_attention(q, k, v, causal=True, dtype=O.F32)
+    qd, kd, vd = to_dev(q), to_dev(k), to_dev(v)
+    cfg = puter_amd.FlashAttentionConfig(64, True)
+    alone, out = empty_dev((s, d), np.float32), empty_dev((s, d), np.float32)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        backend.FlashAttention(cfg, qd, kd, vd, out, s, s, d, d, O.F32)
+    backend.FlashAttention(cfg, qd, kd, vd, alone, s, s, d, d, O.F32)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        eager = [empty_dev((s, d), np.float32) for _ in range(4)]
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        with torch.cuda.stream(side):
+            for e in eager:
+                backend.FlashAttention(cfg, qd, kd, vd, e, s, s, d, d, O.F32)
+        torch.cuda.synchronize()
+        assert_close(to_host(out, np.float32), ref, TOL[O.F32], elem_tol=1e-3, what="captured flash")
+        for e in eager:
+            assert np.array_equal(to_host(e, np.float32), to_host(alone, np.float32))
