@@ -1046,7 +1046,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void matmul_rows_kernel(RwArg
 // columns 32 w .. +31 as 2 accumulators (rows 0..31, 32..63).  LDS layouts: A rows
 // of 128 bytes, chunk c of row r at c ^ (r/2 % 8); B rows of 256 bytes, chunk c at
 // c ^ 4 (r % 4).  With more than one chunk, each block writes its f32 partial tile to
-// a scratch buffer (the library's, one per device) and matmul_splitk_reduce_kernel
+// a scratch buffer (the library's) and matmul_splitk_reduce_kernel
 // sums the chunks in order (so the result does not depend on scheduling) and
 // rounds once.
 namespace sk {

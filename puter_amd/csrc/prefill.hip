@@ -769,7 +769,7 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
 }
 
 // ------------------------------------------------------------ f32 prefill --
-// f32 MultiHeadAttention (head dim 128 or 64, causal or not, sliding window, ALiBi) on
+// f32 MultiHeadAttention (head dim 128 or 64, or any multiple of 4 up to 256; causal or not, sliding window, ALiBi) on
 // v_mfma_f32_32x32x2_f32: exact f32 products, f32 sums, softmax in f32 against a
 // running maximum (the reference's stableSoftmaxRow takes the row max, exp in
 // float64 and a sequential f32 sum; the order of the sums differs, the f32 bar
