@@ -33,24 +33,24 @@ int device_cus();
 // capture: it takes one of two further buffers, which no graph ever holds, so that such a
 // call on one stream needs no order with the replays of a graph on another.
 struct SplitScratch;
+struct ScratchCounters;   // a buffer's counters, at its start (matmul.hip)
 class ScratchLease {
 public:
     ScratchLease(size_t bytes, hipStream_t s, bool eager_only = false);
     ScratchLease(const ScratchLease &) = delete;
     ScratchLease &operator=(const ScratchLease &) = delete;
     int status() const { return status_; }
-    void *ptr() const { return ptr_; }
-    // 0: the default stream's buffer, 1: the other streams'; 2 and 3: the eager-only ones
-    int set() const { return set_; }
+    void *ptr() const;   // the buffer behind its counters
+    ScratchCounters *counters() const { return counters_; }
     int finish();  // call once, after the launches that use ptr()
 private:
     SplitScratch *sc_ = nullptr;
     std::unique_lock<std::mutex> lock_;
     hipStream_t s_;
-    void *ptr_ = nullptr;
+    ScratchCounters *counters_ = nullptr;
     int status_ = 0;
     bool captured_ = false;
-    int set_ = 0;
+    bool ordered_ = false;   // on the default stream
 };
 
 // Whether s is recording a graph (or cannot be asked); if so, the bytes that the largest

@@ -234,16 +234,24 @@ struct MmArgs {
     int M, N, K;
     int tiles_m, tiles_n, groups_m;  // groups_m: 4-tile groups along M
     // two halves of K: the first K of the second half (a multiple of 64), the tile groups of
-    // one half, the pairs' sums ([tile][32][512 threads] float4) and counters
-    int kc, groups, set;
+    // one half, the pairs' sums ([tile][32][512 threads] float4) and, per tile, the blocks that
+    // have finished their half (modulo 2) and the halves written and not yet fetched, both of
+    // which end each launch as they began it, at zero
+    int kc, groups;
     float *ws;
+    unsigned *finished, *written;
 };
 
-// Per scratch buffer and tile of the split 256 x 256 kernel: the blocks that have finished
-// their half (modulo 2), and the halves written and not yet fetched.  Both end each launch
-// as they began it, at zero.
-constexpr int kPairTiles = 384;
-static __device__ unsigned mm_finished[2][kPairTiles], mm_written[2][kPairTiles];   // [the default stream, others]
+// The counters of a scratch buffer, in the buffer itself ahead of the sums that they count (a
+// graph that keeps a buffer's address keeps its counters too, whatever buffer later calls
+// use): zero from the buffer's allocation on, and again after each launch.
+constexpr int kPairTiles = 384;       // tiles of a launch of the split 256 x 256 kernel, at most
+constexpr int kRwMaxTiles = 16384;    // tiles of a split launch of the rows kernel, at most
+struct ScratchCounters {
+    unsigned arrived[kRwMaxTiles];    // the rows kernel's blocks of a tile
+    unsigned finished[kPairTiles], written[kPairTiles];
+};
+static_assert(sizeof(ScratchCounters) % 256 == 0, "the sums behind the counters keep their alignment");
 
 template <int DT>
 __device__ __forceinline__ mm_f32x16 mm_mfma(const mm_i16x4 (&a)[2], const uint4 &b, mm_f32x16 acc) {
@@ -433,7 +441,7 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
         const int slot = tm * p.tiles_n + tn;
         const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(
             (void *)(p.ws + (int64_t)slot * (BM * BN)), (short)0, BM * BN * 4, BUF_WORD3);
-        if (tid == 0) second = (int)atomicInc(&mm_finished[p.set][slot], 1u);
+        if (tid == 0) second = (int)atomicInc(p.finished + slot, 1u);
         __syncthreads();
         if (!__builtin_amdgcn_readfirstlane(second)) {
 #pragma unroll
@@ -444,13 +452,13 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
             }
             __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's sums are at the coherence point
             __syncthreads();
-            if (tid == 0) atomicAdd(&mm_written[p.set][slot], 1u);
+            if (tid == 0) atomicAdd(p.written + slot, 1u);
             return;
         }
         if (tid == 0) {
             for (;;) {
-                const unsigned n = __hip_atomic_load(&mm_written[p.set][slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (n && atomicCAS(&mm_written[p.set][slot], n, n - 1) == n) break;
+                const unsigned n = __hip_atomic_load(p.written + slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (n && atomicCAS(p.written + slot, n, n - 1) == n) break;
                 __builtin_amdgcn_s_sleep(2);
             }
         }
@@ -575,7 +583,8 @@ static int launch_mfma_pair(void *out, const void *left, const void *right, int6
     if (lease.status()) return 1;
     p.kc = (int)((K + 127) / 128 * 64);
     p.ws = static_cast<float *>(lease.ptr());
-    p.set = lease.set() & 1;
+    p.finished = lease.counters()->finished;
+    p.written = lease.counters()->written;
     matmul_mfma_kernel<DT, 4, 4, 64, 2, true><<<(unsigned)((2 * p.groups + 7) / 8 * 8 * 32), 512, 0, s>>>(p);
     return lease.finish();
 }
@@ -860,12 +869,6 @@ __global__ __launch_bounds__(512) void matmul16_small_kernel(uint16_t *__restric
 // block counts itself in.
 typedef float rw_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kRwCols = 128, kRwDepth = 32, kRwWaves = 4, kRwRows = 16, kRwPad = kRwCols + 4;
-constexpr int kRwMaxTiles = 16384;   // column tiles of a split launch, at most
-// per device: the column tiles' arrival counters, zero between launches (the last block's
-// atomicInc wraps to zero): a set beside each of the four growable scratch buffers and one
-// beside the no-alloc entry point's array, each used by one launch at a time like the
-// scratch it stands by
-static __device__ unsigned rw_arrived[5][kRwMaxTiles];
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p) {   // 16 bytes at any element
     uint4 v;
@@ -899,7 +902,8 @@ struct RwArgs {
     uint16_t *out;
     const uint16_t *a, *b;
     float *ws;       // [tile, row tile][chunk][rows][128] sums when split
-    int M, tiles, chunks, mtiles, set;
+    unsigned *arrived;   // [tile, row tile] blocks counted in (the last one's atomicInc wraps to zero)
+    int M, tiles, chunks, mtiles;
     int64_t K, N, kc;   // kc: K per chunk, a multiple of kRwWaves * kRwDepth
 };
 
@@ -1018,7 +1022,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 4 : 2) void matmul_rows_kernel(RwArg
     if (p.chunks == 1) return;
     __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): this wave's sums are at the coherence point
     __syncthreads();
-    if (tid == 0) is_last = atomicInc(&rw_arrived[p.set][slot], (unsigned)p.chunks - 1) == (unsigned)p.chunks - 1;
+    if (tid == 0) is_last = atomicInc(p.arrived + slot, (unsigned)p.chunks - 1) == (unsigned)p.chunks - 1;
     __syncthreads();
     if (!is_last) return;
     for (int o = tid; o < total; o += 256) {
@@ -1227,11 +1231,12 @@ __global__ __launch_bounds__(256) void matmul_splitk_reduce_kernel(uint16_t *c, 
 // freed: a later growth retires it (kept until the process ends) and allocates
 // the new one beside it.  Replays of such a graph share the buffer with eager
 // calls until that growth; the caller orders them (one stream, or its own
-// events), as it orders any two uses of one buffer.
+// events), as it orders any two uses of one buffer.  After it they share nothing: the
+// buffer's counters (ScratchCounters) stand at its start.
 struct SplitScratch {
     std::mutex mu;
-    void *ptr = nullptr;
-    size_t bytes = 0;
+    void *ptr = nullptr;        // the allocation: the counters, then the sums
+    size_t bytes = 0;           // of the sums
     hipEvent_t done = nullptr;  // recorded after the last call that used ptr
     hipStream_t last = nullptr;
     bool used = false;
@@ -1269,10 +1274,18 @@ static int scratch_acquire(SplitScratch &sc, size_t need, hipStream_t s) {
             sc.bytes = 0;
         }
         const size_t grown = (need + ((size_t)1 << 20) - 1) & ~(((size_t)1 << 20) - 1);
-        if (hipMallocAsync(&sc.ptr, grown, s) != hipSuccess) {
+        if (hipMallocAsync(&sc.ptr, sizeof(ScratchCounters) + grown, s) != hipSuccess) {
             (void)hipGetLastError();   // (a caller that runs without scratch must not find it)
             sc.ptr = nullptr;
             return fail(PUTER_ERR_UNAVAILABLE, "matmul: split-K scratch of %zu bytes unavailable", grown);
+        }
+        constexpr int64_t halves = sizeof(ScratchCounters) / sizeof(uint16_t);
+        matmul_zero_kernel<<<generic_blocks(halves), 256, 0, s>>>(static_cast<uint16_t *>(sc.ptr), halves);
+        const int rc = check_launch("scratch counters");
+        if (rc) {
+            (void)hipFreeAsync(sc.ptr, s);
+            sc.ptr = nullptr;
+            return rc;
         }
         sc.bytes = grown;
     }
@@ -1306,17 +1319,17 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s, bool eager_only) : s_(s)
         status_ = fail(PUTER_ERR_INVALID, "scratch: not held for this call under stream capture");
         return;
     }
-    set_ = (s ? 1 : 0) + (eager_only ? 2 : 0);
-    sc_ = &g_split_scratch[dev][set_];
+    const int set = (s ? 1 : 0) + (eager_only ? 2 : 0);
+    ordered_ = !s;
+    sc_ = &g_split_scratch[dev][set];
     lock_ = std::unique_lock<std::mutex>(sc_->mu);
     if (capturing) {
         if (sc_->bytes < bytes) {   // the other buffer, if it is large enough
-            SplitScratch &other = g_split_scratch[dev][1 - set_];
+            SplitScratch &other = g_split_scratch[dev][1 - set];
             lock_.unlock();
             lock_ = std::unique_lock<std::mutex>(other.mu);
             if (other.bytes >= bytes) {
                 sc_ = &other;
-                set_ = 1 - set_;
             } else {
                 lock_ = std::unique_lock<std::mutex>(sc_->mu);
             }
@@ -1331,16 +1344,18 @@ ScratchLease::ScratchLease(size_t bytes, hipStream_t s, bool eager_only) : s_(s)
         }
         sc_->pinned = true;
         captured_ = true;
-        ptr_ = sc_->ptr;
+        counters_ = static_cast<ScratchCounters *>(sc_->ptr);
         return;
     }
     status_ = scratch_acquire(*sc_, bytes, s);
-    if (status_ == PUTER_OK) ptr_ = sc_->ptr;
+    if (status_ == PUTER_OK) counters_ = static_cast<ScratchCounters *>(sc_->ptr);
 }
+
+void *ScratchLease::ptr() const { return counters_ ? counters_ + 1 : nullptr; }
 
 int ScratchLease::finish() {
     if (status_ != PUTER_OK) return status_;
-    if (captured_ || (set_ & 1) == 0) return PUTER_OK;   // the default stream orders its own calls
+    if (captured_ || ordered_) return PUTER_OK;   // the default stream orders its own calls
     if (hipEventRecord(sc_->done, s_) != hipSuccess) return fail(PUTER_ERR_LAUNCH, "scratch: cannot record the event");
     sc_->last = s_;
     sc_->used = true;
@@ -1351,22 +1366,22 @@ int ScratchLease::finish() {
 // ---- the allocation-free Matmul (puter_hip_matmul_noalloc) -----------------
 // Its split-K partials live in a file-scope device array (one copy per GPU,
 // held until the process ends) instead of the growable scratch.  The array
-// holds 16 MiB, the most any split-K launch here can need: at most 512 blocks
+// holds the counters and 16 MiB of sums, the most any split-K launch here can need: at most 512 blocks
 // (chunks x tiles) of 64 x 128 f32 partials for the 16-bit formats and for the
 // f32 VALU kernel's 64 x 64 tiles; the f32 MFMA kernel's chunk count is capped so
 // that its partials (chunks x rows x cols floats) fit it.  Host code never passes the array's name to a kernel (in host code it
 // is a stand-in, not a device address): it passes the address
 // hipGetSymbolAddress returns, looked up once per device on that device's first
 // call.  Every no-alloc call on a GPU shares that GPU's array, so such calls
-// must not overlap on one GPU; each call writes every partial it reads, so
-// nothing needs clearing between calls.
+// must not overlap on one GPU; each call writes every partial it reads and leaves
+// its counters at zero, so nothing needs clearing between calls.
 namespace noalloc {
 constexpr size_t kScratchBytes = (size_t)512 * 64 * 128 * sizeof(float);
-static __device__ __align__(256) float scratch[kScratchBytes / sizeof(float)];
+static __device__ __align__(256) char scratch[sizeof(ScratchCounters) + kScratchBytes];   // (zero when loaded)
 static std::mutex mu;
-static float *ptr[64];  // per device: scratch's device address
+static ScratchCounters *ptr[64];  // per device: scratch's device address
 
-static int address(float **out) {
+static int address(ScratchCounters **out) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
         return fail(PUTER_ERR_UNAVAILABLE, "matmul (no-alloc): no device");
@@ -1376,7 +1391,7 @@ static int address(float **out) {
         const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess || !p)
             return fail(PUTER_ERR_UNAVAILABLE, "matmul (no-alloc): scratch address: %s", hipGetErrorString(e));
-        ptr[dev] = static_cast<float *>(p);
+        ptr[dev] = static_cast<ScratchCounters *>(p);
     }
     *out = ptr[dev];
     return PUTER_OK;
@@ -1387,6 +1402,7 @@ static int address(float **out) {
 // else a lease of the library's growable scratch.
 struct PartialsTarget {
     float *fixed = nullptr;
+    ScratchCounters *counters = nullptr;   // of the no-alloc scratch
 };
 
 // Runs of K of the rows kernel: toward one block per CU (200 of 256 is near enough: 16 x
@@ -1436,7 +1452,7 @@ static int launch_rows_mt(void *out, const void *left, const void *right, int64_
     const int64_t per = (steps + chunks - 1) / chunks;
     chunks = (steps + per - 1) / per;
     RwArgs p{static_cast<uint16_t *>(out), static_cast<const uint16_t *>(left), static_cast<const uint16_t *>(right), tgt.fixed,
-             (int)M, (int)tiles, (int)chunks, (int)mtiles, 4, K, N, per * STEP};
+             tgt.counters ? tgt.counters->arrived : nullptr, (int)M, (int)tiles, (int)chunks, (int)mtiles, K, N, per * STEP};
     auto launch = [&] {
         const int64_t blocks = (tiles * p.chunks + 7) / 8 * 8 * mtiles;
         matmul_rows_kernel<DT, MT><<<(unsigned)blocks, 256, 0, s>>>(p);
@@ -1451,7 +1467,7 @@ static int launch_rows_mt(void *out, const void *left, const void *right, int64_
         return launch();
     }
     p.ws = static_cast<float *>(lease.ptr());
-    p.set = lease.set();
+    p.arrived = lease.counters()->arrived;
     const int rc = launch();
     const int fin = lease.finish();
     return rc ? rc : fin;
@@ -1767,8 +1783,9 @@ static int matmul_entry(void *out, const void *left, const void *right, int64_t 
     }
     PartialsTarget tgt;
     if (no_alloc) {
-        const int rc = noalloc::address(&tgt.fixed);
+        const int rc = noalloc::address(&tgt.counters);
         if (rc) return rc;
+        tgt.fixed = reinterpret_cast<float *>(tgt.counters + 1);
     }
     switch (dtype) {
     case PUTER_BF16: return launch_matmul16<PUTER_BF16>(out, left, right, rows, inner, cols, s, tgt);

@@ -354,3 +354,73 @@ def test_capture_that_would_grow_the_scratch_fails_before_launching(backend):
         ref = O.mha_rows(qh, kh, vh, h, d, (hd, hd + 1), (0, 1), kv_heads=kvh, dtype=O.BF16)
         assert_close(O.to_f32(got[hd], O.BF16), O.to_f32(ref.reshape(h, d)[hd], O.BF16), TOL[O.BF16],
                      elem_tol=None, what=f"head {hd}")
+
+
+def test_matmul_replays_beside_eager_calls_after_a_growth(backend):
+    """After the scratch has grown, the graph of a split Matmul keeps its old buffer, and its
+    replays need no order with eager calls, whose sums and arrival counters are in the new
+    one: replays on one stream and eager calls with other numbers of runs of K on another,
+    unordered, are exact (integer operands), and so are ordered calls afterwards."""
+    import torch
+
+    def operands(m, k, n, seed):
+        rng = np.random.default_rng(seed)
+        a, b = (rng.integers(-2, 3, s).astype(np.float32) for s in ((m, k), (k, n)))
+        return to_dev(O.from_f32(a, O.BF16)), to_dev(O.from_f32(b, O.BF16)), to_dev(O.from_f32(a @ b, O.BF16))
+
+    shapes = [(1, 4096, 1024), (1, 1024, 1024), (4, 2048, 4096), (16, 768, 2048)]   # 16, 8, 8 and 6 runs
+    data = [operands(*s, 1400 + i) for i, s in enumerate(shapes)]
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def calls(which, outs):
+        for i, o in zip(which, outs):
+            m, k, n = shapes[i]
+            backend.Matmul(o, data[i][0], data[i][1], m, k, n, O.BF16)
+
+    def outputs(which):
+        return [torch.zeros_like(data[i][2]) for i in which]
+
+    def exact(which, outs):
+        return all(torch.equal(o, data[i][2]) for i, o in zip(which, outs))
+
+    in_graph, eager = [0, 2] * 8, [1, 3] * 16
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        calls(range(4), outputs(range(4)))      # sizes the buffer of the streams but the default one
+    g_out = outputs(in_graph)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        calls(in_graph, g_out)
+
+    # more scratch than any buffer holds (a capture of the call is refused), then the growth
+    h, kvh, d, seq_k = 2040, 8, 256, 81920
+    cfg = puter_amd.MultiHeadAttentionConfig(h, d, True, 0, 0.0, kvh)
+    q, kv, o = (torch.zeros(n, dtype=torch.int16, device="cuda") for n in (h * d, seq_k * kvh * d, h * d))
+    refused = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(refused, stream=side):
+        o.zero_()
+        with pytest.raises(puter_amd.PuterError):
+            backend.MultiHeadAttentionBatched(cfg, q, kv, kv, o, 1, 1, seq_k, O.BF16)
+    with torch.cuda.stream(side):
+        backend.MultiHeadAttentionBatched(cfg, q, kv, kv, o, 1, 1, seq_k, O.BF16)
+    torch.cuda.synchronize()
+    del q, kv, o
+
+    for rep in range(20):
+        e_out = outputs(eager)
+        for t in g_out:
+            t.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            graph.replay()
+        with torch.cuda.stream(other):
+            calls(eager, e_out)
+        torch.cuda.synchronize()
+        assert exact(in_graph, g_out) and exact(eager, e_out), rep
+    last = outputs(range(4))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        calls(range(4), last)
+    torch.cuda.synchronize()
+    assert exact(range(4), last)
