@@ -268,6 +268,24 @@ __device__ __forceinline__ void unpack_vec(const uint4 &v, float (&f)[Vec<DT>::N
     }
 }
 
+// The same for values that are computed with: f16 widens in hardware (one instruction, exact;
+// a signalling NaN comes out quiet, as the arithmetic would make it).  The software widening
+// takes about ten instructions and twice the registers.  (The empty asm keeps the conversion
+// out of mixed-precision FMAs.)
+template <int DT>
+__device__ __forceinline__ void unpack_value(const uint4 &v, float (&f)[Vec<DT>::N]) {
+    if constexpr (DT == PUTER_F16) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f[i] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+            asm("" : "+v"(f[i]));
+        }
+    } else {
+        unpack_vec<DT>(v, f);
+    }
+}
+
 // Load/convert N contiguous elements (16 bytes) into floats.
 template <int DT>
 __device__ __forceinline__ void load_vec(const void *base, size_t vec_index, float (&f)[Vec<DT>::N]) {

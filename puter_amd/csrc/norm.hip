@@ -488,9 +488,9 @@ __global__ __launch_bounds__(1024) void norm_line_kernel(NormArgs a) {
 #pragma unroll
         for (int j = 0; j < V; ++j) {
             float x[N], b[N], g[N], o[N];
-            unpack_vec<DT>(hv[j], x);
-            unpack_vec<DT>(br[j], b);
-            unpack_vec<DT>(gt[j], g);
+            unpack_value<DT>(hv[j], x);
+            unpack_value<DT>(br[j], b);
+            unpack_value<DT>(gt[j], g);
 #pragma unroll
             for (int i = 0; i < N; ++i) o[i] = i < n[j] ? x[i] + g[i] * b[i] : 0.0f;
             hv[j] = pack_vec<DT>(o);
@@ -505,7 +505,7 @@ __global__ __launch_bounds__(1024) void norm_line_kernel(NormArgs a) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
         float h[N];
-        unpack_vec<DT>(hv[j], h);
+        unpack_value<DT>(hv[j], h);
 #pragma unroll
         for (int i = 0; i < N; ++i) {   // (zeros past the row)
             if constexpr (OP == OP_RMS || OP == OP_ADAPTIVE) s += h[i] * h[i];
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(1024) void norm_line_kernel(NormArgs a) {
 #pragma unroll
         for (int j = 0; j < V; ++j) {
             float h[N];
-            unpack_vec<DT>(hv[j], h);
+            unpack_value<DT>(hv[j], h);
 #pragma unroll
             for (int i = 0; i < N; ++i) {
                 const float d = i < n[j] ? h[i] - mean : 0.0f;
@@ -533,9 +533,9 @@ __global__ __launch_bounds__(1024) void norm_line_kernel(NormArgs a) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
         float h[N], g[N], b[N], o[N];
-        unpack_vec<DT>(hv[j], h);
-        unpack_vec<DT>(gv[j], g);
-        if constexpr (BIAS) unpack_vec<DT>(bv[j], b);
+        unpack_value<DT>(hv[j], h);
+        unpack_value<DT>(gv[j], g);
+        if constexpr (BIAS) unpack_value<DT>(bv[j], b);
 #pragma unroll
         for (int i = 0; i < N; ++i) o[i] = apply_one<DT, OP>(h[i], mean, inv, g[i], BIAS ? b[i] : 0.0f);
         line_store<DT, AL>(pack_vec<DT>(o), a.out, off + e[j], n[j]);
