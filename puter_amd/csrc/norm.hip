@@ -12,9 +12,9 @@
 // written once (for the fused op, 8 B/elem of HBM traffic in bf16):
 //   - norm_row_kernel: a block per row, 1-8 16-byte vectors per thread per
 //     tensor (long rows, many rows);
-//   - norm_wave_kernel (fused norms): one wave64 per row, 4 rows per 256-thread block, the
-//     row as VPL 16-byte vectors per lane (lane l owns vectors j*64 + l, so each
-//     wave-wide load is one contiguous 1 KiB burst); register-only butterflies;
+//   - norm_wave_kernel: one wave64 per row, 4 rows per 256-thread block, the row as
+//     VPL 16-byte vectors per lane (lane l owns vectors j*64 + l, so each wave-wide
+//     load is one contiguous 1 KiB burst); register-only butterflies;
 //   - norm_line_kernel: a block per row for few rows and for any other length and
 //     alignment.
 // Rows too long for a block's registers use the generic block-per-row kernel, which
@@ -101,7 +101,7 @@ __device__ __forceinline__ float apply_one(float h, float mean, float inv, float
 // SHARE (fused gated residual + RMSNorm/LayerNorm, the block's 4 rows in one
 // modulation batch): the gate row, gamma (and beta) are staged once per block
 // in LDS instead of being re-read from L2 by every wave.
-template <int DT, int OP, int VPL, bool SHARE>
+template <int DT, int OP, bool GR, int VPL, bool SHARE = false>
 __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
 #pragma clang fp contract(off)
     constexpr int N = Vec<DT>::N;
@@ -116,48 +116,54 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
     const int64_t batch = (live ? row : 0) / a.rows_per_batch;
 
     uint4 hv[VPL];
-    const uint4 *res = reinterpret_cast<const uint4 *>(a.x) + row_vec;
-    const uint4 *br = reinterpret_cast<const uint4 *>(a.branch) + row_vec;
-    const uint4 *gate = reinterpret_cast<const uint4 *>(a.mod) +
-                        (size_t)(batch * a.mod_cols + a.gate_off) / N;
-    uint4 rv[VPL], bv[VPL], gv[VPL];
+    if constexpr (GR) {
+        const uint4 *res = reinterpret_cast<const uint4 *>(a.x) + row_vec;
+        const uint4 *br = reinterpret_cast<const uint4 *>(a.branch) + row_vec;
+        const uint4 *gate = reinterpret_cast<const uint4 *>(a.mod) +
+                            (size_t)(batch * a.mod_cols + a.gate_off) / N;
+        uint4 rv[VPL], bv[VPL], gv[VPL];
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        rv[j] = ld_stream(res + j * 64 + lane);
-        bv[j] = ld_stream(br + j * 64 + lane);
-        if constexpr (!SHARE) gv[j] = gate[j * 64 + lane];
-    }
-    if constexpr (SHARE) {
-        // the row loads above are in flight while the block fills the table
-        const int64_t b0 = ((int64_t)blockIdx.x * 4) / a.rows_per_batch;
-        const uint4 *g0 = reinterpret_cast<const uint4 *>(a.mod) + (size_t)(b0 * a.mod_cols + a.gate_off) / N;
-        const uint4 *gm = reinterpret_cast<const uint4 *>(a.scale);
-        const uint4 *bt = reinterpret_cast<const uint4 *>(a.bias);
-        for (int i = threadIdx.x; i < ROWV; i += 256) {
-            tbl[i] = g0[i];
-            tbl[ROWV + i] = gm[i];
-            if constexpr (OP == OP_LN) tbl[2 * ROWV + i] = bt[i];
+        for (int j = 0; j < VPL; ++j) {
+            rv[j] = ld_stream(res + j * 64 + lane);
+            bv[j] = ld_stream(br + j * 64 + lane);
+            if constexpr (!SHARE) gv[j] = gate[j * 64 + lane];
         }
-        __syncthreads();
-        if (!live) return;
+        if constexpr (SHARE) {
+            // the row loads above are in flight while the block fills the table
+            const int64_t b0 = ((int64_t)blockIdx.x * 4) / a.rows_per_batch;
+            const uint4 *g0 = reinterpret_cast<const uint4 *>(a.mod) + (size_t)(b0 * a.mod_cols + a.gate_off) / N;
+            const uint4 *gm = reinterpret_cast<const uint4 *>(a.scale);
+            const uint4 *bt = reinterpret_cast<const uint4 *>(a.bias);
+            for (int i = threadIdx.x; i < ROWV; i += 256) {
+                tbl[i] = g0[i];
+                tbl[ROWV + i] = gm[i];
+                if constexpr (OP == OP_LN) tbl[2 * ROWV + i] = bt[i];
+            }
+            __syncthreads();
+            if (!live) return;
 #pragma unroll
-        for (int j = 0; j < VPL; ++j) gv[j] = tbl[j * 64 + lane];
-    }
-    uint4 *hid = reinterpret_cast<uint4 *>(a.hidden) + row_vec;
+            for (int j = 0; j < VPL; ++j) gv[j] = tbl[j * 64 + lane];
+        }
+        uint4 *hid = reinterpret_cast<uint4 *>(a.hidden) + row_vec;
 #pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-        float r[N], b[N], g[N], o[N];
-        unpack_vec<DT>(rv[j], r);
-        unpack_vec<DT>(bv[j], b);
-        unpack_vec<DT>(gv[j], g);
+        for (int j = 0; j < VPL; ++j) {
+            float r[N], b[N], g[N], o[N];
+            unpack_vec<DT>(rv[j], r);
+            unpack_vec<DT>(bv[j], b);
+            unpack_vec<DT>(gv[j], g);
 #pragma unroll
-        for (int i = 0; i < N; ++i) o[i] = r[i] + g[i] * b[i];
-        hv[j] = pack_vec<DT>(o);
-        st_stream(hv[j], hid + j * 64 + lane);
+            for (int i = 0; i < N; ++i) o[i] = r[i] + g[i] * b[i];
+            hv[j] = pack_vec<DT>(o);
+            st_stream(hv[j], hid + j * 64 + lane);
+        }
+    } else {
+        const uint4 *x = reinterpret_cast<const uint4 *>(a.x) + row_vec;
+#pragma unroll
+        for (int j = 0; j < VPL; ++j) hv[j] = ld_stream(x + j * 64 + lane);
     }
 
     float mean = 0.0f, inv;
-    if constexpr (OP == OP_RMS) {
+    if constexpr (OP == OP_RMS || OP == OP_ADAPTIVE) {
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPL; ++j) {
@@ -196,9 +202,14 @@ __global__ __launch_bounds__(256) void norm_wave_kernel(NormArgs a) {
     if constexpr (SHARE) {
         gp = tbl + ROWV;
         if constexpr (OP == OP_LN) bp = tbl + 2 * ROWV;
-    } else {
+    } else if constexpr (OP == OP_RMS || OP == OP_LN) {
         gp = reinterpret_cast<const uint4 *>(a.scale);
         if constexpr (OP == OP_LN) bp = reinterpret_cast<const uint4 *>(a.bias);
+    } else {
+        const uint4 *m = reinterpret_cast<const uint4 *>(a.mod) +
+                         (size_t)(batch * a.mod_cols + a.mod_off) / N;
+        if constexpr (OP == OP_ADAPTIVE) { gp = m; bp = m + H / N; }      // scale, shift
+        else { bp = m; gp = m + H / N; }                                  // shift, scale
     }
     uint4 *out = reinterpret_cast<uint4 *>(a.out) + row_vec;
 #pragma unroll
@@ -669,6 +680,28 @@ static bool launch_line(const NormArgs &a, hipStream_t s, bool vec_ok) {
     return true;
 }
 
+// Where a wave per row beats the any-row kernel, on rows of VPL = 2, 4, 8 or 16 vectors a lane.
+// Fused: 512 rows and more (1024 x 2048 RMSNorm bf16 5.1 us against 5.3, 1024 x 8192 12.6
+// against 13.3), and the shortest rows of any count, where one wave needs no barrier and a block
+// of four rows is fewer blocks to start (LayerNorm f32 16 x 512 2.7 against 2.9).  Unfused, the
+// shortest rows likewise (RMSNorm f32 4096 x 512 3.7 against 4.1, 1 x 512 2.0 against 2.1; not the
+// adaptive norm, nor bf16 beyond 512 rows), and tensors of about 40 to 100 MB in and out, past
+// the L2s: LayerNorm f32 2048 x 4096 10.6 against 16.1, bf16 2048 x 8192 11.7 against 15.4, 3000
+// x 4096 11.7 against 16, 6000 x 2048 10 against 13.6; below and above (the row kernel's range
+// from 4096 long rows on) the any-row kernel is level or faster.  Unfused f16 never: its wave per row
+// widens in software (2048 x 8192 RMSNorm 81 us against 15).
+template <int DT, int OP, bool GR>
+static bool wave_wins(int64_t rows, int64_t vpl) {
+    constexpr bool f32 = DT == PUTER_F32, modded = OP == OP_ADAPTIVE || OP == OP_MODULATED;
+    if (GR) return rows >= 512 || (vpl == 2 && DT != PUTER_F16);
+    switch (vpl) {
+    case 2: return (f32 ? OP != OP_ADAPTIVE : rows < 512 && !modded) || (rows >= 5000 && rows < 10000);
+    case 4: return !f32 && rows >= 4000 && rows < 10000;
+    case 8: return rows >= (f32 ? 2048 : 3000);
+    default: return rows >= (f32 && modded ? 1792 : 1536);
+    }
+}
+
 template <int DT, int OP, bool GR>
 static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
     constexpr int N = Vec<DT>::N;
@@ -682,10 +715,8 @@ static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
     // rows against V = 1), V = 8 for the two-reduction LayerNorm, whose barriers
     // cost less over fewer waves (4096 columns, 64 threads: 4667 -> 5638 / 5014 ->
     // 5999; 8192, 128 threads: 5352 -> 5659 / 5641 -> 5799 against 512 threads).
-    // The fused norms of 512 rows and more keep the wave per row on shorter rows
-    // (1024 x 2048 RMSNorm 5.1 us against 5.3 on the any-row kernel, 1024 x 8192 12.6
-    // against 13.3).  All others, few rows and every other length and alignment,
-    // take the any-row kernel (1 x 4096 RMSNorm 3.8 -> 2.7 us, 256 x 4096 4.9 -> 3.7,
+    // The wave per row serves what wave_wins says; all others, few rows and every other
+    // length and alignment, take the any-row kernel (1 x 4096 RMSNorm 3.8 -> 2.7 us, 256 x 4096 4.9 -> 3.7,
     // 1024 x 8192 LayerNorm 11.0 -> 8.8, all against the wave per row; ModulatedLayerNorm
     // 4608 x 3072 44.2 -> 14.1, GatedResidual+RMSNorm 16384 x 2560 152 -> 58, RMSNorm 2540 x
     // 6361 42.5 -> 19.7 against the generic kernel's three passes of single elements).
@@ -707,17 +738,18 @@ static int launch_norm(const NormArgs &a, hipStream_t s, bool vec_ok) {
             return check_launch("norm");
         }
     }
-    if constexpr (GR) {
-        if (vec_ok && a.H % (64 * N) == 0 && a.rows >= 512) {
-            const bool share = a.rows_per_batch % 4 == 0;   // a block's 4 rows share one gate row
+    if constexpr (GR || DT != PUTER_F16) {
+        const int64_t vpl = a.H / (64 * N);
+        if (vec_ok && a.H % (64 * N) == 0 && wave_wins<DT, OP, GR>(a.rows, vpl)) {
+            const bool share = GR && a.rows_per_batch % 4 == 0;   // a block's 4 rows share one gate row
             const unsigned blocks = (unsigned)((a.rows + 3) / 4);
             const size_t lds = share ? (size_t)a.H * sizeof(typename Elem<DT>::T) * (OP == OP_LN ? 3 : 2) : 0;
 #define PUTER_WAVE(VPL)                                                                           \
     case VPL:                                                                                     \
-        if (share) norm_wave_kernel<DT, OP, VPL, true><<<blocks, 256, lds, s>>>(a);               \
-        else norm_wave_kernel<DT, OP, VPL, false><<<blocks, 256, lds, s>>>(a);                    \
+        if (share) norm_wave_kernel<DT, OP, GR, VPL, GR><<<blocks, 256, lds, s>>>(a);             \
+        else norm_wave_kernel<DT, OP, GR, VPL, false><<<blocks, 256, lds, s>>>(a);                \
         return check_launch("norm");
-            switch (a.H / (64 * N)) {
+            switch (vpl) {
                 PUTER_WAVE(2)
                 PUTER_WAVE(4)
                 PUTER_WAVE(8)

@@ -270,3 +270,15 @@ def test_norms_any_row(backend, dt, rows, h, rpb, shift):
             backend.GatedResidualLayerNorm(hid[shift:], dbr, dm, dg, db, hid[shift:], out[shift:], rows, h, rpb, 6 * h, 0, dt)
         check(hid, hid_ref, "hidden " + kind)
         check(out, O.rmsnorm(hid_ref, g, eps, dt) if kind == "rms" else O.layernorm(hid_ref, g, b, dt), "fused " + kind)
+
+
+@pytest.mark.parametrize("dt", [O.F32, O.BF16, O.F16])
+@pytest.mark.parametrize("vectors,rows,rpb", [
+    (2, 6, 2), (2, 514, 257), (4, 516, 172), (8, 515, 103), (16, 520, 260), (16, 513, 27),
+    (4, 5001, 1667), (8, 3002, 1501), (16, 1793, 163),   # from about 40 MB on the unfused norms too
+])
+def test_norms_wave_per_row(backend, dt, vectors, rows, rpb):
+    """Rows of 64 lanes x 2, 4, 8 or 16 vectors, which a wave each serves: batches of a
+    multiple of four rows (the fused norms' shared tables) and not, a last block of fewer
+    than four rows, in place and between guard elements."""
+    test_norms_any_row(backend, dt, rows, vectors * (256 if dt == O.F32 else 512), rpb, 0)

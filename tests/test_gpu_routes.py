@@ -1,0 +1,54 @@
+"""GPU: which kernels a call launches, where the choice between two of them rests on which
+is faster for its sizes.  The names come from torch's profiler, which sees every launch of
+the process."""
+import pytest
+
+import oracle as O
+import puter_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def launched(call):
+    """The names of the kernels that call launches."""
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    return [e.name for e in p.events() if "puter::" in e.name or "_kernel" in e.name]
+
+
+def zeros(dt, *shape):
+    import torch
+    t = {O.F32: torch.float32, O.BF16: torch.bfloat16, O.F16: torch.float16}[dt]
+    return torch.zeros(shape, dtype=t, device="cuda")
+
+
+@pytest.mark.parametrize("op,dt,rows,h,kernel", [
+    # short rows: a wave each, four to a block
+    ("rms", O.F32, 4096, 512, "norm_wave"), ("ln", O.F32, 1, 512, "norm_wave"), ("rms", O.BF16, 16, 1024, "norm_wave"),
+    ("gr_ln", O.F32, 16, 512, "norm_wave"), ("adaptive", O.F32, 16, 512, "norm_line"),
+    # tensors past the L2s
+    ("ln", O.F32, 2048, 4096, "norm_wave"), ("rms", O.BF16, 2048, 8192, "norm_wave"),
+    ("rms", O.BF16, 3500, 4096, "norm_wave"), ("adaptive", O.BF16, 6000, 2048, "norm_wave"),
+    # few rows, other lengths, and f16
+    ("rms", O.BF16, 1, 4096, "norm_line"), ("ln", O.BF16, 1024, 8192, "norm_line"),
+    ("ln", O.BF16, 4096, 3072, "norm_line"), ("rms", O.F16, 2048, 8192, "norm_line"),
+    ("gr_rms", O.F16, 16, 1024, "norm_line"), ("gr_rms", O.F16, 1024, 2048, "norm_wave"),
+    ("rms", O.BF16, 16384, 4096, "norm_row"),
+])
+def test_norm_kernels(backend, op, dt, rows, h, kernel):
+    x, y, z, g, mod = zeros(dt, rows, h), zeros(dt, rows, h), zeros(dt, rows, h), zeros(dt, h), zeros(dt, 1, 3 * h)
+    cfg = puter_amd.RMSNormConfig(1e-5)
+    names = launched({
+        "rms": lambda: backend.RMSNorm(cfg, x, g, y, rows, h, dt),
+        "ln": lambda: backend.LayerNorm(x, g, g, y, rows, h, dt),
+        "adaptive": lambda: backend.AdaptiveRMSNorm(cfg, x, mod, y, rows, h, rows, 3 * h, dt),
+        "gr_rms": lambda: backend.GatedResidualRMSNorm(cfg, x, x, mod, g, y, z, rows, h, rows, 3 * h, 0, dt),
+        "gr_ln": lambda: backend.GatedResidualLayerNorm(x, x, mod, g, g, y, z, rows, h, rows, 3 * h, 0, dt),
+    }[op])
+    names = [n for n in names if "puter::" in n]
+    assert len(names) == 1 and kernel in names[0], names
+
