@@ -1568,15 +1568,34 @@ static bool mfma_pair_wins(int64_t M, int64_t K, int64_t N) {
     return large <= kPairTiles && K >= 2048 && 50 * r_pair + 120000 / K < std::min(100 * r_large, 55 * r_small + 11);
 }
 
+// Whether the generic kernel (a thread per output) beats the rows kernel on a shape or alignment
+// that only these two take: little K, whose steps of 0.065 us (f16, widened in software, 0.23)
+// stay below the rows kernel's start and its sums in LDS (2.8 us in row tiles of 16, 4.5 of
+// 32, 7.5 of 64), and few outputs.  bf16 65 x 5 x 33 2.1 us against 7.2, 20 x 15 x 129 3.2
+// against 4.7, 7 x 15 x 33 2.7 against 3.1, 1000 x 5 x 4097 11.5 against 14.8; beyond, 1000 x 9 x
+// 4097 15.4 against 13.5, 7 x 23 x 33 3.3 against 3.1, 200 x 65 x 33 level.
+template <int DT>
+static bool generic_wins(int64_t M, int64_t K, int64_t N) {
+    const int rows = M <= 16 ? 0 : M <= 32 ? 1 : 2;
+    constexpr int64_t depth[2][3] = {{17, 33, 56}, {5, 11, 20}};
+    constexpr int64_t work[2][3] = {{6000000, 6000000, 21000000}, {5000000, 5000000, 5000000}};
+    constexpr int f16 = DT == PUTER_F16;
+    return (K <= depth[f16][rows] && M * N * K <= work[f16][rows]) || (!f16 && K <= 3);
+}
+
 template <int DT>
 static int launch_matmul16(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N,
                            hipStream_t s, PartialsTarget tgt) {
     // A few rows (a decode step's projections) take the rows kernel: against the skinny
     // kernel and its reduce launch 1 x 4096 x 4096 14.1 -> 9.5 us, 1 x 4096 x 14336 25.2 ->
     // 22.7, 16 x 14336 x 4096 35.0 -> 24.0, 32 x 4096 x 4096 15.4 -> 13.6; at 64 rows the
-    // skinny kernel wins (64 x 4096 x 14336: 33.1 against 35.3)
+    // skinny kernel wins (64 x 4096 x 14336: 33.1 against 35.3), and where it runs unsplit, with
+    // no second launch: a K of one slice (32 x 64 x 1024 2.9 us against 4.1) and, up to 2048 deep,
+    // columns for a round of blocks (32 x 1024 x 131072 42 against 52); of those up to 16 rows of
+    // little K over more columns yet are the rows kernel's (1 x 64 x 131072 3.6 against 4.7)
     const bool fits = N % 8 == 0 && K % 8 == 0 && aligned16(out) && aligned16(left) && aligned16(right);
-    if (!fits || M <= 32) {
+    const bool skinny = fits && K <= 2048 && skinny_chunks(M, K, N, 0) == 1 && !(M <= 16 && K <= 192 && N > 65536);
+    if (fits ? M <= 32 && !skinny : !generic_wins<DT>(M, K, N)) {
         const int rc = launch_rows<DT>(out, left, right, M, K, N, s, tgt, !fits);
         if (rc != 1) return rc;
     }

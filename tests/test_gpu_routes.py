@@ -52,3 +52,21 @@ def test_norm_kernels(backend, op, dt, rows, h, kernel):
     names = [n for n in names if "puter::" in n]
     assert len(names) == 1 and kernel in names[0], names
 
+
+@pytest.mark.parametrize("dt,rows,inner,cols,kernels", [
+    (O.BF16, 1, 4096, 4096, ["matmul_rows"]), (O.BF16, 32, 4096, 4096, ["matmul_rows"]),
+    # one slice of K, or a round of column tiles: the skinny kernel unsplit
+    (O.BF16, 32, 64, 1024, ["matmul_skinny"]), (O.F16, 4, 32, 4096, ["matmul_skinny"]),
+    (O.BF16, 32, 1024, 65536, ["matmul_skinny"]), (O.BF16, 8, 64, 131072, ["matmul_rows"]),
+    (O.BF16, 64, 4096, 4096, ["matmul_skinny", "matmul_splitk_reduce"]),
+    # unaligned: the generic kernel where K is small
+    (O.BF16, 65, 5, 33, ["matmul_generic"]), (O.BF16, 20, 15, 129, ["matmul_generic"]),
+    (O.F16, 4, 5, 33, ["matmul_generic"]), (O.BF16, 200, 31, 129, ["matmul_generic"]),
+    (O.BF16, 7, 31, 33, ["matmul_rows"]), (O.F16, 200, 31, 129, ["matmul_rows"]),
+    (O.BF16, 1000, 31, 4097, ["matmul_rows"]), (O.BF16, 33, 4096, 32001, ["matmul_rows"]),
+])
+def test_matmul_kernels(backend, dt, rows, inner, cols, kernels):
+    a, b, c = zeros(dt, rows, inner), zeros(dt, inner, cols), zeros(dt, rows, cols)
+    backend.Matmul(c, a, b, rows, inner, cols, dt)   # (the scratch is there)
+    names = launched(lambda: backend.Matmul(c, a, b, rows, inner, cols, dt))
+    assert len(names) == len(kernels) and all(k in n for k, n in zip(kernels, names)), names
