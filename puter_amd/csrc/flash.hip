@@ -360,11 +360,17 @@ __global__ __launch_bounds__(512) void flash_product_kernel(FlashArgs a, const f
 constexpr int64_t kFlashScores = (int64_t)64 << 20;   // bytes of scores held at once
 constexpr int64_t kFlashMaxKeys = 16384;              // a row's keys in one block's registers
 
-// Returns false when the general kernel is to run: few keys, rows past a block, a
-// stream capture (graphs of these calls may replay side by side), or no room.
+// The most keys that a row sees.
+static int64_t flash_visible(const FlashArgs &a) { return a.causal ? std::min(a.seq_k, a.seq_q) : a.seq_k; }
+
+// Returns false when the general kernel is to run: few keys (a step of its key loop is 0.55 us
+// at 64 dims, three launches about 10: causal 4 x 1000 x 64 f32 4.9 us against 11.8, 16 x 1000
+// level, 24 x 1000 15.8 against 12.5; in bf16, whose large heads cost the scores more, level at
+// 30 keys), rows past a block, a stream capture (graphs of these calls may replay side by
+// side), or no room.
 template <int DT>
 static bool run_flash_passes(const FlashArgs &a, hipStream_t s, int *status) {
-    if (a.seq_k < 64 || a.seq_k > kFlashMaxKeys) return false;
+    if (a.seq_k < 64 || a.seq_k > kFlashMaxKeys || flash_visible(a) < (DT == PUTER_BF16 ? 30 : 18)) return false;
     const int64_t ld = (a.seq_k + 3) / 4 * 4;
     const int64_t chunk = std::min<int64_t>(a.seq_q, std::max<int64_t>(32, kFlashScores / (ld * 4) / 32 * 32));
     const size_t need = (size_t)(chunk * ld) * sizeof(float);
@@ -408,13 +414,16 @@ static int run_flash(const puter_flash_config *config, const void *q, const void
     if (seq_q > 0x7FFFFFFF) return fail(PUTER_ERR_INVALID, "flash attention: grid too large");
     if (!q || !k || !v || !o) return fail(PUTER_ERR_NIL, "flash attention: nil buffer");
     const float scale = (float)(1.0 / sqrt((double)depth));
-    if ((dtype == PUTER_BF16 || dtype == PUTER_F16) && value_dim == depth) {
+    FlashArgs a{q, k, v, o, seq_q, seq_k, depth, value_dim, config->causal ? 1 : 0, scale};
+    // (bf16 head sizes other than 64 and 128 over one to three keys: a padded tile costs more
+    // than the general kernel's few steps, 2 x 1 x 40 3.2 us against 3.8, 2 x 3 x 256 8.5 against 8.7)
+    const bool few = dtype == PUTER_BF16 && depth != 64 && depth != 128 && flash_visible(a) <= (depth > 128 ? 3 : 2);
+    if ((dtype == PUTER_BF16 || dtype == PUTER_F16) && value_dim == depth && !few) {
         MhaArgs m{q, k, v, o, 1, seq_q, seq_k, 1, 1, depth, config->causal ? 1 : 0, 0, 0.0f, scale, 0};
         m.nan_rows = 1;
         int status = PUTER_OK;
         if (launch_prefill_mfma(m, dtype, s, &status)) return status;
     }
-    FlashArgs a{q, k, v, o, seq_q, seq_k, depth, value_dim, config->causal ? 1 : 0, scale};
     const size_t lds = sizeof(float) * (size_t)depth;
     {
         int status = PUTER_OK;

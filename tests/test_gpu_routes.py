@@ -70,3 +70,18 @@ def test_matmul_kernels(backend, dt, rows, inner, cols, kernels):
     backend.Matmul(c, a, b, rows, inner, cols, dt)   # (the scratch is there)
     names = launched(lambda: backend.Matmul(c, a, b, rows, inner, cols, dt))
     assert len(names) == len(kernels) and all(k in n for k, n in zip(kernels, names)), names
+
+
+@pytest.mark.parametrize("dt,seq_q,seq_k,dim,causal,kernel", [
+    # rows that see a few keys: the general kernel
+    (O.F32, 4, 1000, 64, True, "flash_generic"), (O.BF16, 1, 1000, 40, True, "flash_generic"),
+    (O.BF16, 20, 1000, 512, True, "flash_generic"), (O.BF16, 1000, 1, 40, False, "flash_generic"),
+    (O.F32, 24, 1000, 64, True, "flash_score"), (O.F32, 1, 1000, 64, False, "flash_score"),
+    (O.BF16, 40, 1000, 512, True, "flash_score"), (O.BF16, 4, 1000, 40, True, "prefill_kernel"),
+    (O.F16, 4, 1, 256, False, "prefill_kernel"),
+])
+def test_flash_kernels(backend, dt, seq_q, seq_k, dim, causal, kernel):
+    q, k, out = zeros(dt, seq_q, dim), zeros(dt, seq_k, dim), zeros(dt, seq_q, dim)
+    cfg = puter_amd.FlashAttentionConfig(64, causal)
+    names = launched(lambda: backend.FlashAttention(cfg, q, k, k, out, seq_q, seq_k, dim, dim, dt))
+    assert kernel in names[0], names
