@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void rope_reg_kernel(RopeArgs a) {
             const int voff = info[k] & 1023, tix = (info[k] >> 10) & 2047;
             if constexpr (MODE == 0) {
                 float f[N], o[N];
-                unpack_vec<DT>(lo[k], f);
+                unpack_value<DT>(lo[k], f);
 #pragma unroll
                 for (int i = 0; i < N / 2; ++i) {
                     const float2 c = c0[tix + i];
@@ -186,8 +186,8 @@ __global__ __launch_bounds__(256) void rope_reg_kernel(RopeArgs a) {
                 st_stream(pack_vec<DT>(o), gb + voff);
             } else {
                 float e[N], od[N], oe[N], oo[N];
-                unpack_vec<DT>(lo[k], e);
-                unpack_vec<DT>(hi[k], od);
+                unpack_value<DT>(lo[k], e);
+                unpack_value<DT>(hi[k], od);
 #pragma unroll
                 for (int i = 0; i < N; ++i) {
                     const float2 c = c0[tix + i];
@@ -450,6 +450,11 @@ static bool launch_rope_reg(RopeArgs a, hipStream_t s) {
         // as many positions per group as fill the registers, bounded by the table
         int64_t ppb = (256 * kRopeVpt) / slab_vec;
         if (ppb * half > kRopeGroupLds) ppb = kRopeGroupLds / half;
+        // (few heads: a group holds many positions, whose float64 sincos a block's threads take
+        // in turn; while blocks are few they are spread to one a thread: bf16 221 tokens x 1 head
+        // x 64 7.6 -> 4.7 us, 4.4 with a thread per pair)
+        if (AXES)
+            while (ppb > 1 && ppb * half > 256 && (a.seq + ppb - 1) / ppb < kRopeMaxBlocks / 2) ppb = (ppb + 1) / 2;
         if (ppb < 1) ppb = 1;
         a.ppb = (int)ppb;
         const int64_t groups = (a.seq + ppb - 1) / ppb;
