@@ -1093,30 +1093,33 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(Prefi
 // lanes over the head dims; the splits are folded in order with weights
 // exp2(m_s - M) (m in the scaled log2 domain), O = sum w_s O_s / sum w_s l_s; a row
 // with no visible key (every m = -inf) is 0, as in the unsplit kernel.
+template <int D, bool PAD>
 __global__ __launch_bounds__(256) void prefill_f32_combine_kernel(PrefillArgs a, int splits, int64_t rows) {
+    constexpr int J = (D + 63) / 64;
+    const int dim = PAD ? a.dim : D;
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int lane = threadIdx.x & 63;
     float M = -INFINITY;
     for (int s = 0; s < splits; ++s) M = fmaxf(M, a.part_ml[s * rows + row].x);
-    float acc[4] = {}, lsum = 0.0f;   // dims lane, lane + 64, ..
+    float acc[J] = {}, lsum = 0.0f;   // dims lane, lane + 64, ..
     if (M != -INFINITY) {
         for (int s = 0; s < splits; ++s) {
             const float2 ml = a.part_ml[s * rows + row];
             const float w = ml.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml.x - M);
             lsum += w * ml.y;
-            const float *po = a.part_o + (s * rows + row) * a.dim;
+            const float *po = a.part_o + (s * rows + row) * dim;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (64 * j + lane < a.dim) acc[j] += w * po[64 * j + lane];
+            for (int j = 0; j < J; ++j)   // (past a padded row's end: its last dim, not stored)
+                acc[j] += w * po[PAD ? min(64 * j + lane, dim - 1) : 64 * j + lane];
         }
     }
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
     // row = (batch, query, head): the output row of the same index, dim floats
-    float *out = reinterpret_cast<float *>(a.o) + row * a.dim;
+    float *out = reinterpret_cast<float *>(a.o) + row * dim;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (64 * j + lane < a.dim) out[64 * j + lane] = acc[j] * inv;
+    for (int j = 0; j < J; ++j)
+        if (!PAD || 64 * j + lane < dim) out[64 * j + lane] = acc[j] * inv;
 }
 
 // The head dim D of the kernel that serves a head dim: the least that holds it.  A dim of
@@ -1234,7 +1237,9 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
             const dim3 grid((unsigned)blocks, (unsigned)splits);
             const unsigned cblocks = (unsigned)((rows + 3) / 4);
             launch(grid);
-            prefill_f32_combine_kernel<<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
+            with_head_dim(m.dim, [&](auto d) {
+                prefill_f32_combine_kernel<d.D, d.PAD><<<cblocks, 256, 0, s>>>(a, (int)splits, rows);
+            });
             const int rc = check_launch("prefill f32 mfma split");
             const int fin = lease.finish();
             *status = rc ? rc : fin;

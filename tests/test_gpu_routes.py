@@ -85,3 +85,18 @@ def test_flash_kernels(backend, dt, seq_q, seq_k, dim, causal, kernel):
     cfg = puter_amd.FlashAttentionConfig(64, causal)
     names = launched(lambda: backend.FlashAttention(cfg, q, k, k, out, seq_q, seq_k, dim, dim, dt))
     assert kernel in names[0], names
+
+
+def mha(backend, dt, seq_q, seq_k, heads, dim, kv_heads=None):
+    q, kv, out = zeros(dt, seq_q, heads * dim), zeros(dt, seq_k, (kv_heads or heads) * dim), zeros(dt, seq_q, heads * dim)
+    cfg = puter_amd.MultiHeadAttentionConfig(heads, dim, True, 0, 0.0, kv_heads or heads)
+    call = lambda: backend.MultiHeadAttention(cfg, q, kv, kv, out, seq_q, seq_k, dt)  # noqa: E731
+    call()
+    return launched(call)
+
+
+def test_split_f32_attention_combines_by_head_dim(backend):
+    """The sums of a split are folded by a kernel of the head dim's own, whose loads the
+    compiler can issue ahead of each other."""
+    names = mha(backend, O.F32, 16, 3000, 8, 128)
+    assert len(names) == 2 and "prefill_f32_combine_kernel<128" in names[1], names
