@@ -1144,6 +1144,37 @@ template <typename F> static void with_head_dim(int64_t dim, F f) {
     else f(PfHeadDim<256, true>{});
 }
 
+// The general kernel or the padded one?  Estimates in us, fitted to 2900 bf16 and 1200 f32
+// shapes (1 to 32 heads, 2 to 300 queries over 40 to 3000 keys, dims 16 to 256; 6% off for the padded
+// kernels, 15% for the general one).  The general kernel has a block per query row and
+// head: a row's keys in steps, 1.7 times slower where the heads that an XCD's rows see overflow
+// its L2, or, once rows fill the chip, all rows' keys at a rate.  f16 needs no such rule: its
+// general kernel widens in software and never wins.
+static double general_us(const MhaArgs &m, bool f32) {
+    const double rows = (double)m.batch * m.seq_q * m.heads, dim = (double)m.dim;
+    double most = (double)m.seq_k, mean = most;   // keys that a row sees
+    if (m.causal) mean = (double)m.shift + 0.5 * (double)(m.seq_q + 1);
+    if (m.window > 0) most = std::min(most, (double)m.window);
+    mean = std::min(std::max(mean, 1.0), most);
+    const double heads = std::max(1.0, std::min((double)m.batch * m.kv_heads, rows / 8));
+    const bool overflows = heads * (double)m.seq_k * dim * (f32 ? 8 : 4) > 4.2e6;
+    const double steps = most * (f32 ? 0.0078 + 0.000162 * dim : 0.0082 + 0.000145 * dim) * (overflows ? 1.7 : 1.0);
+    return (f32 ? 3.9 : 3.7) + std::hypot(steps, rows * mean * (f32 ? 1.3e-5 + 6.6e-7 * dim : 1.8e-5 + 4.4e-7 * dim));
+}
+// The padded kernels: the key tiles of the longest block, in rounds of blocks.
+static double padded_us(const MhaArgs &m, int64_t blocks, int64_t tiles, int64_t splits, bool f32) {
+    const int i = m.dim <= 64 ? 0 : m.dim <= 96 ? 1 : m.dim <= 128 ? 2 : 3;
+    constexpr double base[2][4] = {{3.5, 4.2, 4.6, 6.7}, {3.7, 4.5, 6.2, 8.0}};
+    constexpr double tile[2][4] = {{0.94, 1.14, 1.3, 2.9}, {2.5, 3.7, 6.3, 13.0}};
+    const int64_t room = (int64_t)device_cus() * (m.dim > 128 ? 1 : 2), rounds = (blocks * splits + room - 1) / room;
+    const double sums = splits > 1 ? 1.2 + 0.53 * (double)splits + 4.3e-6 * (double)(splits * m.batch * m.seq_q * m.heads * m.dim) : 0.0;
+    return base[f32][i] + tile[f32][i] * (double)(tiles * rounds) + sums;
+}
+static int64_t prefill_tiles(const MhaArgs &m, int64_t bn) {   // key tiles of the longest block
+    const int64_t keys = m.window > 0 ? std::min(m.seq_k, m.window + fa::BM + bn) : m.seq_k;
+    return (keys + bn - 1) / bn;
+}
+
 // f32 MultiHeadAttention on prefill_f32_kernel: head dims of 4 n up to 256, at least 16 query
 // rows, causal or not, with or without a sliding window and ALiBi.
 static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
@@ -1198,10 +1229,10 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     // (43 unsplit), 640 x 4 x 64 47.5 against 22.1.  From 24 blocks this kernel wins
     // unsplit too (384 x 8 x 64: 32.9 against 36.0, 4 x 128 x 8 x 64: 15.0 against 24.5)
     if (blocks < 24 && (!a.causal || ktiles < 8 || capturing)) return false;
-    // other head dims than 64 and 128: from 2048 rows (batch x queries x heads) on, where the
-    // general kernel's one block per row needs more than one round (2 x 21 x 12 rows over
-    // 173 keys of 96: 10.6 there against 24.9 here; 2 x 60 x 8 over 1500 keys of 256: 218
-    // against 107, 2 x 200 x 16 over 200 keys of 40: 75 against 21)
+    // other head dims than 64 and 128: from 2048 rows (batch x queries x heads) or 512 keys on
+    // (2 x 21 x 12 rows over 173 keys of 96: 10.6 there against 24.9 here; 2 x 60 x 8 over 1500
+    // keys of 256: 218 against 107, 2 x 200 x 16 over 200 keys of 40: 75 against 21), and there
+    // by the estimates above (16 x 32 heads over 700 keys of 256: 77 there against 152)
     if (m.dim != 64 && m.dim != 128 && m.batch * m.seq_q * m.heads < 2048 && ktiles < 16) return false;
     // Small grids split each block's key range over blockIdx.y, partials in the
     // library's scratch: the longest block's key loop, the critical path, shrinks with
@@ -1218,6 +1249,9 @@ static bool launch_prefill_f32(const MhaArgs &m, hipStream_t s, int *status) {
     else if (!a.causal && blocks < cus)
         splits = std::max<int64_t>(1, std::min<int64_t>((2 * cus + blocks - 1) / blocks, ktiles / 16));
     if (capturing) splits = 1;
+    if (m.dim != 64 && m.dim != 128 &&
+        general_us(m, true) < padded_us(m, blocks, (prefill_tiles(m, 32) + splits - 1) / splits, splits, true))
+        return false;
     auto launch = [&](dim3 grid) {
         with_head_dim(m.dim, [&](auto d) {
             if (gen) prefill_f32_kernel<d.D, true, d.PAD><<<grid, 256, 0, s>>>(a);
@@ -1288,6 +1322,12 @@ bool launch_prefill_mfma(const MhaArgs &m, int dtype, hipStream_t s, int *status
     const int64_t blocks = (int64_t)a.qtiles * a.batch * a.heads;
     if (blocks > 0x7FFFFFFF) return false;
     const bool bf = dtype == PUTER_BF16, win = a.window > 0 || a.alibi_s != 0.0f;
+    // few rows of other head dims, by the estimates above (8 x 8 heads over 200 keys of 256: 11.9
+    // us on the general kernel against 18.4; one tile of keys is the padded kernel's up to 128
+    // dims).  FlashAttention has another general kernel, slower than the padded one.
+    if (bf && !m.nan_rows && m.dim != 64 && m.dim != 128 && (m.seq_k > 64 || m.dim > 128) &&
+        general_us(m, false) < padded_us(m, blocks, prefill_tiles(m, 64), 1, false))
+        return false;
     const dim3 grid((unsigned)blocks);
     with_head_dim(m.dim, [&](auto d) {
         if (win) {

@@ -100,3 +100,18 @@ def test_split_f32_attention_combines_by_head_dim(backend):
     compiler can issue ahead of each other."""
     names = mha(backend, O.F32, 16, 3000, 8, 128)
     assert len(names) == 2 and "prefill_f32_combine_kernel<128" in names[1], names
+
+
+@pytest.mark.parametrize("dt,seq_q,seq_k,heads,dim,kernel", [
+    # few rows of head dims other than 64 and 128: a block per row
+    (O.BF16, 8, 200, 8, 256, "mha_"), (O.BF16, 2, 700, 8, 256, "mha_"), (O.BF16, 16, 200, 8, 40, "mha_"),
+    (O.F32, 16, 700, 32, 256, "mha_"), (O.F32, 64, 200, 32, 160, "mha_"), (O.F32, 64, 512, 1, 16, "mha_"),
+    # many, or over many keys
+    (O.BF16, 300, 700, 8, 96, "prefill_kernel"), (O.BF16, 8, 3000, 8, 256, "prefill_kernel"),
+    (O.BF16, 8, 40, 8, 40, "prefill_kernel"), (O.F16, 8, 200, 8, 256, "prefill_kernel"),
+    (O.F32, 300, 700, 16, 96, "prefill_f32_kernel"), (O.F32, 16, 2000, 8, 40, "prefill_f32_kernel"),
+    (O.F32, 16, 3000, 8, 128, "prefill_f32_kernel"),
+])
+def test_attention_kernels(backend, dt, seq_q, seq_k, heads, dim, kernel):
+    names = mha(backend, dt, seq_q, seq_k, heads, dim)
+    assert kernel in names[0], names
