@@ -57,6 +57,10 @@ private:
 // of the buffers that a graph may use holds, which is all a lease can get (matmul.hip).
 bool scratch_capturing(hipStream_t s, size_t *held = nullptr);
 
+// The device array of the allocation-free Matmul on the current device (noalloc.hip).
+constexpr size_t kNoAllocBytes = ((size_t)96 << 20) + ((size_t)67 << 10);
+int noalloc_scratch(void **out);
+
 inline bool is_float_dtype(int dt) { return dt >= PUTER_F32 && dt <= PUTER_F8E5M2; }
 inline bool is_norm_dtype(int dt) { return dt == PUTER_F32 || dt == PUTER_F16 || dt == PUTER_BF16; }
 inline int dtype_bytes(int dt) {

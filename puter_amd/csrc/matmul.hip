@@ -246,6 +246,7 @@ struct MmArgs {
 // graph that keeps a buffer's address keeps its counters too, whatever buffer later calls
 // use): zero from the buffer's allocation on, and again after each launch.
 constexpr int kPairTiles = 384;       // tiles of a launch of the split 256 x 256 kernel, at most
+constexpr size_t kPairTileBytes = (size_t)256 * 256 * sizeof(float);   // and the sums of one
 constexpr int kRwMaxTiles = 16384;    // tiles of a split launch of the rows kernel, at most
 struct ScratchCounters {
     unsigned arrived[kRwMaxTiles];    // the rows kernel's blocks of a tile
@@ -538,6 +539,13 @@ __global__ __launch_bounds__(128 * NW, NW == 4 ? 1 : 2) void matmul_mfma_kernel(
     }
 }
 
+// Where a call's split-K partials go: `fixed` (the no-alloc scratch) when set,
+// else a lease of the library's growable scratch.
+struct PartialsTarget {
+    float *fixed = nullptr;
+    ScratchCounters *counters = nullptr;   // of the no-alloc scratch
+};
+
 // The arguments of a tiling by 64 NW columns and 64 MT rows (64-deep slices); false when the
 // shape does not fit the kernel.
 static bool mfma_args(MmArgs &p, int nw, int mt, void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N) {
@@ -572,20 +580,27 @@ static int launch_mfma(void *out, const void *left, const void *right, int64_t M
 // The 256 x 256 tiles with K in two halves, two blocks a tile.  Returns 1 when the shape does
 // not fit or the scratch has no room, which the undivided kernels do not need.
 template <int DT>
-static int launch_mfma_pair(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s) {
+static int launch_mfma_pair(void *out, const void *left, const void *right, int64_t M, int64_t K, int64_t N, hipStream_t s,
+                            PartialsTarget tgt) {
     MmArgs p;
     if (!mfma_args(p, 4, 4, out, left, right, M, K, N)) return 1;
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
     if (tiles > kPairTiles) return 1;
-    const size_t need = (size_t)tiles * 256 * 256 * sizeof(float);
-    if (scratch_capturing(s)) return 1;
-    ScratchLease lease(need, s, true);
-    if (lease.status()) return 1;
     p.kc = (int)((K + 127) / 128 * 64);
-    p.ws = static_cast<float *>(lease.ptr());
-    p.finished = lease.counters()->finished;
-    p.written = lease.counters()->written;
-    matmul_mfma_kernel<DT, 4, 4, 64, 2, true><<<(unsigned)((2 * p.groups + 7) / 8 * 8 * 32), 512, 0, s>>>(p);
+    auto launch = [&](float *ws, ScratchCounters *counters) {
+        p.ws = ws;
+        p.finished = counters->finished;
+        p.written = counters->written;
+        matmul_mfma_kernel<DT, 4, 4, 64, 2, true><<<(unsigned)((2 * p.groups + 7) / 8 * 8 * 32), 512, 0, s>>>(p);
+    };
+    if (tgt.fixed) {
+        launch(tgt.fixed, tgt.counters);
+        return PUTER_OK;
+    }
+    if (scratch_capturing(s)) return 1;
+    ScratchLease lease((size_t)tiles * kPairTileBytes, s, true);
+    if (lease.status()) return 1;
+    launch(static_cast<float *>(lease.ptr()), lease.counters());
     return lease.finish();
 }
 
@@ -1364,46 +1379,21 @@ int ScratchLease::finish() {
 
 // Returns 1 when the shape does not fit the skinny kernel.
 // ---- the allocation-free Matmul (puter_hip_matmul_noalloc) -----------------
-// Its split-K partials live in a file-scope device array (one copy per GPU,
+// Its split-K partials live in a file-scope device array (noalloc.hip; one copy per GPU,
 // held until the process ends) instead of the growable scratch.  The array
-// holds the counters and 16 MiB of sums, the most any split-K launch here can need: at most 512 blocks
-// (chunks x tiles) of 64 x 128 f32 partials for the 16-bit formats and for the
-// f32 VALU kernel's 64 x 64 tiles; the f32 MFMA kernel's chunk count is capped so
-// that its partials (chunks x rows x cols floats) fit it.  Host code never passes the array's name to a kernel (in host code it
-// is a stand-in, not a device address): it passes the address
-// hipGetSymbolAddress returns, looked up once per device on that device's first
-// call.  Every no-alloc call on a GPU shares that GPU's array, so such calls
+// holds the counters and 96 MiB of sums, the most any split-K launch here can need:
+// the tiles of the 256 x 256 kernel with K in two halves.  The other kernels need at
+// most 16 MiB: at most 512 blocks (chunks x tiles) of 64 x 128 f32 partials for the
+// 16-bit formats and for the f32 VALU kernel's 64 x 64 tiles; the rows kernel's runs
+// and the f32 MFMA kernel's chunks are capped so that their partials fit it.
+// Every no-alloc call on a GPU shares that GPU's array, so such calls
 // must not overlap on one GPU; each call writes every partial it reads and leaves
 // its counters at zero, so nothing needs clearing between calls.
 namespace noalloc {
 constexpr size_t kScratchBytes = (size_t)512 * 64 * 128 * sizeof(float);
-static __device__ __align__(256) char scratch[sizeof(ScratchCounters) + kScratchBytes];   // (zero when loaded)
-static std::mutex mu;
-static ScratchCounters *ptr[64];  // per device: scratch's device address
-
-static int address(ScratchCounters **out) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
-        return fail(PUTER_ERR_UNAVAILABLE, "matmul (no-alloc): no device");
-    std::lock_guard<std::mutex> g(mu);
-    if (!ptr[dev]) {
-        void *p = nullptr;
-        const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        if (e != hipSuccess || !p)
-            return fail(PUTER_ERR_UNAVAILABLE, "matmul (no-alloc): scratch address: %s", hipGetErrorString(e));
-        ptr[dev] = static_cast<ScratchCounters *>(p);
-    }
-    *out = ptr[dev];
-    return PUTER_OK;
-}
+static_assert(sizeof(ScratchCounters) + kPairTiles * kPairTileBytes <= kNoAllocBytes && kScratchBytes <= kPairTiles * kPairTileBytes,
+              "the no-alloc array holds any kernel's counters and sums");
 }  // namespace noalloc
-
-// Where a call's split-K partials go: `fixed` (the no-alloc scratch) when set,
-// else a lease of the library's growable scratch.
-struct PartialsTarget {
-    float *fixed = nullptr;
-    ScratchCounters *counters = nullptr;   // of the no-alloc scratch
-};
 
 // Runs of K of the rows kernel: toward one block per CU (200 of 256 is near enough: 16 x
 // 4096 x 14336, 112 tiles, 24.9 us in 2 runs, 25.5 in 4; 32 tiles 11.2 in 8, 14.3 in 4), each
@@ -1634,8 +1624,8 @@ static int launch_matmul16(void *out, const void *left, const void *right, int64
             const int rc = launch_skinny<DT>(out, left, right, M, K, N, s, tgt, M <= 512 ? 0 : 1024);
             if (rc != 1) return rc;
         }
-        if (!tgt.fixed && mfma_pair_wins(M, K, N)) {
-            const int rc = launch_mfma_pair<DT>(out, left, right, M, K, N, s);
+        if (mfma_pair_wins(M, K, N)) {
+            const int rc = launch_mfma_pair<DT>(out, left, right, M, K, N, s, tgt);
             if (rc != 1) return rc ? rc : check_launch("matmul mfma");
         }
         const int rc = mfma_small_tiles(M, N) ? launch_mfma<DT, 2, 2>(out, left, right, M, K, N, s)
@@ -1802,8 +1792,10 @@ static int matmul_entry(void *out, const void *left, const void *right, int64_t 
     }
     PartialsTarget tgt;
     if (no_alloc) {
-        const int rc = noalloc::address(&tgt.counters);
+        void *array = nullptr;
+        const int rc = noalloc_scratch(&array);
         if (rc) return rc;
+        tgt.counters = static_cast<ScratchCounters *>(array);
         tgt.fixed = reinterpret_cast<float *>(tgt.counters + 1);
     }
     switch (dtype) {

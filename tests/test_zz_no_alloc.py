@@ -1,8 +1,8 @@
 """GPU tier (collected last): the allocation-free Matmul entry point (puter_hip_matmul_noalloc)
 against puter_hip_matmul, both through the C ABI.  The two share every kernel
 and split-K chunking, so the results must be bit-identical.  Two calls in a row
-on the shared static scratch, the second smaller, and a call at the scratch's
-full 16 MiB capacity."""
+on the shared static scratch, the second smaller, and calls at the full 16 MiB
+that most kernels use of the scratch and at its 96 MiB capacity."""
 import ctypes as C
 
 import numpy as np
@@ -33,6 +33,9 @@ def _operands(dt, m, k, n, seed):
     # 16 MiB of partials), then a smaller split-K shape and a ragged one
     (O.BF16, [(128, 4096, 4096), (16, 1024, 512), (5, 256, 136)]),
     (O.F16, [(64, 2048, 1024), (33, 512, 264)]),
+    # 256 x 256 tiles with K in two halves: half a round, and one and a half of them (the
+    # array's full 96 MiB), with a split of the rows kernel between
+    (O.BF16, [(2041, 8200, 4088), (4, 4096, 4096), (3072, 8192, 8192)]),
     # f32: K split inside each block (128x512x512, no scratch), then K split
     # across blocks on the f32 MFMA kernel with partials in the scratch (256x4096x512,
     # 16 chunks: 8 MiB; 1024x8192x1024, chunks capped at 4 to fit the 16 MiB), the
