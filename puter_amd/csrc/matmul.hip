@@ -1580,11 +1580,15 @@ static int launch_matmul16(void *out, const void *left, const void *right, int64
     // kernel and its reduce launch 1 x 4096 x 4096 14.1 -> 9.5 us, 1 x 4096 x 14336 25.2 ->
     // 22.7, 16 x 14336 x 4096 35.0 -> 24.0, 32 x 4096 x 4096 15.4 -> 13.6; at 64 rows the
     // skinny kernel wins (64 x 4096 x 14336: 33.1 against 35.3), and where it runs unsplit, with
-    // no second launch: a K of one slice (32 x 64 x 1024 2.9 us against 4.1) and, up to 2048 deep,
-    // columns for a round of blocks (32 x 1024 x 131072 42 against 52); of those up to 16 rows of
-    // little K over more columns yet are the rows kernel's (1 x 64 x 131072 3.6 against 4.7)
+    // no second launch: a K of one slice (32 x 64 x 1024 2.9 us against 4.1), columns for more than
+    // one round of blocks and up to two of its own (8 x 4096 x 33000 60 against 79, 32 x 8192 x
+    // 45000 158 against 190), and more columns up to 2048 deep (32 x 1024 x 131072 42 against 52;
+    // 8 x 4096 x 80000 135 against 104); of those up to 16 rows of little K over the
+    // most columns are the rows kernel's (1 x 64 x 131072 3.6 against 4.7)
     const bool fits = N % 8 == 0 && K % 8 == 0 && aligned16(out) && aligned16(left) && aligned16(right);
-    const bool skinny = fits && K <= 2048 && skinny_chunks(M, K, N, 0) == 1 && !(M <= 16 && K <= 192 && N > 65536);
+    const int64_t cus = device_cus(), columns = (N + kRwCols - 1) / kRwCols;
+    const bool skinny = fits && skinny_chunks(M, K, N, 0) == 1 && (K <= 2048 || (columns > cus && columns <= 2 * cus)) &&
+                        !(M <= 16 && K <= 192 && N > 65536);
     if (fits ? M <= 32 && !skinny : !generic_wins<DT>(M, K, N)) {
         const int rc = launch_rows<DT>(out, left, right, M, K, N, s, tgt, !fits);
         if (rc != 1) return rc;
@@ -1619,7 +1623,7 @@ static int launch_matmul16(void *out, const void *left, const void *right, int64
         // 543, 2048^3 612 -> 651 unsplit; 1024^3 split four ways fell 165 -> 105, hence
         // the depth floor; from one full round up the MFMA kernels win: 4096 x 1024 x
         // 2048 845 against 601)
-        const bool few_tiles = ((M + 127) / 128) * ((N + 127) / 128) < 2 * (int64_t)device_cus();
+        const bool few_tiles = ((M + 127) / 128) * ((N + 127) / 128) < 2 * cus;
         if (M <= 512 || few_tiles) {
             const int rc = launch_skinny<DT>(out, left, right, M, K, N, s, tgt, M <= 512 ? 0 : 1024);
             if (rc != 1) return rc;

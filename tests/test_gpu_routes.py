@@ -57,7 +57,8 @@ def test_norm_kernels(backend, op, dt, rows, h, kernel):
     (O.BF16, 1, 4096, 4096, ["matmul_rows"]), (O.BF16, 32, 4096, 4096, ["matmul_rows"]),
     # one slice of K, or a round of column tiles: the skinny kernel unsplit
     (O.BF16, 32, 64, 1024, ["matmul_skinny"]), (O.F16, 4, 32, 4096, ["matmul_skinny"]),
-    (O.BF16, 32, 1024, 65536, ["matmul_skinny"]), (O.BF16, 8, 64, 131072, ["matmul_rows"]),
+    (O.BF16, 32, 1024, 65536, ["matmul_skinny"]), (O.BF16, 8, 4096, 33000, ["matmul_skinny"]),
+    (O.BF16, 8, 4096, 80000, ["matmul_rows"]), (O.BF16, 8, 64, 131072, ["matmul_rows"]),
     (O.BF16, 64, 4096, 4096, ["matmul_skinny", "matmul_splitk_reduce"]),
     # unaligned: the generic kernel where K is small
     (O.BF16, 65, 5, 33, ["matmul_generic"]), (O.BF16, 20, 15, 129, ["matmul_generic"]),
