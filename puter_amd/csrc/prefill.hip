@@ -1164,8 +1164,8 @@ static double general_us(const MhaArgs &m, bool f32) {
 // The padded kernels: the key tiles of the longest block, in rounds of blocks.
 static double padded_us(const MhaArgs &m, int64_t blocks, int64_t tiles, int64_t splits, bool f32) {
     const int i = m.dim <= 64 ? 0 : m.dim <= 96 ? 1 : m.dim <= 128 ? 2 : 3;
-    constexpr double base[2][4] = {{3.5, 4.2, 4.6, 6.7}, {3.7, 4.5, 6.2, 8.0}};
-    constexpr double tile[2][4] = {{0.94, 1.14, 1.3, 2.9}, {2.5, 3.7, 6.3, 13.0}};
+    constexpr double base[2][4] = {{3.5, 4.2, 4.6, 7.4}, {3.7, 4.5, 6.2, 8.0}};
+    constexpr double tile[2][4] = {{0.94, 1.14, 1.3, 2.85}, {2.5, 3.7, 6.3, 13.0}};
     const int64_t room = (int64_t)device_cus() * (m.dim > 128 ? 1 : 2), rounds = (blocks * splits + room - 1) / room;
     const double sums = splits > 1 ? 1.2 + 0.53 * (double)splits + 4.3e-6 * (double)(splits * m.batch * m.seq_q * m.heads * m.dim) : 0.0;
     return base[f32][i] + tile[f32][i] * (double)(tiles * rounds) + sums;
