@@ -417,12 +417,11 @@ __global__ __launch_bounds__(THREADS) void page_write_fp8_kernel(uint8_t *__rest
     }
 }
 
-// Rows per write block (a power of two, 2 up to 1024 rows, else 8..1024, about rows / 512;
-// at most 16
-// for the 256-thread blocks of calls up to kSmallWriteRows rows, so R never
-// exceeds the block's threads) and log2 of its table size (2R entries).
-static int64_t write_rows_per_block(int64_t rows, int *table_bits) {
-    int64_t r = rows <= 1024 ? 2 : 8;
+// Rows per write block (a power of two, from 2, when the rows are to be spread, or 8 to 1024,
+// about rows / 512; at most 16 for the 256-thread blocks of calls up to kSmallWriteRows
+// rows, so R never exceeds the block's threads) and log2 of its table size (2R entries).
+static int64_t write_rows_per_block(int64_t rows, bool spread, int *table_bits) {
+    int64_t r = spread ? 2 : 8;
     while (r < kWriteMaxRows && r * 512 < rows) r <<= 1;
     int bits = 0;
     while (((int64_t)1 << bits) < 2 * r) ++bits;
@@ -465,7 +464,10 @@ int puter_hip_kv_page_write(const void *storage, const void *values, const int32
         if (e != hipSuccess) return fail(PUTER_ERR_LAUNCH, "kv page write: copy: %s", hipGetErrorString(e));
     }
     int bits = 0;
-    const int64_t per = write_rows_per_block(value_rows, &bits);
+    // a handful of small rows is one block's work: a second one costs more to start (4 rows of 2 KB
+    // 2.8 us in one block, 3.4 in two; 8 of 4 KB 5.0 and, in four, 3.7; 16 of 128 B 3.2 and 3.5)
+    const bool handful = value_rows <= 16 && (size_t)value_rows * row_bytes <= 16384;
+    const int64_t per = write_rows_per_block(value_rows, value_rows <= 1024 && !handful, &bits);
     const int64_t nblocks = (value_rows + per - 1) / per;
     if (nblocks > 0x7FFFFFFF) return fail(PUTER_ERR_INVALID, "kv page write: too many rows");
     const unsigned blocks = (unsigned)nblocks;
@@ -513,7 +515,7 @@ int puter_hip_kv_page_write_fp8(void *storage, const void *values, const int32_t
         return fail(PUTER_ERR_INVALID, "kv page write fp8: pool rows must be 16-byte aligned");
     hipStream_t s = as_stream(stream);
     int bits = 0;
-    const int64_t per = write_rows_per_block(value_rows, &bits);
+    const int64_t per = write_rows_per_block(value_rows, value_rows <= 1024, &bits);
     const int64_t nblocks = (value_rows + per - 1) / per;
     if (nblocks > 0x7FFFFFFF) return fail(PUTER_ERR_INVALID, "kv page write fp8: too many rows");
     const unsigned blocks = (unsigned)nblocks;

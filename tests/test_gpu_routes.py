@@ -20,6 +20,26 @@ def launched(call):
     return [e.name for e in p.events() if "puter::" in e.name or "_kernel" in e.name]
 
 
+def grids(call):
+    """The blocks of the kernels that call launches."""
+    import json
+    import os
+    import tempfile
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        call()
+        torch.cuda.synchronize()
+    with tempfile.TemporaryDirectory() as d:
+        path = os.path.join(d, "trace.json")
+        p.export_chrome_trace(path)
+        with open(path) as f:
+            events = json.load(f)["traceEvents"]
+    found = [e["args"]["grid"] for e in events if e.get("cat") == "kernel" and "puter::" in e["name"]]
+    return [x * y * z for x, y, z in found]
+
+
 def zeros(dt, *shape):
     import torch
     t = {O.F32: torch.float32, O.BF16: torch.bfloat16, O.F16: torch.float16}[dt]
@@ -84,7 +104,9 @@ def test_matmul_kernels(backend, dt, rows, inner, cols, kernels):
 def test_flash_kernels(backend, dt, seq_q, seq_k, dim, causal, kernel):
     q, k, out = zeros(dt, seq_q, dim), zeros(dt, seq_k, dim), zeros(dt, seq_q, dim)
     cfg = puter_amd.FlashAttentionConfig(64, causal)
-    names = launched(lambda: backend.FlashAttention(cfg, q, k, k, out, seq_q, seq_k, dim, dim, dt))
+    call = lambda: backend.FlashAttention(cfg, q, k, k, out, seq_q, seq_k, dim, dim, dt)  # noqa: E731
+    call()   # (the scratch is there)
+    names = launched(call)
     assert kernel in names[0], names
 
 
@@ -116,3 +138,15 @@ def test_split_f32_attention_combines_by_head_dim(backend):
 def test_attention_kernels(backend, dt, seq_q, seq_k, heads, dim, kernel):
     names = mha(backend, dt, seq_q, seq_k, heads, dim)
     assert kernel in names[0], names
+
+
+@pytest.mark.parametrize("rows,inner,blocks", [(3, 64, 1), (4, 1024, 1), (16, 64, 2), (8, 2048, 4), (64, 1024, 32),
+                                               (1025, 64, 129)])
+def test_page_write_blocks(backend, rows, inner, blocks):
+    """A handful of small rows is written by one block, more rows by two to a block."""
+    import torch
+    pool, values = zeros(O.BF16, 128, 16, inner), zeros(O.BF16, rows, inner)
+    at = torch.arange(rows, dtype=torch.int32, device="cuda")
+    ids, slots = at // 16, at % 16
+    call = lambda: backend.KVPageWrite(pool, values, ids, slots, pool, 128, 16, inner, rows, 0, O.BF16)  # noqa: E731
+    assert grids(call) == [blocks]
