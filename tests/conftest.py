@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -19,3 +20,15 @@ def backend():
         pytest.skip("no GPU")
     import puter_amd
     return puter_amd.Backend()
+
+
+@pytest.fixture
+def no_collection():
+    """For tests that capture a graph: a reference cycle of an earlier test (a caught
+    exception holds its frame, the frame the graph) that the collector takes apart while a
+    stream is capturing destroys that graph there, which the runtime refuses, and torch ends the
+    process.  So cycles are collected before the test, and none while it runs."""
+    gc.collect()
+    gc.disable()
+    yield
+    gc.enable()

@@ -25,7 +25,7 @@ import puter_amd
 from puter_amd._lib import ERR_INVALID
 from helpers import TOL, assert_close, seeded, to_dev, to_host
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("no_collection")]
 
 
 @pytest.mark.parametrize("kv_dt", [O.BF16, O.F8E4M3])

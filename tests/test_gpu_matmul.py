@@ -385,6 +385,7 @@ def test_matmul_16bit_rows_kernel_exact(backend, dt, rows, inner, cols, shift):
         assert np.array_equal(got[shift:shift + rows * cols].reshape(rows, cols), want), (dt, rows, inner, cols, rep)
 
 
+@pytest.mark.usefixtures("no_collection")
 def test_matmul_default_and_side_streams_keep_apart(backend):
     """Split-K calls on the default stream and on two side streams, interleaved without
     synchronisation: the default stream's partials are in a buffer of its own (no events
@@ -427,6 +428,7 @@ def test_matmul_default_and_side_streams_keep_apart(backend):
         (torch.randn(1 << 20, device="cuda") * 2).sum().item()
 
 
+@pytest.mark.usefixtures("no_collection")
 def test_matmul_unaligned_captured_without_scratch(backend):
     """A shape that only the rows kernel takes was never refused under stream capture (the
     generic kernel needs no scratch): captured, it does not split K, so graphs of it need no
@@ -465,6 +467,7 @@ def test_matmul_empty_inner_is_zero(backend, dt, np_dt):
     (1793, 16384, 4096),   # the last row tile of one row
     (4100, 7752, 4096),    # one and a half rounds, row tiles past a multiple of four
 ])
+@pytest.mark.usefixtures("no_collection")
 def test_matmul_16bit_two_halves_of_k_exact(backend, dt, rows, inner, cols):
     """256 x 256 tiles whose K is divided between two blocks, bit for bit: integer operands keep
     every sum exact.  On the default stream and on a side stream (each has its own sums and

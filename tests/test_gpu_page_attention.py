@@ -958,6 +958,7 @@ def test_matmul_f32(backend):
         assert_close(to_host(out, np.float32), ref, TOL[O.F32], elem_tol=1e-3, what="matmul")
 
 
+@pytest.mark.usefixtures("no_collection")
 def test_flash_f32_captured_beside_eager_calls(backend):
     """A captured f32 call takes no scratch (it was never refused there): its replays agree with
     the oracle and need no order with eager calls on another stream, whose scores are in
