@@ -525,50 +525,144 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
 
 // The padded kernels' outputs where an infinity or NaN of V met a P of zero (a masked key
 // of a computed tile, or P's low half): 0 * inf is NaN in the MFMA, while the general
-// kernel, which served these head dims before, never reads a masked key's row.  Such rows
-// (a finite row sum, some output not finite) are summed again here, key by key over the
-// visible keys [k_lo, k_hi), in f32, against the same reference m; the lane's dims are
-// 32d + 8 rb + 4 g .. + 3.  Never taken on finite values.
-template <int DT, int D, int NO>
-__device__ __forceinline__ void prefill_redo(const PrefillArgs &a, const void *qrow, const void *kbase,
-                                             const void *vbase, int64_t krs, int dim, int qi, int g, int k_lo,
-                                             int k_hi, float m, f32x16 (&o)[NO]) {
-    using T = typename Elem<DT>::T;
-    const T *const Q = static_cast<const T *>(qrow);
-#pragma unroll
-    for (int d = 0; d < D / 32; ++d) o[d] = (f32x16){};
-    for (int k = k_lo; k < k_hi; ++k) {
-        const T *const K = static_cast<const T *>(kbase) + k * krs;
-        const T *const V = static_cast<const T *>(vbase) + k * krs;
-        float dot = 0.0f;
-        for (int x = 0; x < dim; ++x) dot += Elem<DT>::load(Q[x]) * Elem<DT>::load(K[x]);
-        if constexpr (DT == PUTER_F16) dot = (float)(_Float16)dot;
-        dot += a.alibi_s * (float)(k - qi);
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(dot, a.scale_log2, -m));
-#pragma unroll
-        for (int d = 0; d < D / 32; ++d)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int c = 32 * d + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (c < dim) o[d][r] += p * Elem<DT>::load(V[c]);
-            }
-    }
-}
-// whether a lane's O holds an infinity or NaN
-template <int D, int NO> __device__ __forceinline__ bool prefill_spoiled(const f32x16 (&o)[NO]) {
+// kernel, which served these head dims before, never reads a masked key's row.  A block
+// with such outputs (a finite row sum, some output not finite) walks its key tiles once more
+// against the final reference m: values that are not finite count as zero in the products,
+// and what a row sees of them is counted on the MFMA too, per tile, by products of 0 / 1
+// with a value's class (a visible key of probability zero makes an infinity a NaN, as 0 *
+// inf does).  Only outputs that were not finite are replaced.  The second walk costs what the
+// first does and is never taken on finite values; a lane summing its row key by key took
+// 18 ms for bf16 2 x 700 of 1500 keys x 16 heads of 96 with a NaN in V, the general kernel 1.0; now
+// 107 us, 36 without the NaN.
+// It runs after the first walk's outputs are stored and loads Q again: with more alive the first
+// walk of 129 to 256 dims slowed by 4 to 9%, now by 2 to 3% (not inlined, by the stack that a call
+// needs: 34 -> 38 us).
+constexpr float kPfPos = 1.0f, kPfNeg = 128.0f, kPfNan = 16384.0f;   // up to 64 keys a tile: digits that stay apart
+// a lane's outputs that are not finite: bit 16 (d % 2) + r of word d / 2; whether there are any
+template <int NO> __device__ __forceinline__ bool prefill_spoiled(const f32x16 (&o)[NO], uint32_t (&bits)[(NO + 1) / 2]) {
     float t = 0.0f;
 #pragma unroll
-    for (int d = 0; d < D / 32; ++d)
+    for (int d = 0; d < NO; ++d)
 #pragma unroll
         for (int r = 0; r < 16; ++r) t = __builtin_fmaf(o[d][r], 0.0f, t);
-    return t != 0.0f;   // 0 * x is NaN for an infinite or NaN x
+    if (t == 0.0f) return false;   // (0 * x is NaN for an infinite or NaN x)
+#pragma unroll
+    for (int d = 0; d < NO; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            if (!(__builtin_fabsf(o[d][r]) < INFINITY)) bits[d >> 1] |= 1u << (16 * (d & 1) + r);
+    return true;
 }
-// the keys of [0, seq_k) that query qi sees: [first, last)
-__device__ __forceinline__ int prefill_first_key(const PrefillArgs &a, int qi) {
-    return a.window > 0 ? max(0, qi - a.window + 1) : 0;
+// adds the infinities and NaNs that were counted
+__device__ __forceinline__ void prefill_add_classes(f32x16 &o, const f32x16 &count) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const uint32_t n = (uint32_t)count[r];
+        if (n & 127) o[r] += INFINITY;
+        if (n >> 7 & 127) o[r] -= INFINITY;
+        if (n >> 14) o[r] = NAN;
+    }
 }
-__device__ __forceinline__ int prefill_last_key(const PrefillArgs &a, int qi) {
-    return a.causal ? min(qi + a.shift + 1, a.seq_k) : a.seq_k;
+template <int DT, int D, bool GEN>
+__device__ __forceinline__ void prefill_redo(const PrefillArgs &a, const uint16_t *qrow, const uint16_t *kbase,
+                                             const uint16_t *vbase, char *ks, char *vs, const int (&kg)[PfDim<D>::NI],
+                                             const int (&vg)[PfDim<D>::NI], const int (&ka)[PfDim<D>::KS],
+                                             const int (&va)[PfDim<D>::DB], int tlo, int ntiles, int qi, int g,
+                                             int wave, float m, float inv, const uint32_t (&bits)[(PfDim<D>::DB + 1) / 2], uint16_t *orow) {
+    using namespace fa;
+    using T = PfDim<D>;
+    using V8 = typename PfFormat<DT>::V8;
+    using E = typename PfFormat<DT>::E;
+    constexpr uint32_t EXP = DT == PUTER_BF16 ? 0x7F80u : 0x7C00u;
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    const int first = GEN && a.window > 0 ? qi - a.window + 1 : 0;
+    const int last = a.causal ? min(qi + a.shift, a.seq_k - 1) : a.seq_k - 1;
+    const float mref = m == -INFINITY ? 0.0f : m;
+    bool spoiled = false;
+#pragma unroll
+    for (int w = 0; w < (T::DB + 1) / 2; ++w) spoiled |= bits[w] != 0;
+    const bool mine = __any(spoiled);
+    V8 qf[T::KS];
+#pragma unroll
+    for (int t = 0; t < T::KS; ++t)
+        qf[t] = 16 * t + 8 * g < a.dim ? __builtin_bit_cast(V8, *reinterpret_cast<const uint4 *>(qrow + 16 * t + 8 * g)) : (V8){};
+    f32x16 o[T::DB];
+#pragma unroll
+    for (int d = 0; d < T::DB; ++d) o[d] = (f32x16){};
+    for (int it = tlo; it < ntiles; ++it) {
+        const int kv0 = it * BN;
+        prefill_copy_tile<D, true>(a, kbase, vbase, kv0, kg, vg, ks, vs, wave);
+        wait_tile_copies();
+        __syncthreads();
+        if (mine) {
+#pragma unroll 1
+            for (int c = 0; c < 2; ++c) {
+                f32x16 s = (f32x16){};
+#pragma unroll
+                for (int t = 0; t < T::KS; ++t)
+                    s = pf_mfma<DT>(*reinterpret_cast<const V8 *>(ks + c * 32 * T::RB + ka[t]), qf[t], s);
+                V8 p[2], seen[2], zero[2];
+                PfLow<DT, true> low[2];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = kv0 + 32 * c + 8 * (r >> 2) + 4 * g + (r & 3);
+                    float dot = s[r];
+                    if constexpr (DT == PUTER_F16) dot = (float)(_Float16)dot;
+                    if (GEN) dot += a.alibi_s * (float)(key - qi);
+                    const bool vis = key >= first && key <= last;
+                    const float e = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(dot, a.scale_log2, -mref)) : 0.0f;
+                    pf_set<DT, true>(p[r >> 3], low[r >> 3], r & 7, e);
+                    seen[r >> 3][r & 7] = (E)(vis ? 1.0f : 0.0f);
+                    zero[r >> 3][r & 7] = (E)(vis && e == 0.0f ? 1.0f : 0.0f);
+                }
+#pragma unroll
+                for (int d = 0; d < T::DB; ++d) {
+                    u16x8 v[2];
+                    bool bad = false;
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const char *q = vs + va[d] + (32 * c + 16 * h) * T::RB;
+                        const i16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(q));
+                        const i16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4 *)(q + 8 * T::RB));
+                        v[h] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                        u16x8 fin;
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const bool f = (v[h][j] & EXP) != EXP;
+                            bad |= !f;
+                            fin[j] = f ? v[h][j] : (uint16_t)0;
+                        }
+                        o[d] = pf_pv<DT, true>(__builtin_bit_cast(V8, fin), p[h], low[h], o[d]);
+                    }
+                    if (!__any(bad)) continue;
+                    f32x16 count = (f32x16){};
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        V8 cls, inf;
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const uint32_t x = v[h][j], mag = x & 0x7FFFu;
+                            cls[j] = (E)(mag < EXP ? 0.0f : mag > EXP ? kPfNan : x >> 15 ? kPfNeg : kPfPos);
+                            inf[j] = (E)(mag == EXP ? kPfNan : 0.0f);
+                        }
+                        count = pf_mfma<DT>(cls, seen[h], count);
+                        count = pf_mfma<DT>(inf, zero[h], count);
+                    }
+                    prefill_add_classes(o[d], count);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!spoiled) return;
+#pragma unroll
+    for (int d = 0; d < T::DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int at = 32 * d + 8 * (r >> 2) + 4 * g + (r & 3);
+            if ((bits[d >> 1] >> (16 * (d & 1) + r) & 1) && at < a.dim)
+                orow[at] = __builtin_bit_cast(uint16_t, (E)(o[d][r] * inv));
+        }
 }
 
 // GEN: a sliding window (a.window > 0) or an ALiBi slope is set; without either
@@ -589,10 +683,12 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
     __shared__ __attribute__((aligned(1024))) char k1s[T::TILE];
     __shared__ __attribute__((aligned(1024))) char v0s[T::TILE];
     __shared__ __attribute__((aligned(1024))) char v1s[T::TILE];
+    __shared__ int redo;   // PAD: bit w: some output of dims 64 w .. + 63 is not finite
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, g = lane >> 5;
+    if (PAD && tid == 0) redo = 0;
 
     // block -> (query tile, batch, head)
     const int id = blockIdx.x;
@@ -740,10 +836,15 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
     // normalise and store: lane holds O[qi][32d + 8*(r/4) + 4g + r%4]
     const float ltot = swap_halves_sum(st.l);
     const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
+    uint32_t bits[(T::DB + 1) / 2] = {};
+    bool spoiled = false;
     if constexpr (PAD) {
-        if (ltot > 0.0f && qi < a.seq_q && prefill_spoiled<D>(st.o))
-            prefill_redo<DT, D>(a, qbase + (int64_t)qi * qrs, kbase, vbase, krs, dim, qi, g, prefill_first_key(a, qi),
-                                prefill_last_key(a, qi), st.m, st.o);
+        spoiled = ltot > 0.0f && qi < a.seq_q && prefill_spoiled(st.o, bits);
+        if (spoiled) {
+#pragma unroll
+            for (int w = 0; w < (T::DB + 1) / 2; ++w)
+                if (bits[w]) atomicOr(&redo, 1 << w);
+        }
         // a NaN row sum (a NaN score): zeros, or NaN from FlashAttention, as the general kernels
         if (!(ltot > 0.0f)) {
             const float z = a.nan_rows ? ltot : 0.0f;
@@ -765,6 +866,13 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
                 for (int i = 0; i < 4; ++i) v[i] = (E)(PAD && !(ltot > 0.0f) ? st.o[d][4 * rb + i] : st.o[d][4 * rb + i] * inv);
                 *reinterpret_cast<V4 *>(orow + 32 * d + 8 * rb + 4 * g) = v;
             }
+    }
+    if constexpr (PAD) {
+        __syncthreads();
+        if (__builtin_expect(!redo, 1)) return;
+        const int64_t row = (int64_t)min(qi, a.seq_q - 1) * qrs;
+        prefill_redo<DT, D, GEN>(a, qbase + row, kbase, vbase, k0s, v0s, kg, vg, ka, va, tlo, ntiles, qi, g, wave, st.m, inv, bits,
+                                 a.o + (qbase - a.q) + row);
     }
 }
 
@@ -799,6 +907,96 @@ template <int D> struct PfF32Dim {
     static constexpr int vswz(int r) { return ((r >> 2) & 1) << 3; }   // in chunks (8 = 32 floats)
 };
 
+// prefill_redo for f32 (a value is one float per lane and MFMA step).  Beyond 128 dims two blocks
+// of 32 a walk, those that need it: with all of them alive the first walk spilled (129 -> 136 us
+// for 2 x 512 x 8 of 256, now 128).
+constexpr int redo_blocks(int D) { return D > 128 ? 2 : D / 32; }
+constexpr int redo_words(int D) { return (redo_blocks(D) + 1) / 2; }
+template <int D, bool GEN, typename Copy>
+__device__ __forceinline__ void prefill_f32_redo(const PrefillArgs &a, Copy copy_tile, const float *qrow, char *ks, char *vs,
+                                                 int kr, const int (&vr)[redo_blocks(D)], int d0, int tlo, int thi, int qi,
+                                                 int l32, int h, float m, float inv, const uint32_t (&bits)[redo_words(D)],
+                                                 float *orow) {
+    using T = PfF32Dim<D>;
+    const int first = GEN && a.window > 0 ? qi - a.window + 1 : 0;
+    const int last = a.causal ? min(qi + a.shift, a.seq_k - 1) : a.seq_k - 1;
+    const float mref = m == -INFINITY ? 0.0f : m;
+    constexpr int NB = redo_blocks(D);
+    bool spoiled = false;
+#pragma unroll
+    for (int w = 0; w < redo_words(D); ++w) spoiled |= bits[w] != 0;
+    const bool mine = __any(spoiled);
+    f32x4 qf[T::KG];
+#pragma unroll
+    for (int g = 0; g < T::KG; ++g)
+        qf[g] = 8 * g + 4 * h < a.dim ? *reinterpret_cast<const f32x4 *>(qrow + 8 * g + 4 * h) : (f32x4){};
+    f32x16 o[NB];
+#pragma unroll
+    for (int db = 0; db < NB; ++db) o[db] = (f32x16){};
+    for (int it = tlo; it < thi; ++it) {
+        const int kv0 = it * T::BN;
+        copy_tile(kv0, ks, vs);
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0)
+        __syncthreads();
+        if (mine) {
+            f32x16 p = (f32x16){};
+#pragma unroll
+            for (int g = 0; g < T::KG; ++g) {
+                const f32x4 kv = *reinterpret_cast<const f32x4 *>(ks + kr + (((2 * g + h) ^ T::kswz(l32)) << 4));
+#pragma unroll
+                for (int s4 = 0; s4 < 4; ++s4) p = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[s4], qf[g][s4], p, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);   // as in the first walk
+            }
+            uint32_t seen = 0, zero = 0;   // register r's key: visible, and of probability zero
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kv0 + 8 * (r >> 2) + 4 * h + (r & 3);
+                float dot = p[r];
+                if (GEN) dot += a.alibi_s * (float)(key - qi);
+                const bool vis = key >= first && key <= last;
+                p[r] = vis ? __builtin_amdgcn_exp2f(__builtin_fmaf(dot, a.scale_log2_lo, __builtin_fmaf(dot, a.scale_log2, -mref))) : 0.0f;
+                seen |= (uint32_t)vis << r;
+                zero |= (uint32_t)(vis && p[r] == 0.0f) << r;
+            }
+#pragma unroll
+            for (int db = 0; db < NB; ++db) {
+                f32x16 t = (f32x16){};
+                bool bad = false;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float v = *reinterpret_cast<const float *>(vs + (8 * (r >> 2) + (r & 3)) * T::RB + vr[db]);
+                    const bool f = __builtin_fabsf(v) < INFINITY;
+                    bad |= !f;
+                    t = __builtin_amdgcn_mfma_f32_32x32x2f32(f ? v : 0.0f, p[r], t, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[db][r] += t[r];
+                if (!__any(bad)) continue;
+                t = (f32x16){};
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const float v = *reinterpret_cast<const float *>(vs + (8 * (r >> 2) + (r & 3)) * T::RB + vr[db]);
+                    const float cls = v != v ? kPfNan : v == INFINITY ? kPfPos : v == -INFINITY ? kPfNeg : 0.0f;
+                    const float inf = __builtin_fabsf(v) == INFINITY ? kPfNan : 0.0f;
+                    t = __builtin_amdgcn_mfma_f32_32x32x2f32(cls, (float)(seen >> r & 1), t, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_32x32x2f32(inf, (float)(zero >> r & 1), t, 0, 0, 0);
+                }
+                prefill_add_classes(o[db], t);
+            }
+        }
+        __syncthreads();
+    }
+    if (!spoiled) return;
+#pragma unroll
+    for (int db = 0; db < NB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int at = 32 * (d0 + db) + 8 * (r >> 2) + 4 * h + (r & 3);
+            if ((bits[db >> 1] >> (16 * (db & 1) + r) & 1) && at < a.dim) orow[at] = o[db][r] * inv;
+        }
+}
+
 template <int D, bool GEN, bool PAD>
 __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(PrefillArgs a) {
     using T = PfF32Dim<D>;
@@ -807,10 +1005,12 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(Prefi
     __shared__ __attribute__((aligned(1024))) char k1s[T::TILE];
     __shared__ __attribute__((aligned(1024))) char v0s[T::TILE];
     __shared__ __attribute__((aligned(1024))) char v1s[T::TILE];
+    __shared__ int redo;   // PAD: bit w: some output of dims 64 w .. + 63 is not finite
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, h = lane >> 5;
+    if (PAD && tid == 0) redo = 0;
 
     // block -> (query tile, batch, head), heaviest tiles first, a kv group's query
     // heads on one XCD (as prefill_kernel)
@@ -909,11 +1109,11 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(Prefi
     // fragment reads: K row l32, group g at chunk (2 g + h) ^ kswz(l32); V row
     // 8 g + 4 h + s, column (32 db + l32) ^ 32 h (vswz(row) = 8 chunks iff h = 1)
     const int kr = l32 * T::RB;
-    int vr[8];
+    int vr[T::DB];
 #pragma unroll
     for (int db = 0; db < T::DB; ++db) vr[db] = 4 * h * T::RB + (((32 * db + l32) ^ (32 * h)) << 2);
 
-    f32x16 o[8];
+    f32x16 o[T::DB];
 #pragma unroll
     for (int db = 0; db < T::DB; ++db) o[db] = (f32x16){};
     float m = -INFINITY, l = 0.0f;
@@ -1039,22 +1239,29 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(Prefi
     if (it < thi) tile(it, k0s, v0s, k1s, v1s);
 
     const float ltot = swap_halves_sum(l);
+    uint32_t bits[(T::DB + 1) / 2] = {};
+    bool spoiled = false;
     if constexpr (PAD) {
-        if (ltot > 0.0f && qi < a.seq_q && prefill_spoiled<D>(o))
-            prefill_redo<PUTER_F32, D>(a, qbase + (int64_t)qi * qrs, kbase, vbase, krs, dim, qi, h,
-                                       max(prefill_first_key(a, qi), tlo * BN), min(prefill_last_key(a, qi), thi * BN), m, o);
+        spoiled = ltot > 0.0f && qi < a.seq_q && prefill_spoiled(o, bits);
+        if (spoiled) {
+#pragma unroll
+            for (int w = 0; w < (T::DB + 1) / 2; ++w)
+                if (bits[w]) atomicOr(&redo, 1 << w);
+        }
         if (!(ltot > 0.0f)) {   // a NaN score: zeros, as the general kernel
 #pragma unroll
             for (int db = 0; db < 8; ++db)
                 if (db < T::DB) o[db] = (f32x16){};
         }
     }
+    float *orow;
+    float inv = 1.0f;
     if (a.part_ml) {
         // split: the row's (max, sum) and unnormalised output to the partials
+        const int64_t prow = (((int64_t)blockIdx.y * a.batch + b) * a.seq_q + qi) * a.heads + hd;
+        orow = a.part_o + prow * dim;
         if (qi < a.seq_q) {
-            const int64_t prow = (((int64_t)blockIdx.y * a.batch + b) * a.seq_q + qi) * a.heads + hd;
             if (h == 0) a.part_ml[prow] = make_float2(m, ltot);
-            float *orow = a.part_o + prow * dim;
 #pragma unroll
             for (int db = 0; db < 8; ++db) {
                 if (db >= T::DB) break;
@@ -1068,22 +1275,39 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_f32_kernel(Prefi
                 }
             }
         }
-        return;
+    } else {
+        // normalise and store: lane holds O[qi][32 db + 8 (r/4) + 4 h + r%4]
+        inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
+        orow = reinterpret_cast<float *>(a.o) + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)hd * dim;
+        if (qi < a.seq_q) {
+#pragma unroll
+            for (int db = 0; db < 8; ++db) {
+                if (db >= T::DB) break;
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) {
+                    if (32 * db + 8 * rb + 4 * h >= dim) continue;   // dim % 4 == 0
+                    f32x4 v;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = o[db][4 * rb + i] * inv;
+                    *reinterpret_cast<f32x4 *>(orow + 32 * db + 8 * rb + 4 * h) = v;
+                }
+            }
+        }
     }
-    // normalise and store: lane holds O[qi][32 db + 8 (r/4) + 4 h + r%4]
-    const float inv = ltot > 0.0f ? 1.0f / ltot : 0.0f;
-    if (qi < a.seq_q) {
-        float *orow = reinterpret_cast<float *>(a.o) + (int64_t)b * a.seq_q * qrs + (int64_t)qi * qrs + (int64_t)hd * dim;
-#pragma unroll
-        for (int db = 0; db < 8; ++db) {
-            if (db >= T::DB) break;
-#pragma unroll
-            for (int rb = 0; rb < 4; ++rb) {
-                if (32 * db + 8 * rb + 4 * h >= dim) continue;   // dim % 4 == 0
-                f32x4 v;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = o[db][4 * rb + i] * inv;
-                *reinterpret_cast<f32x4 *>(orow + 32 * db + 8 * rb + 4 * h) = v;
+    if constexpr (PAD) {   // outputs that are not finite, once they are stored
+        __syncthreads();
+        if (!redo) return;
+        const float *qrow = qbase + (int64_t)min(qi, a.seq_q - 1) * qrs;
+        if constexpr (D <= 128) {
+            prefill_f32_redo<D, GEN>(a, copy_tile, qrow, k0s, v0s, kr, vr, 0, tlo, thi, qi, l32, h, m, inv, bits, orow);
+        } else {
+            const int groups = __builtin_amdgcn_readfirstlane(redo);
+#pragma unroll 1
+            for (int w = 0; w < T::DB / 2; ++w) {
+                if (!(groups >> w & 1)) continue;
+                const int at = 4 * h * T::RB, vd[2] = {at + (((64 * w + l32) ^ (32 * h)) << 2), at + (((64 * w + 32 + l32) ^ (32 * h)) << 2)};
+                const uint32_t mine[1] = {w == 0 ? bits[0] : w == 1 ? bits[1] : w == 2 ? bits[2] : bits[3]};
+                prefill_f32_redo<D, GEN>(a, copy_tile, qrow, k0s, v0s, kr, vd, 2 * w, tlo, thi, qi, l32, h, m, inv, mine, orow);
             }
         }
     }

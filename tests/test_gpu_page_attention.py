@@ -425,6 +425,88 @@ def test_mha_other_head_dims_infinite_values(backend, dt, d):
     assert_close(got[:-1], ref[:-1], TOL[dt], elem_tol=None, what=f"mha d {d} with NaN and inf values")
 
 
+@pytest.mark.parametrize("dt", [O.BF16, O.F16, O.F32])
+@pytest.mark.parametrize("d,sq,sk,h,kvh,causal,window,alibi", [
+    (40, 130, 300, 16, 4, True, 0, 0.0), (96, 200, 200, 12, 12, True, 70, 0.0), (96, 257, 333, 8, 2, False, 0, 0.0),
+    (120, 150, 700, 16, 4, True, 0, 0.1), (256, 140, 520, 16, 16, True, 0, 0.0), (160, 300, 100, 8, 8, False, 0, 0.0),
+])
+def test_mha_other_head_dims_not_finite(backend, dt, d, sq, sk, h, kvh, causal, window, alibi):
+    """Infinities of either sign, both in one dim, NaNs, and an infinity at a visible key whose
+    probability is zero (0 * inf): each output is NaN, infinite or finite as the sum over the
+    keys that its query sees (those masked are not read), and the finite ones have its values."""
+    import puter_amd
+    q, k = (encode(seeded(730 + i, (s, n * d), 0.0, d ** -0.25), dt) for i, (s, n) in enumerate(((sq, h), (sk, kvh))))
+    v = seeded(732, (sk, kvh * d)).reshape(sk, kvh, d)
+    q, k = (decode(x, dt).reshape(-1, n, d).copy() for x, n in ((q, h), (k, kvh)))
+    q[:, :, 0] = 8.0
+    k[:, :, 0], k[7, :, 0] = 0.0, -2048.0            # key 7: a score of -16384 / sqrt(d)
+    q, k = (encode(x.reshape(len(x), -1), dt) for x in (q, k))
+    v[2, :, 0], v[sk // 2, :, 1], v[sk // 2, :, 33] = np.inf, -np.inf, np.inf
+    v[sk // 3, :, 33], v[5, 0, 3], v[7, :, 20] = -np.inf, np.nan, np.inf
+    v[sk - 1, 0] = np.nan
+    v = encode(v.reshape(sk, -1), dt)
+    out = empty_dev((sq, h * d), NP[dt])
+    cfg = puter_amd.MultiHeadAttentionConfig(h, d, causal, window, alibi, kvh)
+    backend.MultiHeadAttention(cfg, to_dev(q), to_dev(k), to_dev(v), out, sq, sk, dt)
+    got = decode(to_host(out, NP[dt]), dt)
+    q, k, v = (decode(x, dt).astype(np.float64).reshape(-1, n, d) for x, n in ((q, h), (k, kvh), (v, kvh)))
+    at, key = np.arange(sq)[:, None], np.arange(sk)[None, :]
+    seen = np.full((sq, sk), True)
+    if causal:
+        seen &= key <= at + sk - sq
+    if window:
+        seen &= at - key < window
+    ref = np.empty((sq, h, d))
+    for i in range(h):
+        x = v[:, i * kvh // h]
+        score = np.where(seen, q[:, i] @ k[:, i * kvh // h].T / np.sqrt(d) + alibi * (key - at), -np.inf)
+        p = np.exp(score - score.max(axis=1, keepdims=True))
+        nan = seen @ np.isnan(x) | (seen & (p == 0)) @ np.isinf(x)
+        up, down = (seen @ (x == s * np.inf) for s in (1, -1))
+        y = p @ np.where(np.isfinite(x), x, 0) / p.sum(axis=1, keepdims=True)
+        ref[:, i] = np.where(nan | up & down, np.nan, np.where(up, np.inf, np.where(down, -np.inf, y)))
+    ref = ref.reshape(sq, h * d)
+    assert not np.isfinite(ref).all() and np.isfinite(ref).any() and np.isinf(ref).any()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    assert np.array_equal(got[inf], ref[inf]) and np.array_equal(np.isinf(got), inf)
+    fin = np.isfinite(ref)
+    assert_close(np.where(fin, got, 0), np.where(fin, ref, 0), TOL[dt], elem_tol=None, what=f"mha d {d} not finite")
+
+
+@pytest.mark.parametrize("dt", [O.BF16, O.F16, O.F32])
+@pytest.mark.parametrize("d", [40, 96, 256])
+def test_mha_other_head_dims_not_finite_in_time(backend, dt, d):
+    """Values that are not finite cost a second walk over the keys, not a row's keys one by
+    one (hundreds of times the call): at most four times a call on finite values was
+    measured, the bound is twelve."""
+    import torch
+    import puter_amd
+    sq, sk, h = 512, 1024, 8
+    q, k, v = (to_dev(encode(seeded(740 + i, (s, h * d), 0.0, d ** -0.25), dt)) for i, s in enumerate((sq, sk, sk)))
+    bad = v.clone()
+    bad[3] = to_dev(encode(np.full(1, np.nan, np.float32), dt))[0]
+    out = empty_dev((sq, h * d), NP[dt])
+    cfg = puter_amd.MultiHeadAttentionConfig(h, d, True, 0, 0.0, h)
+
+    def us(values):
+        call = lambda: backend.MultiHeadAttention(cfg, q, k, values, out, sq, sk, dt)  # noqa: E731
+        call()
+        best = float("inf")
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                call()
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end) * 250)
+        return best
+
+    finite, spoiled = us(v), us(bad)
+    assert spoiled < 12 * finite, (finite, spoiled)
+
+
 @pytest.mark.parametrize("dt", [O.BF16, O.F16])
 @pytest.mark.parametrize("b,sk,h,kvh,causal,window", [
     (1, 4096, 32, 8, True, 0),     # configs[4]'s heads at one sequence's full context
