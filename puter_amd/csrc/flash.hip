@@ -182,19 +182,9 @@ __global__ __launch_bounds__(256) void flash_score_kernel(FlashArgs a, float *S,
     }
 }
 
-// flash_exp for x <= 0 or NaN (which passes through the polynomial)
+// flash_exp for x <= 0 or NaN, without a branch
 __device__ __forceinline__ float flash_exp_neg(float x) {
-    const float z = __fmul_rn(x, 1.4426950408889634f);
-    int32_t k = (int32_t)z;
-    if (z < 0) k--;
-    const float f = __fsub_rn(z, (float)k);
-    float p = __fmul_rn(f, 0.00133389f);
-    p = __fmul_rn(f, __fadd_rn(0.00961812f, p));
-    p = __fmul_rn(f, __fadd_rn(0.05550410f, p));
-    p = __fmul_rn(f, __fadd_rn(0.24022650f, p));
-    p = __fmul_rn(f, __fadd_rn(0.69314718f, p));
-    p = __fadd_rn(1.0f, p);
-    const float y = __uint_as_float(__float_as_uint(p) + ((uint32_t)k << 23));
+    const float y = fast_exp32_body(x);
     return x < -87.33654f ? 0.0f : x != x ? x : y;
 }
 
