@@ -1395,13 +1395,13 @@ static_assert(sizeof(ScratchCounters) + kPairTiles * kPairTileBytes <= kNoAllocB
               "the no-alloc array holds any kernel's counters and sums");
 }  // namespace noalloc
 
-// Runs of K of the rows kernel: toward one block per CU (200 of 256 is near enough: 16 x
+// Runs of K of the rows kernel: toward one block per CU (200 of the 256 are near enough: 16 x
 // 4096 x 14336, 112 tiles, 24.9 us in 2 runs, 25.5 in 4; 32 tiles 11.2 in 8, 14.3 in 4), each
 // run two 128-deep steps or more, or one step in at most 8 runs (1 x 768 x 768 5.4 -> 4.5).
 static int64_t rows_chunks(int64_t blocks, int64_t K) {
     const int64_t steps = (K + kRwWaves * kRwDepth - 1) / (kRwWaves * kRwDepth);
     int64_t c = 1;
-    while (c < 16 && c * blocks < 200) c *= 2;
+    while (c < 16 && c * blocks * 32 < (int64_t)device_cus() * 25) c *= 2;
     return std::min<int64_t>(c, std::max<int64_t>(steps / 2, std::min<int64_t>(steps, 8)));
 }
 
@@ -1545,7 +1545,9 @@ static bool mfma_small_tiles(int64_t M, int64_t N) {
 }
 
 // 256 x 256 tiles with K in two halves: twice the blocks of half the work, for grids that fill
-// half a round (or one and a half) of them.  In units of 1/100 of a large round: a half round
+// half a round (or one and a half) of them.  (Under 512 small tiles the skinny kernel is asked
+// first, so of the half rounds only those of whole tiles get here: 2000 x 14336 x 4096 does, 1900
+// and 1500 rows do not.)  In units of 1/100 of a large round: a half round
 // 50, and 30 us (1200 / K of a round) for the sums that change hands; a small round 55, the
 // launch's first and last slices 11 (one small round measured 66, three 165 - 190).
 // 2000 x 14336 x 4096 247 -> 211 us, 2048 x 8192 x 4096 142 -> 125, 2048 x 28672 x 4096 488 ->
