@@ -510,7 +510,7 @@ int puter_hip_kv_page_write_fp8(void *storage, const void *values, const int32_t
     if (reinterpret_cast<uintptr_t>(status) & 3) return fail(PUTER_ERR_INVALID, "kv page write fp8: misaligned status word");
     const int64_t inner = kv_heads * head_dim;
     uint8_t *dst = static_cast<uint8_t *>(storage) + storage_offset;
-    // the 16-byte fp8 stores need 16-byte aligned rows
+    // (the contract's alignment; the stores are of 8 bytes, whole units of a row)
     if (((reinterpret_cast<uintptr_t>(dst) | (uintptr_t)inner) & 15) != 0)
         return fail(PUTER_ERR_INVALID, "kv page write fp8: pool rows must be 16-byte aligned");
     hipStream_t s = as_stream(stream);

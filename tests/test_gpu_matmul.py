@@ -219,9 +219,8 @@ def test_matmul_skinny_two_streams_share_the_scratch_safely(backend):
 
 
 def test_matmul_unaligned_16bit_falls_back(backend):
-    """A left operand at an odd element offset is not 16-byte aligned: the MFMA and
-    split-K paths are skipped for the generic kernel, whose result still meets the
-    bar."""
+    """A left operand at an odd element offset is not 16-byte aligned: the kernels that copy
+    16 bytes into LDS are skipped for the rows kernel, whose result meets the bar."""
     import torch
     rows, inner, cols = 64, 256, 512
     a = O.from_f32(seeded(971, (rows, inner)), O.BF16)
@@ -464,13 +463,14 @@ def test_matmul_empty_inner_is_zero(backend, dt, np_dt):
 @pytest.mark.parametrize("dt", [O.BF16, O.F16])
 @pytest.mark.parametrize("rows,inner,cols", [
     (2041, 8200, 4088),    # half a round of 256 x 256 tiles; ragged rows and columns, the second half of K ragged
-    (1793, 16384, 4096),   # the last row tile of one row
+    (1793, 16384, 4096),   # fewer than 512 tiles of 128 x 128: the skinny kernel's
+    (2817, 8192, 8192),    # one and a half rounds, the last row tile of one row
     (4100, 7752, 4096),    # one and a half rounds, row tiles past a multiple of four
 ])
 @pytest.mark.usefixtures("no_collection")
 def test_matmul_16bit_two_halves_of_k_exact(backend, dt, rows, inner, cols):
-    """256 x 256 tiles whose K is divided between two blocks, bit for bit: integer operands keep
-    every sum exact.  On the default stream and on a side stream (each has its own sums and
+    """256 x 256 tiles whose K is divided between two blocks (and a size that just is not), bit
+    for bit: integer operands keep every sum exact.  On the default stream and on a side stream (each has its own sums and
     counters) without synchronisation between the calls, and under capture, which takes the
     undivided kernel."""
     import torch

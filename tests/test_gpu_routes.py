@@ -85,6 +85,10 @@ def test_norm_kernels(backend, op, dt, rows, h, kernel):
     (O.F16, 4, 5, 33, ["matmul_generic"]), (O.BF16, 200, 31, 129, ["matmul_generic"]),
     (O.BF16, 7, 31, 33, ["matmul_rows"]), (O.F16, 200, 31, 129, ["matmul_rows"]),
     (O.BF16, 1000, 31, 4097, ["matmul_rows"]), (O.BF16, 33, 4096, 32001, ["matmul_rows"]),
+    # 256 x 256 tiles with K in two halves, where they fill half a round or one and a half
+    (O.BF16, 2041, 8200, 4088, ["64, 2, true>"]), (O.F16, 2817, 8192, 8192, ["64, 2, true>"]),
+    (O.BF16, 4100, 7752, 4096, ["64, 2, true>"]), (O.BF16, 1793, 16384, 4096, ["matmul_skinny"]),
+    (O.BF16, 4096, 4096, 4096, ["64, 2, false>"]),
 ])
 def test_matmul_kernels(backend, dt, rows, inner, cols, kernels):
     a, b, c = zeros(dt, rows, inner), zeros(dt, inner, cols), zeros(dt, rows, cols)
