@@ -19,7 +19,7 @@
  *     makes itself is a split-K scratch shared by puter_hip_matmul (16-bit
  *     formats with at most 512 rows or under two rounds of 128x128 tiles, or of
  *     sizes or alignments that the 16-byte copies cannot take, or of grids of
- *     256x256 tiles that fill about half a round, F32
+ *     256x256 tiles that fill half a round or one and a half, F32
  *     outputs of fewer 128x128 tiles than the device has CUs, when K is split
  *     across blocks rather than inside them) and
  *     puter_hip_multi_head_attention[_batched] with seq_q == 1 (bf16 / f16 at
@@ -43,7 +43,8 @@
  *     the same call, or a larger one, outside the capture first (F32 attention,
  *     scaled-dot-product attention, and Matmul with unaligned 16-bit operands or in
  *     256x256 tiles use no scratch under capture, and where an eager call of theirs
- *     finds no room it runs without).  Replays share
+ *     finds no room it runs without: it adds in another order then, so the last bits
+ *     of a replay can differ from the eager call's).  Replays share
  *     the buffer with eager scratch-using calls until such a growth, so the
  *     caller orders them (one stream, or its own events).
  *
@@ -387,7 +388,8 @@ PUTER_API int puter_hip_quant(void *dst, const void *src, int64_t count, float s
 /* out[rows, cols] = left[rows, inner] . right[inner, cols], row-major, in F32, F64,
  * BF16 or F16 (16-bit formats accumulate in f32 and round once).  BF16 / F16 with
  * at least 8 columns run on MFMA, whatever their sizes and alignment (fastest with
- * cols % 8 == 0, inner % 8 == 0 and 16-byte aligned buffers); with at
+ * cols % 8 == 0, inner % 8 == 0 and 16-byte aligned buffers; without those, small
+ * products of little `inner` take a thread per output); with at
  * most 512 rows they split `inner` across blocks and keep f32 partials in the
  * library's per-device scratch (calls on different streams are ordered on the
  * device by an event); so does F32 when the output has fewer than 256 64x64

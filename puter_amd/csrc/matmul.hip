@@ -34,10 +34,11 @@
 // to XCDs in 4 x 8 groups (consecutive block ids run round-robin over the 8
 // XCDs), so the blocks an XCD runs at once share their A and B panels in its L2.
 // Requirements of the MFMA path: N % 8 == 0, K % 8 == 0, 16-byte aligned
-// buffers, 256 * K * 2 and BK * N * 2 below 2^31; at most 32 rows, and the shapes
-// and alignments these exclude, take the rows kernel (16-byte loads into registers
-// at any element); fewer than 8 columns the generic kernel (one thread per output, f32
-// accumulation in index order).
+// buffers, 256 * K * 2 and BK * N * 2 below 2^31; at most 32 rows (but where the skinny
+// kernel runs unsplit), and the shapes and alignments these exclude, take the rows kernel
+// (16-byte loads into registers at any element); fewer than 8 columns, and of those
+// shapes little K with few outputs (generic_wins), the generic kernel (one thread per
+// output, f32 accumulation in index order).
 //
 // f32: small outputs of moderate depth take the small kernel (32 x 32 or 16 x 16
 // tiles, K split over the 8 waves of each block on the f32 MFMA); other shapes with K
