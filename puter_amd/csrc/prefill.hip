@@ -523,6 +523,36 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
     }
 }
 
+// Byte offsets of a lane's tile copies (source side, swizzled; chunks past the head dim: an
+// offset past the buffer's range, read as zeros) and of its fragment reads: K row l32 (+32c),
+// chunk (2t + g) ^ kswz(l32); V: lane group q = lane/16, i = lane%16 = 4j + m reads key row
+// 4(q/2) + j, dims 16(q%2) + 4m .. +3 of dim block d: chunk (4d + 2(q%2) + m/2) ^ vswz(row),
+// half m%2
+template <int D>
+__device__ __forceinline__ void prefill_offsets(int kv_heads, int dim, int lane, int wave, int (&kg)[PfDim<D>::NI],
+                                                int (&vg)[PfDim<D>::NI], int (&ka)[PfDim<D>::KS], int (&va)[PfDim<D>::DB]) {
+    using T = PfDim<D>;
+    const int rs2 = kv_heads * dim * 2;
+    const int pos = lane % T::NC;
+#pragma unroll
+    for (int i = 0; i < T::NI; ++i) {
+        const int row = 4 * T::RPI * i + T::RPI * wave + lane / T::NC;
+        const int kc = pos ^ T::kswz(row), vc = pos ^ T::vswz(row);
+        kg[i] = 8 * kc < dim ? row * rs2 + (kc << 4) : fa::OOB;
+        vg[i] = 8 * vc < dim ? row * rs2 + (vc << 4) : fa::OOB;
+    }
+    const int l32 = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int t = 0; t < T::KS; ++t) ka[t] = l32 * T::RB + (((2 * t + g) ^ T::kswz(l32)) << 4);
+    const int q = lane >> 4, i = lane & 15, j = i >> 2, m = i & 3;
+    const int row = 4 * (q >> 1) + j;
+#pragma unroll
+    for (int d = 0; d < T::DB; ++d) {
+        const int chunk = (4 * d + 2 * (q & 1) + (m >> 1)) ^ T::vswz(row);
+        va[d] = row * T::RB + (chunk << 4) + 8 * (m & 1);
+    }
+}
+
 // The padded kernels' outputs where an infinity or NaN of V met a P of zero (a masked key
 // of a computed tile, or P's low half): 0 * inf is NaN in the MFMA, while the general
 // kernel, which served these head dims before, never reads a masked key's row.  A block
@@ -533,10 +563,10 @@ __device__ __forceinline__ void prefill_step_pipelined(const PrefillArgs &a, con
 // inf does).  Only outputs that were not finite are replaced.  The second walk costs what the
 // first does and is never taken on finite values; a lane summing its row key by key took
 // 18 ms for bf16 2 x 700 of 1500 keys x 16 heads of 96 with a NaN in V, the general kernel 1.0; now
-// 107 us, 36 without the NaN.
-// It runs after the first walk's outputs are stored and loads Q again: with more alive the first
-// walk of 129 to 256 dims slowed by 4 to 9%, now by 2 to 3% (not inlined, by the stack that a call
-// needs: 34 -> 38 us).
+// 110 us, 36 without the NaN.
+// It runs after the first walk's outputs are stored, loads Q again and finds the lane's offsets
+// again: with more alive the first walk of 129 to 256 dims slowed by 2 to 9% (one register more and
+// its V reads no longer ran ahead; not inlined, by the stack that a call needs: 34 -> 38 us).
 constexpr float kPfPos = 1.0f, kPfNeg = 128.0f, kPfNan = 16384.0f;   // up to 64 keys a tile: digits that stay apart
 // a lane's outputs that are not finite: bit 16 (d % 2) + r of word d / 2; whether there are any
 template <int NO> __device__ __forceinline__ bool prefill_spoiled(const f32x16 (&o)[NO], uint32_t (&bits)[(NO + 1) / 2]) {
@@ -751,35 +781,8 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
         tfree = max(tlo, (max(0, qmax - a.window + 1) + BN - 1) / BN);
     }
 
-    // byte offsets of this lane's tile copies (source side, swizzled) ...
-    int kg[T::NI], vg[T::NI];
-    {
-        // chunks past the head dim: an offset past the buffer's range, read as zeros
-        const int rs2 = a.kv_heads * dim * 2;
-        const int pos = lane % T::NC;
-#pragma unroll
-        for (int i = 0; i < T::NI; ++i) {
-            const int row = 4 * T::RPI * i + T::RPI * wave + lane / T::NC;
-            const int kc = pos ^ T::kswz(row), vc = pos ^ T::vswz(row);
-            kg[i] = 8 * kc < dim ? row * rs2 + (kc << 4) : OOB;
-            vg[i] = 8 * vc < dim ? row * rs2 + (vc << 4) : OOB;
-        }
-    }
-    // ... and of its fragment reads: K row l32 (+32c), chunk (2t + g) ^ kswz(l32);
-    // V: lane group q = lane/16, i = lane%16 = 4j + m reads key row 4(q/2) + j,
-    // dims 16(q%2) + 4m .. +3 of dim block d: chunk (4d + 2(q%2) + m/2) ^ vswz(row), half m%2
-    int ka[T::KS], va[T::DB];
-#pragma unroll
-    for (int t = 0; t < T::KS; ++t) ka[t] = l32 * T::RB + (((2 * t + g) ^ T::kswz(l32)) << 4);
-    {
-        const int q = lane >> 4, i = lane & 15, j = i >> 2, m = i & 3;
-        const int row = 4 * (q >> 1) + j;
-#pragma unroll
-        for (int d = 0; d < T::DB; ++d) {
-            const int chunk = (4 * d + 2 * (q & 1) + (m >> 1)) ^ T::vswz(row);
-            va[d] = row * T::RB + (chunk << 4) + 8 * (m & 1);
-        }
-    }
+    int kg[T::NI], vg[T::NI], ka[T::KS], va[T::DB];
+    prefill_offsets<D>(a.kv_heads, dim, lane, wave, kg, vg, ka, va);
     PrefillState<D> st;
 #pragma unroll
     for (int d = 0; d < T::DB; ++d) st.o[d] = (f32x16){};
@@ -870,6 +873,11 @@ __global__ __launch_bounds__(256, D > 128 ? 1 : 2) void prefill_kernel(PrefillAr
     if constexpr (PAD) {
         __syncthreads();
         if (__builtin_expect(!redo, 1)) return;
+        // (the lane and its offsets afresh, so that none of them is alive for this in the first walk)
+        const int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), g = lane >> 5;
+        const int qi = qfirst + (lane & 31);
+        int kg[T::NI], vg[T::NI], ka[T::KS], va[T::DB];
+        prefill_offsets<D>(a.kv_heads, dim, lane, wave, kg, vg, ka, va);
         const int64_t row = (int64_t)min(qi, a.seq_q - 1) * qrs;
         prefill_redo<DT, D, GEN>(a, qbase + row, kbase, vbase, k0s, v0s, kg, vg, ka, va, tlo, ntiles, qi, g, wave, st.m, inv, bits,
                                  a.o + (qbase - a.q) + row);
